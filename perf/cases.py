@@ -213,4 +213,4 @@ def tolerance(case):
     # a step through separate norm and merge launches is 3.1e-2 .. 4.1e-2 (largest 0.21) from the
     # folded one, a prompt through windows of 32 tokens 4.5e-2 .. 6.8e-2 (0.43) from windows of
     # 64, through plain torch operations between the matrix products 0.10 (0.61)
-    return {"rel": 0.15, "max": 0.8} if kind == "step" else {"rel": 0.2, "max": 1.5}
+    return {"rel": 0.15, "max": 0.8} if kind == "step" else {"rel": 0.2, "max": 0.95}
