@@ -307,6 +307,13 @@ __device__ __forceinline__ uint4 lds0_u128(uint32_t addr) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// 16 bytes a lane from global memory into LDS at `at` (uniform) + 16 * lane, no register between.
+__device__ __forceinline__ void load_to_lds16(const uint16_t *src, uint32_t at) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint16_t *)src,
+                                   reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(at), 16, 0, 0);
+}
+__device__ __forceinline__ void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Compute units of the current device (256 on an MI355X), cached after the first call.
 inline int device_cu_count() {
   static int cached = [] {

@@ -7,9 +7,11 @@ nothing registers one, ``weight`` is a read-only 0-element stand-in, so neither
 
 Layout glue lives here: callers hand ``[..., K]`` activations, the kernels take ``[K, N]``
 (token index fastest) and answer ``[M, N]``.  One token is a view (no copy) and goes to the
-GEMV; more tokens go to the MFMA GEMM in windows of at most 32, each window's answer
-written straight into its rows of the one output buffer.  The bias is added afterwards in
-bf16, as the reference does (``linear.py:62-63,79-80``), so both seats round alike.
+GEMV; more tokens go to the token-major product, which takes and leaves rows as they are, or,
+through a small matrix, to the MFMA GEMM in windows of at most 32, each window's answer
+written straight into its rows of the one output buffer.  The bias is added after the
+product's bf16 rounding, as the reference does (``linear.py:62-63,79-80``), so all seats
+round alike.
 """
 
 from __future__ import annotations
@@ -20,13 +22,18 @@ import torch
 from torch import nn
 
 from ..chr0.loader import ChrMatrix
-from ..nf4 import LIVE_MAX_N, nf4_gemm
+from ..nf4 import LIVE_MAX_N, nf4_gemm, nf4_wide
 from ..nf4.plan import k_pad
 from ..ring.host_image import HostImage
 
 __all__ = ["CompressedLinear", "nf4_linear", "k_pad"]
 
 GROUP_SIZE = 64
+#: Matrices of fewer codes stay in windows of 32 tokens: launches of a few us either way
+#: (512x512 at 32 tokens 12.7 us in a window, 10.0 token-major), and their windows multiply
+#: bf16(level * scale), not the level and the scale apart, which callers of small seats see in
+#: the last bit.
+WIDE_MIN_CODES = 1 << 17
 
 
 def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: int, K: int,  # noqa: N803
@@ -41,6 +48,13 @@ def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: in
     rows = x.to(torch.bfloat16).reshape(n, K)
     if n == 1:
         out = nf4_gemm(packed, scale, rows.reshape(K, 1), M, K, K_pad).reshape(1, M)
+    elif M * K >= WIDE_MIN_CODES:
+        # the launch adds a bias it can add as torch would: bf16, one element a feature, no graph
+        folds = (bias is not None and bias.dtype == torch.bfloat16 and tuple(bias.shape) == (M,)
+                 and bias.is_contiguous() and bias.device == rows.device and not bias.requires_grad)
+        out = nf4_wide(packed, scale, rows, M, K, K_pad, bias=bias if folds else None)
+        if folds:
+            bias = None
     else:
         out = torch.empty((n, M), dtype=torch.bfloat16, device=rows.device)
         for lo in range(0, n, LIVE_MAX_N):

@@ -59,6 +59,7 @@ __all__ = [
     "dv2_add_cols",
     "dv2_gemm_qkv",
     "dv2_gemm_swiglu",
+    "nf4_wide",
     "library_path",
 ]
 
@@ -158,6 +159,8 @@ EXPORTS = (
     ("chr_dv2_argmax_commit", ctypes.c_int, [_P, _I, _P, _P, _P, _P, _P, _I, _P]),
     ("chr_dv2_argmax_ws_bytes", ctypes.c_int64, []),
     ("chr_dv2_argmax_commit_ws", ctypes.c_int, [_P, _I, _P, _P, _P, _P, _P, _I, _P, ctypes.c_int64, _P]),
+    ("chr_nf4_wide", ctypes.c_int, [_DP, _P, ctypes.c_int64, _I, _P, _P, ctypes.c_int64, _P, _P]),
+    ("chr_nf4_wide_ws", ctypes.c_int64, [_DP, _I]),
     ("chr_nf4_abi_version", ctypes.c_int, []),
 )
 
@@ -1042,4 +1045,34 @@ def dv2_gemm_swiglu(gate, up, x: torch.Tensor) -> torch.Tensor:
     rc = lib.chr_dv2_gemm_swiglu(ctypes.byref(devs[0]), ctypes.byref(devs[1]), x.data_ptr(), y.data_ptr(),
                                  n, None if ws is None else ws.data_ptr(), need, _stream())
     _check_rc("chr_dv2_gemm_swiglu", rc)
+    return y
+
+
+def nf4_wide(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int, K: int,  # noqa: N803
+             K_pad: int, *, bias: torch.Tensor | None = None) -> torch.Tensor:  # noqa: N803
+    """``x [N, K]`` bf16, any N, times the transpose of the packed matrix: ``[N, M]`` (+ ``bias``,
+    one bf16 element a feature).  A ragged K is padded with zeros into a copy, rows that are not
+    contiguous in whole 16-byte pieces are copied."""
+    M, K, K_pad = int(M), int(K), int(K_pad)
+    _need(packed.is_cuda and scale.is_cuda and x.is_cuda, "packed, scale, and x must be CUDA tensors")
+    _need(x.dtype == torch.bfloat16 and x.dim() == 2 and int(x.size(1)) == K and int(x.size(0)) >= 1,
+          f"x must be bfloat16 [N, {K}]")
+    _check_packed(packed, scale, M, K, K_pad)
+    packed, scale = packed.contiguous(), scale.contiguous()
+    if K != K_pad:
+        x = torch.nn.functional.pad(x, (0, K_pad - K))
+    elif x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < K or x.data_ptr() % 16 != 0:
+        x = x.clone(memory_format=torch.contiguous_format)
+    n = int(x.size(0))
+    _need(bias is None or (bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
+                           and bias.numel() == M), f"bias must be contiguous CUDA bf16 of {M} elements")
+    lib = _load_ext()
+    w = _dev(packed, scale, M, K, K_pad)
+    floats = int(lib.chr_nf4_wide_ws(ctypes.byref(w), n))
+    ws = torch.empty(floats, dtype=torch.float32, device=x.device) if floats > 0 else None
+    y = torch.empty((n, M), dtype=torch.bfloat16, device=x.device)
+    rc = lib.chr_nf4_wide(ctypes.byref(w), x.data_ptr(), int(x.stride(0)), n, y.data_ptr(),
+                          None if ws is None else ws.data_ptr(), floats, None if bias is None else bias.data_ptr(),
+                          _stream())
+    _check_rc("chr_nf4_wide", rc)
     return y

@@ -409,6 +409,21 @@ int chr_dv2_argmax_commit_ws(const void *logits, int32_t n, void *next_token, vo
                              void *position, void *finished, const void *eos_id, int32_t commit,
                              void *ws, int64_t ws_bytes, void *stream);
 
+/* ---- Any number of tokens, token-major ---------------------------------------------------------
+ * y [N, M] = x [N, K] dequant(W)^T (+ bias[M], bf16, added after the product's bf16 rounding) for
+ * any N >= 1, the K elements of a token contiguous (rows x_stride elements apart) and the M features
+ * of a token contiguous.  The entries above take at most 64 columns of feature-major data: a longer
+ * call is cut into windows, each of which reads and decodes the whole matrix (the reference's host
+ * cuts at 32, gpu/decodev2/linear.py:96-113).  No counterpart in the reference's C-ABI.
+ *   - x 16-byte and y 8-byte aligned (-5); x_stride % 8 == 0 and x_stride >= K_pad (-3): where K is
+ *     not a multiple of 64 the caller's rows are K_pad long, with zeros behind K
+ *   - ws: chr_nf4_wide_ws floats (0: none; -1: bad arguments), 16-byte aligned (-5; too few: -7)
+ *   - weights enter as bf16(level) and every 64-wide group's sum takes its scale in fp32, as in the
+ *     tile of chr_nf4_gemm that finishes its rows itself */
+int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y,
+                 float *ws, int64_t ws_floats, const void *bias, void *stream);
+int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N);
+
 /* Library version, for the loader's sanity check. */
 int chr_nf4_abi_version(void);
 

@@ -1,0 +1,98 @@
+"""The token-major product of any number of tokens, against the decoded matrix in 64 bits, and
+through the linear seat."""
+
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from deepfold_amd import nf4
+from deepfold_amd.chr0.loader import ChrMatrix
+from deepfold_amd.host import CompressedLinear, k_pad
+from oracle import nf4_oracle as oc
+
+BF16 = torch.bfloat16
+
+
+def test_arguments_are_refused_before_any_launch():
+    lib = nf4._load_ext()
+    p = 0x4000
+
+    def rc(m=128, k=256, kp=256, n=65, stride=256, x=p, y=p, packed=0x1000, scale=0x2000):
+        w = nf4._Dev(m, k, kp, packed, scale)
+        return lib.chr_nf4_wide(ctypes.byref(w), x, stride, n, y, None, 0, None, None)
+
+    assert lib.chr_nf4_wide(None, p, 256, 4, p, None, 0, None, None) == -1
+    assert rc(x=None) == -1 and rc(y=None) == -1 and rc(n=0) == -2
+    assert rc(m=0) == -3 and rc(packed=None) == -3 and rc(stride=248) == -3 and rc(stride=260) == -3
+    assert rc(kp=320) == -4 and rc(packed=0x1008) == -5 and rc(scale=0x2001) == -5
+    assert rc(x=p + 2) == -5 and rc(y=p + 2) == -5
+    w = nf4._Dev(5120, 13824, 13824, 0x1000, 0x2000)
+    need = lib.chr_nf4_wide_ws(ctypes.byref(w), 128)
+    assert need > 0 and need % (128 * 5120) == 0       # few tokens, long K: split
+    assert lib.chr_nf4_wide(ctypes.byref(w), p, 13824, 128, p, p, need - 1, None, None) == -7
+    assert lib.chr_nf4_wide(ctypes.byref(w), p, 13824, 128, p, p + 4, need, None, None) == -5
+    assert lib.chr_nf4_wide_ws(ctypes.byref(w), 0) == -1
+
+
+def matrix(m, k, seed, sigma=0.05):
+    w = np.random.default_rng(seed).standard_normal((m, k)).astype(np.float32) * sigma
+    p, s = oc.c_encode(w)
+    dense = torch.from_numpy(oc.c_decode(p, s, m, k).copy()).cuda().double()
+    return (torch.from_numpy(p).cuda(), torch.from_numpy(np.ascontiguousarray(s).view(np.float16)).cuda(), m), dense
+
+
+def rand(*shape, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(*shape, generator=g, device="cuda").to(BF16)
+
+
+def close(got, want):
+    # one bf16 rounding of the result (2^-9 of it at most, 1.7e-3 of its norm) and one of every level
+    # (1.4e-3): 2.2e-3 of the norm; a bias rounds again
+    got, want = got.double(), want.double()
+    assert bool(torch.isfinite(got).all())
+    assert float((got - want).norm()) <= 5e-3 * float(want.norm())
+    assert float((got - want).abs().max()) <= 2e-2 * max(float(want.abs().max()), 1e-3)
+
+
+# tile edges (16, 32, 64, 128 tokens; 256, 512 rows), odd group counts (a last half stage), ragged K (padded
+# copy), rows that are no whole vectors, few tokens over a long K (splits)
+SHAPES = [(1, 64, 64), (2, 300, 128), (17, 5120, 1088), (33, 256, 576), (65, 256, 64), (63, 255, 192), (129, 513, 320), (70, 1030, 200), (128, 130, 2048),
+          (257, 77, 1111), (66, 5120, 4160), (520, 512, 640)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,k", SHAPES)
+@pytest.mark.parametrize("bias", [False, True])
+def test_product(n, m, k, bias):
+    mat, w = matrix(m, k, seed=m + k)
+    x = rand(n, k, seed=n)
+    b = rand(m, seed=5) if bias else None
+    want = x.double() @ w.t()
+    got = nf4.nf4_wide(*mat[:2], x, m, k, k_pad(k), bias=b)
+    close(got, want + b.double() if bias else want)
+    # rows of a wider buffer, aligned or not, give the same bits
+    for off in (8, 3):
+        wide = torch.zeros((n, k + 16), dtype=BF16, device="cuda")
+        wide[:, off:off + k] = x
+        assert torch.equal(nf4.nf4_wide(*mat[:2], wide[:, off:off + k], m, k, k_pad(k), bias=b), got)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 16, 17, 32, 33, 64, 65, 257])
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+def test_linear_seat_across_the_window(n, dtype):
+    m, k = 640, 500
+    (p, s, _), w = matrix(m, k, seed=9)
+    lin = CompressedLinear(k, m, bias=True, device="cuda", dtype=dtype)
+    lin.attach(ChrMatrix("t", m, k, k_pad(k), p, s))
+    lin.set_bias(rand(m, seed=1).to(dtype))
+    x = rand(n, k, seed=2)
+    y = lin(x)
+    assert y.dtype == dtype                        # a wider bias still widens the answer
+    close(y, x.double() @ w.t() + lin.bias.double())
+    assert torch.equal(lin(x.t().contiguous().t()), y)   # K not the fastest axis
