@@ -5,10 +5,23 @@
 
 #include "nf4_common.h"
 
-#include <algorithm>
-
 namespace chr {
 namespace {
+
+typedef __attribute__((ext_vector_type(4))) float F32x4;
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true));
+}
+
+// largest of sixteen neighbouring lanes, in all of them
+__device__ __forceinline__ uint32_t group_max16_u32(uint32_t v) {
+  v = max(v, dpp_u32<kDppQuadXor1>(v));
+  v = max(v, dpp_u32<kDppQuadXor2>(v));
+  v = max(v, dpp_u32<kDppRowHalfMirror>(v));
+  return max(v, dpp_u32<kDppRowMirror>(v));
+}
 
 __device__ __forceinline__ void load_lut_lds(float *lut) {
   if (threadIdx.x < 16) {
@@ -18,27 +31,74 @@ __device__ __forceinline__ void load_lut_lds(float *lut) {
 }
 
 // ---- codec twins -------------------------------------------------------------
-// One thread per packed dword (8 weights).  out is [M, K] fp32.
+// out is [M, K] fp32, four weights a thread and kDequantQuads such quads, a workgroup's quads
+// back to back: every store is a 16-byte piece of a wavefront's whole kilobyte, and the loads (two
+// bytes a quad) are all issued before the first store.  Bound by the fp32 it writes, past the caches
+// (the non-temporal hint): 5120x27648 in 90 us (7.1 TB/s; 128 without the hint, 93 / 102 with one or
+// eight quads), where eight weights a thread in eight 4-byte stores 32 bytes apart took 332.  The
+// 16-entry table has no bank conflicts (equal codes read one address, others other banks).
+constexpr int kDequantQuads = 4;
+
+template <typename Index>
 __global__ __launch_bounds__(256) void dequant_f32(const uint8_t *__restrict__ packed,
                                                    const uint16_t *__restrict__ scale,
-                                                   float *__restrict__ out, int M, int K,
+                                                   float *__restrict__ out, Index quads, int K4,
                                                    int K_pad) {
   __shared__ float lut[16];
   load_lut_lds(lut);
-  const int dpr = K_pad >> 3;  // dwords per row
-  const size_t total = static_cast<size_t>(M) * dpr;
-  for (size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x; i < total;
-       i += static_cast<size_t>(gridDim.x) * 256) {
-    const int r = static_cast<int>(i / dpr);
-    const int d = static_cast<int>(i - static_cast<size_t>(r) * dpr);
-    const uint32_t w = reinterpret_cast<const uint32_t *>(packed)[i];
-    const float s = f16_to_f32(scale[static_cast<size_t>(r) * (K_pad >> 6) + (d >> 3)]);
-    float *o = out + static_cast<size_t>(r) * K + (d << 3);
+  const Index q0 = static_cast<Index>(blockIdx.x) * (256 * kDequantQuads) + threadIdx.x;
+  uint32_t w[kDequantQuads];
+  uint16_t s[kDequantQuads];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if ((d << 3) + j < K) {
-        o[j] = lut[(w >> (4 * j)) & 0xFu] * s;
-      }
+  for (int u = 0; u < kDequantQuads; ++u) {
+    const Index q = min(q0 + static_cast<Index>(256 * u), quads - 1);
+    const Index r = q / static_cast<Index>(K4);
+    const int d = static_cast<int>(q - r * static_cast<Index>(K4));
+    w[u] = reinterpret_cast<const uint16_t *>(packed + static_cast<size_t>(r) * (K_pad >> 1))[d];
+    s[u] = scale[static_cast<size_t>(r) * (K_pad >> 6) + (d >> 4)];
+  }
+#pragma unroll
+  for (int u = 0; u < kDequantQuads; ++u) {
+    const Index q = q0 + static_cast<Index>(256 * u);
+    if (q < quads) {
+      const float f = f16_to_f32(s[u]);
+      const F32x4 v = {lut[w[u] & 0xFu] * f, lut[(w[u] >> 4) & 0xFu] * f, lut[(w[u] >> 8) & 0xFu] * f,
+                       lut[w[u] >> 12] * f};
+      __builtin_nontemporal_store(v, reinterpret_cast<F32x4 *>(out) + q);
+    }
+  }
+}
+
+// Rows that are no whole quads (K % 4 != 0, or an output that is not 16-byte aligned): one weight a
+// store, so a wavefront still writes 256 consecutive bytes, and Q of them a thread: eight where there
+// is work for them (9000x5001 in 45 us, 59 with four, 107 before), four below.
+constexpr int64_t kManyWeights = int64_t{1} << 23;
+
+template <typename Index, int Q>
+__global__ __launch_bounds__(256) void dequant_f32_ragged(const uint8_t *__restrict__ packed,
+                                                          const uint16_t *__restrict__ scale,
+                                                          float *__restrict__ out, Index count, int K,
+                                                          int K_pad) {
+  __shared__ float lut[16];
+  load_lut_lds(lut);
+  const Index i0 = static_cast<Index>(blockIdx.x) * (256 * Q) + threadIdx.x;
+  uint8_t w[Q];
+  uint16_t s[Q];
+  bool odd[Q];
+#pragma unroll
+  for (int u = 0; u < Q; ++u) {
+    const Index i = min(i0 + static_cast<Index>(256 * u), count - 1);
+    const Index r = i / static_cast<Index>(K);
+    const int k = static_cast<int>(i - r * static_cast<Index>(K));
+    w[u] = packed[static_cast<size_t>(r) * (K_pad >> 1) + (k >> 1)];
+    s[u] = scale[static_cast<size_t>(r) * (K_pad >> 6) + (k >> 6)];
+    odd[u] = (k & 1) != 0;
+  }
+#pragma unroll
+  for (int u = 0; u < Q; ++u) {
+    const Index i = i0 + static_cast<Index>(256 * u);
+    if (i < count) {
+      __builtin_nontemporal_store(lut[odd[u] ? w[u] >> 4 : w[u] & 0xF] * f16_to_f32(s[u]), out + i);
     }
   }
 }
@@ -76,61 +136,160 @@ __global__ __launch_bounds__(256) void embed_rows(const uint8_t *__restrict__ pa
   }
 }
 
-// One wavefront per group of 64 weights: lane i owns column 64g + i.
-// Steps are those of the CPU encoder (internal/nf4/nf4.go:129-185): absmax,
-// binary16 scale, divide by the widened scale, clip, nearest level by squared
-// distance in fp32 with the first minimum winning.
+// ---- quantiser ---------------------------------------------------------------
+// The CPU encoder takes the level with the smallest squared distance, in fp32, the first of equal
+// ones (internal/nf4/nf4.go:129-185).  Between two neighbouring levels both distances are monotone
+// in u, also after rounding, so there is one smallest u from which the upper level wins:
+// crossing(j), found here by bisection over binary32 patterns with the same fp32 operations.
+constexpr float level_at(int j) { return __builtin_bit_cast(float, kLevelBits[j]); }
+constexpr float square_from(float u, int j) {
+  const float d = u - level_at(j);
+  return d * d;
+}
+// binary32 patterns in numeric order, for bisection over both signs
+constexpr int64_t ordered(float f) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, f);
+  return (b >> 31) != 0 ? -static_cast<int64_t>(b & 0x7FFFFFFFu) : static_cast<int64_t>(b);
+}
+constexpr float from_ordered(int64_t o) {
+  return __builtin_bit_cast(float, static_cast<uint32_t>(o < 0 ? (0x80000000u | static_cast<uint32_t>(-o)) : static_cast<uint32_t>(o)));
+}
+constexpr float crossing(int j) {
+  int64_t lo = ordered(level_at(j)), hi = ordered(level_at(j + 1));  // lower wins at lo, upper at hi
+  while (hi - lo > 1) {
+    const int64_t mid = lo + (hi - lo) / 2;
+    const float u = from_ordered(mid);
+    if (square_from(u, j + 1) < square_from(u, j)) {
+      hi = mid;
+    } else {
+      lo = mid;
+    }
+  }
+  return from_ordered(hi);
+}
+
+// [-1, 1] in 32 cells of 1/16 (and one for u = 1): neighbouring crossings are further apart than a
+// cell and none lies within 2^-12 of a cell's border, where rounding (u + 1) * 16 could name the
+// neighbour (cells_hold), so a u's code is the number of crossings left of its cell plus one comparison.
+constexpr int kCells = 33;
+struct CellTable {
+  float cross[kCells];  // the crossing inside the cell, or one no u reaches
+  uint32_t below[kCells];
+};
+constexpr CellTable make_cells() {
+  CellTable t{};
+  for (int c = 0; c < kCells; ++c) {
+    t.cross[c] = 4.f;
+    t.below[c] = 0;
+    for (int j = 0; j < 15; ++j) {
+      const float x = (crossing(j) + 1.f) * 16.f;
+      if (x < static_cast<float>(c)) {
+        ++t.below[c];
+      } else if (x < static_cast<float>(c + 1)) {
+        t.cross[c] = crossing(j);
+      }
+    }
+  }
+  return t;
+}
+constexpr bool cells_hold() {
+  for (int j = 0; j < 15; ++j) {
+    const float x = (crossing(j) + 1.f) * 16.f;
+    const float off = x - static_cast<float>(static_cast<int>(x));
+    if (off < 0x1p-12f || off > 1.f - 0x1p-12f) {
+      return false;
+    }
+    if (j > 0 && static_cast<int>(x) == static_cast<int>((crossing(j - 1) + 1.f) * 16.f)) {
+      return false;
+    }
+  }
+  return true;
+}
+static_assert(cells_hold(), "one crossing a cell, none at a border");
+__device__ __constant__ const CellTable kCellTable = make_cells();
+
+// Sixteen lanes a group, four weights a lane (VEC: one 16-byte load; otherwise rows are not whole
+// pieces and the four are loaded one by one), kQuantUnroll groups a lane with all loads first.
+// Steps are those of the CPU encoder: absmax, binary16 scale, divide by the widened scale, clip,
+// nearest level.  Bound by reading the fp32; one weight a lane, a wavefront a group and fifteen
+// squared distances a weight took 302 us at 13824x5120 (vector arithmetic), so 71 (4.5 TB/s; 68 with
+// four or eight groups a lane, which take 7 and 8 us at 1000x1111 against 5).
+constexpr int kQuantUnroll = 2;
+
+template <bool VEC>
 __global__ __launch_bounds__(256) void quantize_groups(const float *__restrict__ src,
                                                        uint8_t *__restrict__ packed,
                                                        uint16_t *__restrict__ scale,
-                                                       int32_t *status, int M, int K, int K_pad) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int ng = K_pad >> 6;
-  const size_t groups = static_cast<size_t>(M) * ng;
-  const size_t wave_id = static_cast<size_t>(blockIdx.x) * (256 / kWave) + (threadIdx.x >> 6);
-  const size_t n_waves = static_cast<size_t>(gridDim.x) * (256 / kWave);
-  for (size_t gi = wave_id; gi < groups; gi += n_waves) {
-    const int r = static_cast<int>(gi / ng);
-    const int g = static_cast<int>(gi - static_cast<size_t>(r) * ng);
-    const int c = (g << 6) + lane;
-    const float v = c < K ? src[static_cast<size_t>(r) * K + c] : 0.f;
-    const bool finite = (f32_to_bits(v) & 0x7F800000u) != 0x7F800000u;
-    if (__any(!finite)) {
+                                                       int32_t *status, int64_t groups, int K,
+                                                       int ng) {
+  __shared__ float cross[kCells];
+  __shared__ uint32_t below[kCells];
+  if (threadIdx.x < kCells) {
+    cross[threadIdx.x] = kCellTable.cross[threadIdx.x];
+    below[threadIdx.x] = kCellTable.below[threadIdx.x];
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 15;
+  const int64_t g0 = static_cast<int64_t>(blockIdx.x) * (16 * kQuantUnroll) + (threadIdx.x >> 4);
+  F32x4 v[kQuantUnroll];
+#pragma unroll
+  for (int n = 0; n < kQuantUnroll; ++n) {
+    const int64_t gi = min(g0 + 16 * n, groups - 1);
+    // (a 32-bit division wherever the index allows it)
+    const int64_t r = groups <= INT32_MAX ? static_cast<int64_t>(static_cast<uint32_t>(gi) / static_cast<uint32_t>(ng)) : gi / ng;
+    const int c = (static_cast<int>(gi - r * ng) << 6) + 4 * lane;
+    const float *p = src + r * K + c;
+    if constexpr (VEC) {
+      v[n] = c < K ? *reinterpret_cast<const F32x4 *>(p) : F32x4{0.f, 0.f, 0.f, 0.f};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[n][e] = c + e < K ? p[e] : 0.f;
+      }
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < kQuantUnroll; ++n) {
+    const int64_t gi = g0 + 16 * n;
+    if (gi >= groups) {
+      break;
+    }
+    uint32_t top = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      // magnitudes as integers order like the numbers, non-finite ones above all finite
+      top = max(top, f32_to_bits(v[n][e]) & 0x7FFFFFFFu);
+    }
+    top = group_max16_u32(top);
+    if (top >= 0x7F800000u) {
       if (lane == 0 && status != nullptr) {
         atomicOr(status, 1);
       }
       continue;
     }
-    float s32 = group_max<64>(fabsf(v));
+    float s32 = bits_to_f32(top);
     if (s32 == 0.f) {
       s32 = 1.f;
     }
-    uint16_t s16 = f32_to_f16_rne(s32);
+    uint16_t s16 = __builtin_bit_cast(uint16_t, static_cast<_Float16>(s32));
     float s = f16_to_f32(s16);
-    const bool bad = ((f32_to_bits(s) & 0x7F800000u) == 0x7F800000u) || !(s > 0.f);
-    if (bad) {
-      s32 = s32 > 65504.f ? 65504.f : 1.f;
-      s16 = f32_to_f16_rne(s32);
+    if (((f32_to_bits(s) & 0x7F800000u) == 0x7F800000u) || !(s > 0.f)) {
+      s16 = s32 > 65504.f ? 0x7BFFu : 0x3C00u;  // the largest finite scale, or one
       s = f16_to_f32(s16);
     }
-    float u = v / s;
-    u = u > 1.f ? 1.f : (u < -1.f ? -1.f : u);
-    uint32_t best_j = 0;
-    float d = u - bits_to_f32(kLutBits[0]);
-    float best = d * d;
+    uint32_t codes = 0;
 #pragma unroll
-    for (uint32_t j = 1; j < 16; ++j) {
-      d = u - bits_to_f32(kLutBits[j]);
-      const float d2 = d * d;
-      if (d2 < best) {
-        best = d2;
-        best_j = j;
-      }
+    for (int e = 0; e < 4; ++e) {
+      float u = v[n][e] / s;
+      u = u > 1.f ? 1.f : (u < -1.f ? -1.f : u);
+      const int cell = static_cast<int>((u + 1.f) * 16.f);
+      codes |= (below[cell] + (u >= cross[cell] ? 1u : 0u)) << (4 * e);
     }
-    const uint32_t hi = static_cast<uint32_t>(__shfl_down(static_cast<int>(best_j), 1, kWave));
-    if ((lane & 1) == 0) {
-      packed[static_cast<size_t>(r) * (K_pad >> 1) + (g << 5) + (lane >> 1)] =
-          static_cast<uint8_t>((hi << 4) | best_j);
+    if (aligned2(packed)) {
+      reinterpret_cast<uint16_t *>(packed)[gi * 16 + lane] = static_cast<uint16_t>(codes);
+    } else {
+      packed[gi * 32 + 2 * lane] = static_cast<uint8_t>(codes);
+      packed[gi * 32 + 2 * lane + 1] = static_cast<uint8_t>(codes >> 8);
     }
     if (lane == 0) {
       scale[gi] = s16;
@@ -163,10 +322,32 @@ extern "C" int chr_nf4_dequant(const chr_nf4_dev_t *w, float *out, void *stream)
   if ((reinterpret_cast<uintptr_t>(w->packed) & 3u) != 0 || !aligned2(w->scale)) {
     return -5;
   }
-  const size_t total = static_cast<size_t>(w->M) * (w->K_pad >> 3);
-  const unsigned blocks = static_cast<unsigned>(std::min<size_t>((total + 255) / 256, 65536));
-  dequant_f32<<<dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
-      w->packed, w->scale, out, w->M, w->K, w->K_pad);
+  const int64_t count = static_cast<int64_t>(w->M) * w->K;
+  const bool whole = (w->K & 3) == 0 && aligned16(out);
+  const int64_t items = whole ? count / 4 : count;
+  const int per = 256 * (whole || count < kManyWeights ? kDequantQuads : 8);
+  const int64_t blocks = (items + per - 1) / per;
+  if (blocks > INT32_MAX) {
+    return -3;
+  }
+  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  // 32-bit indexes (and divisions) unless the last workgroup's would pass 2^32
+  const bool narrow = items < (int64_t{1} << 32) - per;
+  auto run = [&](auto kernel, auto n, int row) {
+    kernel<<<grid, block, 0, st>>>(w->packed, w->scale, out, n, row, w->K_pad);
+  };
+  if (whole && narrow) {
+    run(dequant_f32<uint32_t>, static_cast<uint32_t>(items), w->K / 4);
+  } else if (whole) {
+    run(dequant_f32<uint64_t>, static_cast<uint64_t>(items), w->K / 4);
+  } else if (count < kManyWeights) {
+    run(dequant_f32_ragged<uint32_t, kDequantQuads>, static_cast<uint32_t>(items), w->K);
+  } else if (narrow) {
+    run(dequant_f32_ragged<uint32_t, 8>, static_cast<uint32_t>(items), w->K);
+  } else {
+    run(dequant_f32_ragged<uint64_t, 8>, static_cast<uint64_t>(items), w->K);
+  }
   return launch_rc();
 }
 
@@ -198,11 +379,21 @@ extern "C" int chr_nf4_quantize(const float *src, const chr_nf4_dev_t *dst, int3
   if (const int rc = desc_rc(dst)) {
     return rc;
   }
-  const size_t groups = static_cast<size_t>(dst->M) * (dst->K_pad >> 6);
-  const unsigned blocks = static_cast<unsigned>(std::min<size_t>((groups + 3) / 4, 1u << 20));
-  quantize_groups<<<dim3(blocks), dim3(256), 0, static_cast<hipStream_t>(stream)>>>(
-      src, const_cast<uint8_t *>(dst->packed), const_cast<uint16_t *>(dst->scale), status, dst->M,
-      dst->K, dst->K_pad);
+  const int ng = dst->K_pad >> 6;
+  const int64_t groups = static_cast<int64_t>(dst->M) * ng;
+  const int64_t blocks = (groups + 16 * kQuantUnroll - 1) / (16 * kQuantUnroll);
+  if (blocks > INT32_MAX) {
+    return -3;
+  }
+  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  uint8_t *packed = const_cast<uint8_t *>(dst->packed);
+  uint16_t *scale = const_cast<uint16_t *>(dst->scale);
+  if ((dst->K & 3) == 0 && aligned16(src)) {
+    quantize_groups<true><<<grid, block, 0, st>>>(src, packed, scale, status, groups, dst->K, ng);
+  } else {
+    quantize_groups<false><<<grid, block, 0, st>>>(src, packed, scale, status, groups, dst->K, ng);
+  }
   return launch_rc();
 }
 
