@@ -1,0 +1,684 @@
+// Several whole windows of a prompt at once, with the bits of one window after the other.
+//
+// The chunk prefill (dv2_prefill.hip, gemm_stream64 in nf4_gemm.hip) takes 64 tokens at a time: every
+// window reads and decodes all weights again, in launches too short to fill the chip.  Activations of
+// 48 to 64 layers in bf16 carry any change of a sum's order into every later element, so these
+// kernels keep each sum in the window's order -- the products group by group as the 64-column tile
+// adds them, the norms' squares block by block as that tile and rms_cols add them -- and change only
+// which launch and workgroup a token is computed in.  All data is token-major, [N, features] with
+// N a multiple of 64.
+
+#include "nf4_common.h"
+
+namespace chr {
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 Bf16x8;
+typedef __attribute__((ext_vector_type(4))) float F32x4;
+typedef __attribute__((ext_vector_type(16))) float F32x16;
+typedef __attribute__((ext_vector_type(4))) uint32_t Raw16;
+
+constexpr int kPromptMats = 3;
+constexpr int kWindow = 64;       // tokens of a window, and of a workgroup here
+constexpr int kChunk = 256;       // K of a stage: four groups, as in the 64-column tile
+constexpr int kBlocks = 4;        // 32-row blocks of a wavefront
+constexpr int kTileRows = 2 * kBlocks * 32;
+constexpr int kXStage = kWindow * kChunk * 2;
+constexpr int kScaleStage = 4 * kTileRows * 4;
+constexpr int kXAddr = kPairTableBytes;
+constexpr int kScaleAddr = kXAddr + 2 * kXStage;
+constexpr int kPromptLds = kScaleAddr + 2 * kScaleStage;
+constexpr int kPromptThreads = 512;
+
+struct PromptArgs {
+  const uint8_t *packed[kPromptMats];
+  const uint16_t *scale[kPromptMats];
+  int first[kPromptMats + 1];  // concatenated row each matrix starts at
+  const uint16_t *x;
+  uint16_t *y;
+  float *part;  // [splits][N][rows] (SwiGLU: gate features, then up), or null
+  const uint16_t *bias;
+  int M;        // output features; of one matrix when PAIR
+  int N, K, chunks, split_chunks, tiles_m, tiles_n;
+};
+
+__device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
+  const float a = bf16_to_f32(f32_to_bf16(gate));
+  const float act = bf16_to_f32(f32_to_bf16(a / (1.f + expf(-a))));
+  return f32_to_bf16(act * bf16_to_f32(f32_to_bf16(up)));
+}
+
+// Bound: the matrix cores and the LDS reads beside them where the launch fills the chip (gate and up
+// of 27648 x 5120 at 1792 tokens 1.49 ms, 0.68 PFLOP/s), the table, first loads and the meeting of
+// the sums where a split is a few chunks (5120 x 5120 at 1792 in 3 splits 270 us, 0.35).  The window
+// launches it stands for took 57 ms for a 14B prompt of 512 tokens and 484 for a 32B one of 1791;
+// with it 32 and 308.
+//
+// 256 rows x 64 tokens.  As in the 64-column tile a wavefront sums group w % 4 of every chunk of
+// 256, four 16-wide products a group in the same order of k, scaled into its accumulators group by
+// group; here it holds 128 rows x 64 tokens (RB = 4 row blocks), half w / 4 of the tile, so a lookup
+// serves 64 tokens, x is read from LDS once for 128 rows, and a chunk is 32 products of 32 clocks a
+// wavefront between barriers.  Tokens are the rows of the result: a lane holds one weight row's column
+// and its scale.  PAIR: row blocks alternate between gate and up.
+//
+// Codes: a lane pair fetches the 32 bytes of a row's group, ds_bpermute hands them to the lanes that
+// multiply them; x straight to LDS in 128-byte rows (a token's group), 16-byte pieces XORed with the
+// row's low bits; scales through LDS; all one chunk ahead.  At the end the four wavefronts' sums of
+// an output meet in LDS in group order.
+template <bool PAIR>
+__global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a) {
+  extern __shared__ __align__(16) uint32_t smem[];
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = wave & 3, half = wave >> 2;
+  const int r = lane & 31, h = lane >> 5;
+  const uint32_t lane4 = static_cast<uint32_t>(lane) * 4;
+
+  // each XCD takes a run of tiles, token tiles fastest: workgroups that share weights meet in one L2
+  const int total = static_cast<int>(gridDim.x);
+  const int xcd = static_cast<int>(blockIdx.x) & 7;
+  const int tile = xcd * (total >> 3) + min(xcd, total & 7) + (static_cast<int>(blockIdx.x) >> 3);
+  const int tn = tile % a.tiles_n;
+  const int tms = tile / a.tiles_n;
+  const int tm = tms % a.tiles_m;
+  const int split = tms / a.tiles_m;
+  const int c_lo = split * a.split_chunks;
+  const int c_hi = min(c_lo + a.split_chunks, a.chunks);
+  const int tok0 = tn * kWindow;
+  const int groups = a.chunks * 4;
+
+  // row of a matrix for row `lr` of the tile (clamped: rows past the end are not stored)
+  auto out_row = [&](int lr) {
+    if constexpr (PAIR) {
+      return tm * (kTileRows / 2) + (lr >> 6) * 32 + (lr & 31);
+    } else {
+      return tm * kTileRows + lr;
+    }
+  };
+  auto locate = [&](int lr, int &mat) {
+    int row = min(out_row(lr), a.M - 1);
+    if constexpr (PAIR) {
+      mat = (lr >> 5) & 1;
+    } else {
+      mat = row >= a.first[2] ? 2 : (row >= a.first[1] ? 1 : 0);
+      row -= a.first[mat];
+    }
+    return row;
+  };
+  const uint8_t *wp[kBlocks];
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+    int mat;
+    const int row = locate(half * (kTileRows / 2) + b * 32 + (lane >> 1), mat);
+    const uint8_t *base = mat == 0 ? a.packed[0] : (mat == 1 ? a.packed[1] : a.packed[2]);
+    wp[b] = base + static_cast<size_t>(row) * groups * 32 + g * 32 + (lane & 1) * 16;
+  }
+  const uint16_t *sp;
+  {
+    int mat;
+    const int row = locate(tid >> 1, mat);
+    const uint16_t *base = mat == 0 ? a.scale[0] : (mat == 1 ? a.scale[1] : a.scale[2]);
+    sp = base + static_cast<size_t>(row) * groups + (tid & 1) * 2;
+  }
+  const int from_lane4 = (2 * r + h) * 4;
+  const uint16_t *xp =
+      a.x + static_cast<size_t>(tok0 + wave * 8 + (lane >> 3)) * a.K + ((lane & 7) ^ (lane >> 3)) * 8;
+
+  auto load_x = [&](int c, int buf) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {  // group p of the chunk, tokens 8 wave .. + 8
+      load_to_lds16(xp + c * kChunk + p * kGroup,
+                    static_cast<uint32_t>(kXAddr + buf * kXStage + p * (kWindow * 128) + wave * 1024));
+    }
+  };
+  uint4 cw[kBlocks];
+  uint32_t ns;
+  auto load_w = [&](int c, int b) { cw[b] = *reinterpret_cast<const uint4 *>(wp[b] + static_cast<size_t>(c) * 128); };
+  auto load_s = [&](int c) { ns = *reinterpret_cast<const uint32_t *>(sp + c * 4); };
+  auto store_s = [&](int buf) {
+    const uint32_t at = static_cast<uint32_t>(kScaleAddr + buf * kScaleStage + ((tid & 1) * 2 * kTileRows + (tid >> 1)) * 4);
+    *reinterpret_cast<__attribute__((address_space(3))) float *>(at) = f16_to_f32(static_cast<uint16_t>(ns));
+    *reinterpret_cast<__attribute__((address_space(3))) float *>(at + kTileRows * 4) = f16_to_f32(static_cast<uint16_t>(ns >> 16));
+  };
+
+  load_x(c_lo, 0);
+  load_s(c_lo);
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+    load_w(c_lo, b);
+  }
+  for (int b = wave; b < 256; b += kPromptThreads / kWave) {
+    smem[b * 64 + lane] = bf16_bits_rne(kLutBits[b & 15]) | (bf16_bits_rne(kLutBits[b >> 4]) << 16);
+  }
+  store_s(0);
+  lds_loads_done();
+  __syncthreads();
+
+  F32x16 acc[kBlocks][2];
+#pragma unroll
+  for (int b = 0; b < kBlocks; ++b) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[b][t][v] = 0.f;
+      }
+    }
+  }
+  int buf = 0;
+  for (int c = c_lo; c < c_hi; ++c) {
+    // the requests of the next chunk (the last one asks for its own again: the waits below count
+    // requests); a row block's codes are asked for where the block's own are read
+    const int next = min(c + 1, c_hi - 1);
+    load_x(next, buf ^ 1);
+    load_s(next);
+    asm volatile("" ::: "memory");
+    Bf16x8 xf[2][4];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t at = static_cast<uint32_t>(kXAddr + buf * kXStage + g * (kWindow * 128) + (t * 32 + r) * 128 +
+                                                  (((4 * h + j) ^ (r & 7)) << 4));
+        xf[t][j] = __builtin_bit_cast(Bf16x8, lds0_u128(at));
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b) {
+      uint32_t code[4] = {cw[b].x, cw[b].y, cw[b].z, cw[b].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        code[j] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from_lane4, static_cast<int>(code[j])));
+      }
+      load_w(next, b);
+      const float s = *reinterpret_cast<const __attribute__((address_space(3))) float *>(
+          static_cast<uint32_t>(kScaleAddr + buf * kScaleStage + (g * kTileRows + half * (kTileRows / 2) + b * 32 + r) * 4));
+      Bf16x8 wf[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t w = code[j];
+        const Raw16 f = {pair_at<0>(w, lane4), pair_at<1>(w, lane4), pair_at<2>(w, lane4), pair_at<3>(w, lane4)};
+        wf[j] = __builtin_bit_cast(Bf16x8, f);
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        F32x16 d;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          d[v] = 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[t][j], wf[j], d, 0, 0, 0);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          acc[b][t][v] = fmaf(s, d[v], acc[b][t][v]);
+        }
+      }
+      asm volatile("" ::: "memory");  // keeps a later block's codes and lookups out of this one's registers
+    }
+    store_s(buf ^ 1);
+    lds_loads_done();
+    __syncthreads();
+    buf ^= 1;
+  }
+
+  // the four wavefronts' sums of every output meet in LDS (the table and x are done with), two row
+  // blocks at a time; wavefront (half, g) finishes result rows 8g .. 8g + 7 of each 32 tokens
+  float *sums = reinterpret_cast<float *>(smem);
+  static_assert(2 * 2 * 8 * 16 * kWave * 4 <= kScaleAddr, "the sums of two row blocks fit");
+  const size_t row_floats = static_cast<size_t>(PAIR ? 2 * a.M : a.M);
+#pragma unroll
+  for (int pass = 0; pass < kBlocks / 2; ++pass) {
+    if (pass > 0) {
+      __syncthreads();
+    }
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          sums[(((b * 2 + t) * 8 + wave) * 16 + v) * kWave + lane] = acc[2 * pass + b][t][v];
+        }
+      }
+    }
+    __syncthreads();
+    int row[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      row[b] = out_row(half * (kTileRows / 2) + (2 * pass + b) * 32 + r);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int v = 4 * g + u;
+        float o[2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          o[b] = 0.f;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            o[b] += sums[(((b * 2 + t) * 8 + 4 * half + q) * 16 + v) * kWave + lane];
+          }
+        }
+        const size_t tok = static_cast<size_t>(tok0 + t * 32 + 8 * g + 4 * h + u);
+        if constexpr (PAIR) {
+          if (row[0] < a.M) {
+            if (a.part != nullptr) {
+              float *dst = a.part + (static_cast<size_t>(split) * a.N + tok) * row_floats + row[0];
+              dst[0] = o[0];
+              dst[a.M] = o[1];
+            } else {
+              a.y[tok * a.M + row[0]] = swiglu_bf16(o[0], o[1]);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int b = 0; b < 2; ++b) {
+            if (row[b] < a.M) {
+              if (a.part != nullptr) {
+                a.part[(static_cast<size_t>(split) * a.N + tok) * row_floats + row[b]] = o[b];
+              } else {
+                uint16_t out = f32_to_bf16(o[b]);
+                if (a.bias != nullptr) {
+                  out = f32_to_bf16(bf16_to_f32(out) + bf16_to_f32(a.bias[row[b]]));
+                }
+                a.y[tok * a.M + row[b]] = out;
+              }
+            }
+          }
+        }
+      }
+    }
+  }
+}
+
+__device__ __forceinline__ F32x4 sum_in_order(const float *p, int splits, size_t stride) {
+  F32x4 s = *reinterpret_cast<const F32x4 *>(p);
+#pragma unroll 4
+  for (int j = 1; j < splits; ++j) {
+    const F32x4 v = *reinterpret_cast<const F32x4 *>(p + j * stride);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[e] += v[e];
+    }
+  }
+  return s;
+}
+
+// The splits of a product, four features a thread: bf16 of the sum (+ bias), or silu(gate) * up.
+template <bool PAIR>
+__global__ __launch_bounds__(256) void prompt_reduce(const float *__restrict__ part, int splits, int64_t quads, int M,
+                                                     int64_t count, const uint16_t *__restrict__ bias,
+                                                     uint16_t *__restrict__ y) {
+  const int64_t q = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (q >= quads) {
+    return;
+  }
+  const int64_t at = q * 4;
+  const int m = static_cast<int>(at % M);
+  uint16_t o[4];
+  if constexpr (PAIR) {
+    const float *p = part + (at / M) * 2 * M + m;
+    const F32x4 g = sum_in_order(p, splits, 2 * count), u = sum_in_order(p + M, splits, 2 * count);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = swiglu_bf16(g[e], u[e]);
+    }
+  } else {
+    const F32x4 s = sum_in_order(part + at, splits, count);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      o[e] = f32_to_bf16(s[e]);
+      if (bias != nullptr) {
+        o[e] = f32_to_bf16(bf16_to_f32(o[e]) + bf16_to_f32(bias[m + e]));
+      }
+    }
+  }
+  *reinterpret_cast<uint2 *>(y + at) =
+      make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
+}
+
+// One workgroup a token, a thread 16 consecutive features: x += bf16(sum of the splits) (+ bias), and
+// with norm_w h = RMSNorm(x).  The squares are added as the 64-column tile's column sums and rms_cols
+// add them: a block of 16 rows in the order 0 4 1 5 2 6 3 7 8 12 9 13 10 14 11 15, sixteen chains of
+// every sixteenth block, the chains in order.
+__global__ __launch_bounds__(1024) void prompt_add_rms(const float *__restrict__ part, int splits, size_t stride, int M,
+                                                       const uint16_t *__restrict__ bias, uint16_t *__restrict__ x,
+                                                       const uint16_t *__restrict__ norm_w, float eps,
+                                                       uint16_t *__restrict__ h) {
+  __shared__ float block_sum[1024], chain[16];
+  const int b = threadIdx.x, blocks = M / 16;
+  const size_t at = static_cast<size_t>(blockIdx.x) * M + b * 16;
+  float f[16];
+  if (b < blocks) {
+    uint32_t packed[8];
+    *reinterpret_cast<uint4 *>(packed) = *reinterpret_cast<const uint4 *>(x + at);
+    *reinterpret_cast<uint4 *>(packed + 4) = *reinterpret_cast<const uint4 *>(x + at + 8);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const F32x4 s = sum_in_order(part + at + 4 * q, splits, stride);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 4 * q + e;
+        float t = bf16_to_f32(f32_to_bf16(s[e]));
+        if (bias != nullptr) {
+          t = bf16_to_f32(f32_to_bf16(t + bf16_to_f32(bias[b * 16 + i])));
+        }
+        const float was = (i & 1) != 0 ? bf16_hi(packed[i >> 1]) : bf16_lo(packed[i >> 1]);
+        f[i] = bf16_to_f32(f32_to_bf16(was + t));
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      packed[q] = f32x2_to_bf16x2(f[2 * q], f[2 * q + 1]);
+    }
+    *reinterpret_cast<uint4 *>(x + at) = *reinterpret_cast<const uint4 *>(packed);
+    *reinterpret_cast<uint4 *>(x + at + 8) = *reinterpret_cast<const uint4 *>(packed + 4);
+    float sum = 0.f;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int lo = 8 * (v >> 2) + (v & 3);
+      sum = __fadd_rn(sum, __fmul_rn(f[lo], f[lo]));
+      sum = __fadd_rn(sum, __fmul_rn(f[lo + 4], f[lo + 4]));
+    }
+    block_sum[b] = sum;
+  }
+  if (norm_w == nullptr) {
+    return;
+  }
+  __syncthreads();
+  if (b < 16) {
+    float t = 0.f;
+    for (int i = b; i < blocks; i += 16) {
+      t += block_sum[i];
+    }
+    chain[b] = t;
+  }
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    t += chain[i];
+  }
+  const float inv = rsqrtf(t / static_cast<float>(M) + eps);
+  if (b < blocks) {
+    uint32_t out[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      out[q] = f32x2_to_bf16x2((bf16_to_f32(norm_w[b * 16 + 2 * q]) * f[2 * q]) * inv,
+                               (bf16_to_f32(norm_w[b * 16 + 2 * q + 1]) * f[2 * q + 1]) * inv);
+    }
+    *reinterpret_cast<uint4 *>(h + at) = *reinterpret_cast<const uint4 *>(out);
+    *reinterpret_cast<uint4 *>(h + at + 8) = *reinterpret_cast<const uint4 *>(out + 4);
+  }
+}
+
+// RMSNorm of rows nobody left sums for (the embedding's), squares added as rms_cols adds those of a
+// 64-column tile it reads itself: 128 chains of every 128th feature, eight neighbouring chains by
+// halves, the sixteen results in order.
+__global__ __launch_bounds__(128) void prompt_rms(const uint16_t *__restrict__ x, const uint16_t *__restrict__ w,
+                                                  uint16_t *__restrict__ h, int M, float eps) {
+  __shared__ float part[16];
+  const uint16_t *row = x + static_cast<size_t>(blockIdx.x) * M;
+  uint16_t *dst = h + static_cast<size_t>(blockIdx.x) * M;
+  float ss = 0.f;
+  for (int k = threadIdx.x; k < M; k += 128) {
+    const float v = bf16_to_f32(row[k]);
+    ss = fmaf(v, v, ss);
+  }
+  ss += __shfl_down(ss, 4, 8);
+  ss += __shfl_down(ss, 2, 8);
+  ss += __shfl_down(ss, 1, 8);
+  if ((threadIdx.x & 7) == 0) {
+    part[threadIdx.x >> 3] = ss;
+  }
+  __syncthreads();
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    t += part[i];
+  }
+  const float inv = rsqrtf(t / static_cast<float>(M) + eps);
+  for (int k = threadIdx.x; k < M; k += 128) {
+    dst[k] = f32_to_bf16((bf16_to_f32(w[k]) * bf16_to_f32(row[k])) * inv);
+  }
+}
+
+// Rotate-half RoPE of rows [q | k | v] and the cache write: rope_kv_cols (dv2_prefill.hip) on
+// token-major data, the same arithmetic.  A thread takes W dims of a head's lower half and their
+// partners.
+template <int W>
+__global__ __launch_bounds__(256) void rope_kv_rows(const uint16_t *__restrict__ qkv, int n, int n_q, int n_kv, int hd,
+                                                    int start, uint16_t *__restrict__ q_out,
+                                                    uint16_t *__restrict__ k_cache, uint16_t *__restrict__ v_cache,
+                                                    const uint16_t *__restrict__ cos, const uint16_t *__restrict__ sin) {
+  const int half = hd / 2;
+  const int per_head = half / W;
+  const int64_t items = static_cast<int64_t>(n) * (n_q + n_kv) * per_head;
+  for (int64_t it = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; it < items;
+       it += static_cast<int64_t>(gridDim.x) * 256) {
+    const int d0 = static_cast<int>(it % per_head) * W;
+    const int hid = static_cast<int>((it / per_head) % (n_q + n_kv));
+    const int64_t tok = it / per_head / (n_q + n_kv);
+    const uint16_t *src = qkv + (tok * (n_q + 2 * n_kv) + hid) * hd + d0;
+    const int64_t pos = start + tok;
+    const uint16_t *c = cos + pos * hd + d0, *s = sin + pos * hd + d0;
+    uint16_t lo[W], hi[W];
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      const float a0 = bf16_to_f32(src[e]), a1 = bf16_to_f32(src[half + e]);
+      lo[e] = f32_to_bf16(a0 * bf16_to_f32(c[e]) + (-a1) * bf16_to_f32(s[e]));
+      hi[e] = f32_to_bf16(a1 * bf16_to_f32(c[half + e]) + a0 * bf16_to_f32(s[half + e]));
+    }
+    uint16_t *dst = q_out + (tok * n_q + hid) * hd + d0;
+    if (hid >= n_q) {
+      const int64_t at = (pos * n_kv + (hid - n_q)) * hd + d0;
+      dst = k_cache + at;
+      const uint16_t *v = src + static_cast<int64_t>(n_kv) * hd;
+#pragma unroll
+      for (int e = 0; e < W; ++e) {
+        v_cache[at + e] = v[e];
+        v_cache[at + half + e] = v[half + e];
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      dst[e] = lo[e];
+      dst[half + e] = hi[e];
+    }
+  }
+}
+
+// Checks shared by the products; fills what the matrices decide.
+int prompt_args(const chr_nf4_dev_t *w, int32_t n_mats, bool pair, int32_t N, PromptArgs &a) {
+  if (w == nullptr) {
+    return -1;
+  }
+  if (N < kWindow || N % kWindow != 0) {
+    return -2;
+  }
+  if (n_mats < 1 || n_mats > kPromptMats || (pair && (n_mats != 2 || w[0].M != w[1].M))) {
+    return -3;
+  }
+  int64_t rows = 0;
+  for (int i = 0; i < n_mats; ++i) {
+    if (w[i].M < 1 || w[i].K < 1 || w[i].packed == nullptr || w[i].scale == nullptr || w[i].K != w[0].K) {
+      return -3;
+    }
+    if (!k_pad_ok(w[i].K, w[i].K_pad)) {
+      return -4;
+    }
+    if (!aligned16(w[i].packed) || (reinterpret_cast<uintptr_t>(w[i].scale) & 7u) != 0) {
+      return -5;
+    }
+    a.packed[i] = w[i].packed;
+    a.scale[i] = w[i].scale;
+    a.first[i] = static_cast<int>(rows);
+    rows += w[i].M;
+  }
+  a.split_chunks = window64_chunks(w, n_mats);
+  if (a.split_chunks < 1 || w[0].K % kChunk != 0 || rows > INT32_MAX / 2 || rows % 4 != 0 || w[0].M % 4 != 0) {
+    return -3;
+  }
+  for (int i = n_mats; i <= kPromptMats; ++i) {
+    a.first[i] = static_cast<int>(rows);
+  }
+  a.M = pair ? w[0].M : static_cast<int>(rows);
+  a.N = N;
+  a.K = w[0].K;
+  a.chunks = a.K / kChunk;
+  a.tiles_m = (a.M + kTileRows / (pair ? 2 : 1) - 1) / (kTileRows / (pair ? 2 : 1));
+  a.tiles_n = N / kWindow;
+  return 0;
+}
+
+int prompt_splits(const PromptArgs &a) { return (a.chunks + a.split_chunks - 1) / a.split_chunks; }
+
+template <bool PAIR>
+int prompt_launch(const PromptArgs &a, hipStream_t st) {
+  const int64_t grid = static_cast<int64_t>(a.tiles_m) * a.tiles_n * prompt_splits(a);
+  if (grid > INT32_MAX) {
+    return -3;
+  }
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(&prompt_gemm<PAIR>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                          kPromptLds) != hipSuccess) {
+    (void)hipGetLastError();
+    return -6;
+  }
+  prompt_gemm<PAIR><<<dim3(static_cast<unsigned>(grid)), dim3(kPromptThreads), kPromptLds, st>>>(a);
+  return launch_rc();
+}
+
+}  // namespace
+}  // namespace chr
+
+using namespace chr;
+
+extern "C" int64_t chr_dv2_prompt_ws(const chr_nf4_dev_t *w, int32_t n_mats, int32_t kind, int32_t N) {
+  PromptArgs a{};
+  if (kind < 0 || kind > 2 || prompt_args(w, n_mats, kind == 1, N, a) != 0) {
+    return -1;
+  }
+  const int splits = prompt_splits(a);
+  return splits == 1 && kind != 2 ? 0 : static_cast<int64_t>(splits) * N * a.M * (kind == 1 ? 2 : 1);
+}
+
+extern "C" int chr_dv2_prompt_gemm(const chr_nf4_dev_t *w, int32_t n_mats, int32_t swiglu, const void *x, int32_t N,
+                                   void *y, float *ws, int64_t ws_floats, const void *bias, void *stream) {
+  if (x == nullptr || y == nullptr) {
+    return -1;
+  }
+  PromptArgs a{};
+  const bool pair = swiglu != 0;
+  if (const int rc = prompt_args(w, n_mats, pair, N, a)) {
+    return rc;
+  }
+  if (pair && bias != nullptr) {
+    return -3;
+  }
+  const int splits = prompt_splits(a);
+  const int64_t need = chr_dv2_prompt_ws(w, n_mats, pair ? 1 : 0, N);
+  if (!aligned16(x) || !aligned16(y) || (need > 0 && !aligned16(ws))) {
+    return -5;
+  }
+  if (need > 0 && (ws == nullptr || ws_floats < need)) {
+    return -7;
+  }
+  a.x = static_cast<const uint16_t *>(x);
+  a.y = static_cast<uint16_t *>(y);
+  a.bias = static_cast<const uint16_t *>(bias);
+  a.part = need > 0 ? ws : nullptr;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int rc = pair ? prompt_launch<true>(a, st) : prompt_launch<false>(a, st);
+  if (rc != 0 || need == 0) {
+    return rc;
+  }
+  const int64_t count = static_cast<int64_t>(N) * a.M;
+  const dim3 grid(static_cast<unsigned>((count / 4 + 255) / 256)), block(256);
+  if (pair) {
+    prompt_reduce<true><<<grid, block, 0, st>>>(a.part, splits, count / 4, a.M, count, nullptr, a.y);
+  } else {
+    prompt_reduce<false><<<grid, block, 0, st>>>(a.part, splits, count / 4, a.M, count, a.bias, a.y);
+  }
+  return launch_rc();
+}
+
+extern "C" int chr_dv2_prompt_add_rms(const chr_nf4_dev_t *w, const void *x, int32_t N, void *residual, const void *bias,
+                                      const void *norm_w, float eps, void *h, float *ws, int64_t ws_floats,
+                                      void *stream) {
+  if (x == nullptr || residual == nullptr || (norm_w != nullptr && h == nullptr)) {
+    return -1;
+  }
+  PromptArgs a{};
+  if (const int rc = prompt_args(w, 1, false, N, a)) {
+    return rc;
+  }
+  if (a.M % 16 != 0 || a.M / 16 > 1024) {
+    return -3;
+  }
+  const int64_t need = chr_dv2_prompt_ws(w, 1, 2, N);
+  if (!aligned16(x) || !aligned16(residual) || !aligned16(h) || !aligned16(ws)) {
+    return -5;
+  }
+  if (ws == nullptr || ws_floats < need) {
+    return -7;
+  }
+  a.x = static_cast<const uint16_t *>(x);
+  a.part = ws;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (const int rc = prompt_launch<false>(a, st)) {
+    return rc;
+  }
+  const int threads = (a.M / 16 + kWave - 1) / kWave * kWave;
+  prompt_add_rms<<<dim3(static_cast<unsigned>(N)), dim3(static_cast<unsigned>(threads)), 0, st>>>(
+      ws, prompt_splits(a), static_cast<size_t>(N) * a.M, a.M, static_cast<const uint16_t *>(bias),
+      static_cast<uint16_t *>(residual), static_cast<const uint16_t *>(norm_w), eps, static_cast<uint16_t *>(h));
+  return launch_rc();
+}
+
+extern "C" int chr_dv2_prompt_rms(const void *x, const void *w, void *h, int32_t N, int32_t M, float eps, void *stream) {
+  if (x == nullptr || w == nullptr || h == nullptr) {
+    return -1;
+  }
+  if (N < 1 || M < 1) {
+    return -3;
+  }
+  prompt_rms<<<dim3(static_cast<unsigned>(N)), dim3(128), 0, static_cast<hipStream_t>(stream)>>>(
+      static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w), static_cast<uint16_t *>(h), M, eps);
+  return launch_rc();
+}
+
+extern "C" int chr_dv2_rope_kv_rows(const void *qkv, void *q_out, int32_t N, int32_t n_q, int32_t n_kv, int32_t hd,
+                                    int32_t start, int32_t max_seq, void *k_cache, void *v_cache, const void *cos,
+                                    const void *sin, void *stream) {
+  if (qkv == nullptr || q_out == nullptr || k_cache == nullptr || v_cache == nullptr || cos == nullptr || sin == nullptr) {
+    return -1;
+  }
+  if (N < 1) {
+    return -2;
+  }
+  if (n_q < 1 || n_kv < 1 || hd < 2 || (hd & 1) != 0 || max_seq < 1 || start < 0 || N > max_seq - start) {
+    return -3;
+  }
+  const bool quads = hd % 8 == 0;
+  const int64_t items = static_cast<int64_t>(N) * (n_q + n_kv) * (hd / 2 / (quads ? 4 : 1));
+  const dim3 grid(static_cast<unsigned>(items / 256 < 65535 ? items / 256 + 1 : 65536)), block(256);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  auto run = [&](auto kernel) {
+    kernel<<<grid, block, 0, st>>>(static_cast<const uint16_t *>(qkv), N, n_q, n_kv, hd, start,
+                                   static_cast<uint16_t *>(q_out), static_cast<uint16_t *>(k_cache),
+                                   static_cast<uint16_t *>(v_cache), static_cast<const uint16_t *>(cos),
+                                   static_cast<const uint16_t *>(sin));
+  };
+  if (quads) {
+    run(rope_kv_rows<4>);
+  } else {
+    run(rope_kv_rows<1>);
+  }
+  return launch_rc();
+}

@@ -334,6 +334,10 @@ inline int device_cu_count() {
   return cached;
 }
 
+// How a launch of these matrices side by side at exactly 64 columns splits K: chunks of 256 a split,
+// or 0 where it would not run the tile that adds its groups in that order (nf4_gemm.hip).
+int window64_chunks(const chr_nf4_dev_t *w, int n_mats);
+
 inline int launch_rc() { return hipGetLastError() == hipSuccess ? 0 : -6; }
 
 }  // namespace chr

@@ -2294,6 +2294,7 @@ int gemm_lds_ready() {
 }
 
 }  // namespace
+
 }  // namespace chr
 
 using namespace chr;
@@ -2617,6 +2618,17 @@ int gemm_launch(const chr_nf4_dev_t *const *w, int nseg, const void *x, void *y,
 }
 
 }  // namespace
+
+int window64_chunks(const chr_nf4_dev_t *w, int n_mats) {
+  for (int i = 0; i < n_mats; ++i) {
+    if ((reinterpret_cast<uintptr_t>(w[i].scale) & 7u) != 0) {
+      return 0;
+    }
+  }
+  const StackPlan sp = plan_stack(w, n_mats, kPlanMaxN, /*have_ws=*/1);
+  return sp.stream == 2 ? ceil_div(ceil_div(w[0].K_pad, kWideChunkK), sp.grid_y) : 0;
+}
+
 }  // namespace chr
 
 extern "C" int chr_nf4_gemm_ws_max(const chr_nf4_dev_t *w, const void *x, void *y, int32_t N,

@@ -13,7 +13,8 @@ from __future__ import annotations
 import torch
 
 from ..nf4 import (LIVE_MAX_N, PLAN_MAX_N, dv2_add_cols, dv2_attn_chunk, dv2_gemm_qkv, dv2_gemm_swiglu,
-                   dv2_rms_cols, dv2_rope_kv_cols, dv2_sq_blocks, dv2_swiglu_elems, nf4_gemm)
+                   dv2_prompt_add_rms, dv2_prompt_gemm, dv2_prompt_rms, dv2_prompt_serves, dv2_rms_cols,
+                   dv2_rope_kv_cols, dv2_rope_kv_rows, dv2_sq_blocks, dv2_swiglu_elems, nf4_gemm)
 from .embed import gather_embed
 from .linear import DeviceLinear, DeviceWeights, nf4_linear
 from .ops import causal_attend, rms, split_qkv, swiglu
@@ -94,9 +95,15 @@ class ChunkPrefill:
 
     ``width`` is the chunk ``consume_prompt`` cuts prompts into: up to 64 tokens, twice the
     reference's 32, so the weights are streamed half as often (the 33..64-column GEMM tile
-    dequantises each weight once for both 32-column blocks)."""
+    dequantises each weight once for both 32-column blocks).
+
+    ``run_windows`` takes several whole windows in one token-major pass, layer by layer, with
+    the bits ``run`` leaves on one after the other; ``whole_windows(n)`` says how many of ``n``
+    tokens ``consume_prompt`` sends there."""
 
     MAX_WIDTH = int(PLAN_MAX_N)
+    #: tokens of one pass over several windows: bounds its activations and partials
+    PASS_MAX = 2048
 
     def __init__(self, state: DecodeState, weights: DeviceWeights, *, use_graph: bool = True,
                  width: int | None = None) -> None:
@@ -125,6 +132,52 @@ class ChunkPrefill:
                 self._qkv_bias.append(torch.cat([
                     m.bias if m.bias is not None else torch.zeros(m.M, dtype=torch.bfloat16, device=dev)
                     for m in mats]).contiguous())
+
+    def _serves_windows(self) -> bool:
+        """Whether every product of the model is one the pass over several windows repeats (asked
+        once per distinct shape)."""
+        spec = self.state.spec
+        kinds = {}
+        for ly in self.weights.layers:
+            if ly.gate.bias is not None or ly.up.bias is not None or (ly.wqkv is not None and ly.wqkv.bias is not None):
+                return False
+            qkv = (ly.wqkv,) if ly.wqkv is not None else (ly.q, ly.k, ly.v)
+            for kind, mats in ((0, qkv), (2, (ly.o,)), (1, (ly.gate, ly.up)), (2, (ly.down,))):
+                plain = all(m.packed.is_contiguous() and m.scale.is_contiguous() and m.packed.data_ptr() % 16 == 0
+                            and m.scale.data_ptr() % 8 == 0 for m in mats)
+                kinds.setdefault((kind, mats[0].K, tuple(m.M for m in mats), plain), mats)
+        return (spec.hidden % 16 == 0 and spec.hidden <= 16384
+                and all(plain and dv2_prompt_serves([(m.packed, m.scale, m.M) for m in mats], k, kind)
+                        for (kind, k, _, plain), mats in kinds.items()))
+
+    def whole_windows(self, n: int) -> int:
+        """Tokens in front of an ``n``-token prompt that go through together: its whole windows,
+        where there are two or more of the default width."""
+        whole = int(n) - int(n) % self.MAX_WIDTH
+        if self.width != self.MAX_WIDTH or whole < 2 * self.MAX_WIDTH or not self._serves_windows():
+            return 0
+        return whole
+
+    def _windows_pass(self, ids: torch.Tensor, start: int) -> None:
+        state, weights, spec = self.state, self.weights, self.state.spec
+        n = int(ids.numel())
+        x = gather_embed(weights.embed, ids)                                        # [n, hidden]
+        attn = torch.empty((n, spec.q_dim), dtype=torch.bfloat16, device=x.device)
+        h = dv2_prompt_rms(x, weights.layers[0].norm1, spec.rms_eps)
+        for li, layer in enumerate(weights.layers):
+            qkv = (layer.wqkv,) if layer.wqkv is not None else (layer.q, layer.k, layer.v)
+            y = dv2_prompt_gemm([(m.packed, m.scale, m.M) for m in qkv], h, spec.hidden, bias=self._qkv_bias[li])
+            k_cache, v_cache = state.kv.layer(li)
+            q = dv2_rope_kv_rows(y, spec.n_q, k_cache, v_cache, state.cos, state.sin, start)
+            dv2_attn_chunk(q, k_cache, v_cache, attn, self.first_len, spec.attn_scale, feature_major=False)
+            h = dv2_prompt_add_rms(layer.o.packed, layer.o.scale, attn, layer.o.M, layer.o.K, x, bias=layer.o.bias,
+                                   norm_w=layer.norm2, eps=spec.rms_eps)
+            act = dv2_prompt_gemm([(m.packed, m.scale, m.M) for m in (layer.gate, layer.up)], h, spec.hidden, swiglu=True)
+            last = li + 1 == len(weights.layers)
+            h = dv2_prompt_add_rms(layer.down.packed, layer.down.scale, act, layer.down.M, layer.down.K, x,
+                                   bias=layer.down.bias, norm_w=None if last else weights.layers[li + 1].norm1,
+                                   eps=spec.rms_eps)
+        self.last_hidden.copy_(x[n - 1])
 
     def _chunk(self, n: int) -> None:
         state, weights, spec = self.state, self.weights, self.state.spec
@@ -172,21 +225,40 @@ class ChunkPrefill:
         g.replay()
 
     def run(self, token_ids: torch.Tensor, start: int, *, logits: bool = True) -> None:
+        ids, start = self._checked(token_ids, start)
+        n = int(ids.numel())
+        if n > self.MAX_WIDTH:
+            raise ValueError(f"prefill chunk of {n} tokens exceeds {self.MAX_WIDTH}")
+        self.ids[:n].copy_(ids)
+        self.start.fill_(start)
+        self.first_len.fill_(start + 1)
+        self._replay(n)
+        self._finish(start + n, logits)
+
+    def run_windows(self, token_ids: torch.Tensor, start: int, *, logits: bool = True) -> None:
+        ids, start = self._checked(token_ids, start)
+        n = int(ids.numel())
+        if self.whole_windows(n) != n:
+            raise ValueError(f"{n} tokens are not two or more whole windows this model takes together")
+        for first in range(0, n, self.PASS_MAX):
+            part = ids[first:first + self.PASS_MAX]
+            self.first_len.fill_(start + first + 1)
+            self._windows_pass(part, start + first)
+        self._finish(start + n, logits)
+
+    def _checked(self, token_ids: torch.Tensor, start: int) -> tuple[torch.Tensor, int]:
         state, spec = self.state, self.state.spec
         ids = token_ids.reshape(-1).to(device=state.device, dtype=torch.long)
         n = int(ids.numel())
         if n < 1:
             raise ValueError("prefill chunk must be non-empty")
-        if n > self.MAX_WIDTH:
-            raise ValueError(f"prefill chunk of {n} tokens exceeds {self.MAX_WIDTH}")
         start = int(start)
-        seq = start + n
-        if start < 0 or seq > spec.max_seq:
-            raise ValueError(f"prefill {start}..{seq} exceeds max_seq={spec.max_seq}")
-        self.ids[:n].copy_(ids)
-        self.start.fill_(start)
-        self.first_len.fill_(start + 1)
-        self._replay(n)
+        if start < 0 or start + n > spec.max_seq:
+            raise ValueError(f"prefill {start}..{start + n} exceeds max_seq={spec.max_seq}")
+        return ids, start
+
+    def _finish(self, seq: int, logits: bool) -> None:
+        state, spec = self.state, self.state.spec
         state.position.fill_(seq)
         state.valid_len.fill_(seq)
         if not logits:

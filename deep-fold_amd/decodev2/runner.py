@@ -54,7 +54,15 @@ def consume_prompt(state: DecodeState, weights: DeviceWeights, token_ids: Sequen
     if slot0 + len(ids) > state.spec.max_seq:
         raise ValueError(f"prompt {slot0}+{len(ids)} exceeds max_seq={state.spec.max_seq}")
     on_device = torch.as_tensor(ids, dtype=torch.long).to(state.device)
+    first_window = 0
+    if prefill is not None and chunk is None:
+        # the whole windows in front go through together, with the bits of one after the other
+        first_window = prefill.whole_windows(len(ids))
+        if first_window:
+            prefill.run_windows(on_device[:first_window], slot0, logits=first_window == len(ids))
     for first, past, final in _windows(len(ids), _window_width(state, chunk, prefill)):
+        if past <= first_window:
+            continue
         window = on_device[first:past]
         if prefill is None:
             forward_prefill(state, weights, window, start=slot0 + first, logits=final)

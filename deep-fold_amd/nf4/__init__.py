@@ -60,6 +60,11 @@ __all__ = [
     "dv2_gemm_qkv",
     "dv2_gemm_swiglu",
     "nf4_wide",
+    "dv2_prompt_serves",
+    "dv2_prompt_gemm",
+    "dv2_prompt_add_rms",
+    "dv2_prompt_rms",
+    "dv2_rope_kv_rows",
     "library_path",
 ]
 
@@ -161,6 +166,11 @@ EXPORTS = (
     ("chr_dv2_argmax_commit_ws", ctypes.c_int, [_P, _I, _P, _P, _P, _P, _P, _I, _P, ctypes.c_int64, _P]),
     ("chr_nf4_wide", ctypes.c_int, [_DP, _P, ctypes.c_int64, _I, _P, _P, ctypes.c_int64, _P, _P]),
     ("chr_nf4_wide_ws", ctypes.c_int64, [_DP, _I]),
+    ("chr_dv2_prompt_ws", ctypes.c_int64, [_DP, _I, _I, _I]),
+    ("chr_dv2_prompt_gemm", ctypes.c_int, [_DP, _I, _I, _P, _I, _P, _P, ctypes.c_int64, _P, _P]),
+    ("chr_dv2_prompt_add_rms", ctypes.c_int, [_DP, _P, _I, _P, _P, _P, _F, _P, _P, ctypes.c_int64, _P]),
+    ("chr_dv2_prompt_rms", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P]),
+    ("chr_dv2_rope_kv_rows", ctypes.c_int, [_P, _P, _I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P]),
     ("chr_nf4_abi_version", ctypes.c_int, []),
 )
 
@@ -1076,3 +1086,107 @@ def nf4_wide(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int,
                           _stream())
     _check_rc("chr_nf4_wide", rc)
     return y
+
+
+# ---- several whole windows of a prompt at once -------------------------------------------------
+def _prompt_mats(mats, K: int):  # noqa: N803
+    for packed, scale, m in mats:
+        _check_packed(packed, scale, int(m), K, K)
+        _need(packed.is_contiguous() and scale.is_contiguous(), "packed and scale must be contiguous")
+    return (_Dev * len(mats))(*[_dev(p, s, int(m), K, K) for p, s, m in mats])
+
+
+def dv2_prompt_serves(mats, K: int, kind: int) -> bool:  # noqa: N803
+    """Whether ``dv2_prompt_gemm`` (``kind`` 0, with ``swiglu`` 1) or ``dv2_prompt_add_rms`` (2) takes
+    these matrices ``(packed, scale, M)`` of one K: a 64-column launch of them runs the tile whose sums
+    they repeat."""
+    if K % 256 != 0 or not all(p.is_contiguous() and s.is_contiguous() for p, s, _ in mats):
+        return False
+    return int(_load_ext().chr_dv2_prompt_ws(_prompt_mats(mats, K), len(mats), int(kind), 64)) >= 0
+
+
+def _prompt_x(x: torch.Tensor, K: int) -> int:  # noqa: N803
+    _bf16_cuda(x, "x")
+    _need(x.dim() == 2 and int(x.size(1)) == K and int(x.size(0)) % 64 == 0, f"x must be [64 n, {K}]")
+    return int(x.size(0))
+
+
+def _prompt_ws(devs, n_mats: int, kind: int, n: int, device):
+    floats = int(_load_ext().chr_dv2_prompt_ws(devs, n_mats, kind, n))
+    _need(floats >= 0, "chr_dv2_prompt_ws: these matrices are not served")
+    return floats, torch.empty(floats, dtype=torch.float32, device=device) if floats else None
+
+
+def dv2_prompt_gemm(mats, x: torch.Tensor, K: int, *, bias: torch.Tensor | None = None,  # noqa: N803
+                    swiglu: bool = False) -> torch.Tensor:
+    """Token-major ``[64 n, K] -> [64 n, sum of M]`` through matrices side by side (+ ``bias``), or,
+    with ``swiglu``, ``silu(x W_0^T) * (x W_1^T)``: the bits of ``dv2_gemm_qkv`` / ``nf4_gemm`` /
+    ``dv2_gemm_swiglu`` on every 64 tokens."""
+    n = _prompt_x(x, K)
+    devs = _prompt_mats(mats, K)
+    m_out = int(mats[0][2]) if swiglu else sum(int(m) for _, _, m in mats)
+    _need(bias is None or (bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
+                           and bias.numel() == m_out), f"bias must be contiguous CUDA bf16 of {m_out} elements")
+    floats, ws = _prompt_ws(devs, len(mats), int(swiglu), n, x.device)
+    y = torch.empty((n, m_out), dtype=torch.bfloat16, device=x.device)
+    rc = _load_ext().chr_dv2_prompt_gemm(devs, len(mats), int(swiglu), x.data_ptr(), n, y.data_ptr(),
+                                         None if ws is None else ws.data_ptr(), floats,
+                                         None if bias is None else bias.data_ptr(), _stream())
+    _check_rc("chr_dv2_prompt_gemm", rc)
+    return y
+
+
+def dv2_prompt_add_rms(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int, K: int,  # noqa: N803
+                       residual: torch.Tensor, *, bias: torch.Tensor | None = None,
+                       norm_w: torch.Tensor | None = None, eps: float = 1e-6) -> torch.Tensor | None:
+    """In place ``residual [64 n, M] += x W^T (+ bias)``; with ``norm_w`` returns RMSNorm(residual):
+    the bits of ``nf4_gemm(..., residual=, colsq=)`` and ``dv2_rms_cols(..., colsq=)`` on every 64
+    tokens."""
+    M = int(M)
+    n = _prompt_x(x, K)
+    devs = _prompt_mats([(packed, scale, M)], K)
+    _bf16_cuda(residual, "residual")
+    _need(residual.is_contiguous() and residual.numel() == n * M, f"residual must be {n} contiguous rows of {M}")
+    for t, name in ((bias, "bias"), (norm_w, "norm_w")):
+        _need(t is None or (t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() and t.numel() == M),
+              f"{name} must be contiguous CUDA bf16 of {M} elements")
+    floats, ws = _prompt_ws(devs, 1, 2, n, x.device)
+    h = None if norm_w is None else torch.empty((n, M), dtype=torch.bfloat16, device=x.device)
+    rc = _load_ext().chr_dv2_prompt_add_rms(devs, x.data_ptr(), n, residual.data_ptr(),
+                                            None if bias is None else bias.data_ptr(),
+                                            None if norm_w is None else norm_w.data_ptr(), float(eps),
+                                            None if h is None else h.data_ptr(), ws.data_ptr(), floats, _stream())
+    _check_rc("chr_dv2_prompt_add_rms", rc)
+    return h
+
+
+def dv2_prompt_rms(x: torch.Tensor, w: torch.Tensor, eps: float) -> torch.Tensor:
+    """RMSNorm of every row of ``x [n, M]``: the bits of ``dv2_rms_cols`` on whole 64-token windows."""
+    _bf16_cuda(x, "x")
+    _bf16_cuda(w, "w")
+    _need(x.dim() == 2 and x.is_contiguous() and w.numel() == x.size(1), "x must be [n, M] and w hold M elements")
+    h = torch.empty_like(x)
+    _check_rc("chr_dv2_prompt_rms", _load_ext().chr_dv2_prompt_rms(x.data_ptr(), w.data_ptr(), h.data_ptr(), int(x.size(0)),
+                                                                   int(x.size(1)), float(eps), _stream()))
+    return h
+
+
+def dv2_rope_kv_rows(qkv, n_q: int, k_cache, v_cache, cos, sin, start: int) -> torch.Tensor:
+    """Rows ``[q | k | v]`` of n tokens at positions ``start ..``: returns rotated q ``[n, n_q*hd]`` and
+    writes rotated k and v to their cache rows, as ``dv2_rope_kv_cols`` does."""
+    _bf16_cuda(qkv, "qkv")
+    _need(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.dim() == 3 and v_cache.shape == k_cache.shape
+          and k_cache.dtype == torch.bfloat16 and v_cache.dtype == torch.bfloat16 and k_cache.is_cuda,
+          "caches must be contiguous CUDA bf16 [max_seq,n_kv,hd]")
+    max_seq, n_kv, hd = (int(t) for t in k_cache.shape)
+    for t, name in ((cos, "cos"), (sin, "sin")):
+        _bf16_cuda(t, name)
+        _need(t.is_contiguous() and t.numel() >= max_seq * hd, f"{name} must hold max_seq*hd elements")
+    _need(qkv.dim() == 2 and qkv.is_contiguous() and int(qkv.size(1)) == (int(n_q) + 2 * n_kv) * hd,
+          "qkv must be contiguous [n, (n_q + 2 n_kv)*hd]")
+    n = int(qkv.size(0))
+    q = torch.empty((n, int(n_q) * hd), dtype=torch.bfloat16, device=qkv.device)
+    rc = _load_ext().chr_dv2_rope_kv_rows(qkv.data_ptr(), q.data_ptr(), n, int(n_q), n_kv, hd, int(start), max_seq,
+                                          k_cache.data_ptr(), v_cache.data_ptr(), cos.data_ptr(), sin.data_ptr(), _stream())
+    _check_rc("chr_dv2_rope_kv_rows", rc)
+    return q

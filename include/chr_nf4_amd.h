@@ -424,6 +424,33 @@ int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_
                  float *ws, int64_t ws_floats, const void *bias, void *stream);
 int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N);
 
+/* ---- Several whole windows of a prompt at once, token-major ------------------------------------
+ * What the entries of the chunked prefill compute for one 64-token window after the other, for
+ * N = 64 k tokens in one launch (-2 otherwise), with the same bits: every sum in the order the
+ * 64-column tile and chr_dv2_rms_cols(_sq) add it.  x [N, K], y, residual and h [N, M], all 16-byte
+ * aligned (-5, as is ws).  -3 where a 64-column launch of the matrices would not run that tile.
+ * No counterpart in the reference's C-ABI. */
+
+/* fp32 elements a launch needs: kind 0 chr_dv2_prompt_gemm, 1 with swiglu, 2 chr_dv2_prompt_add_rms;
+ * -1: not served. */
+int64_t chr_dv2_prompt_ws(const chr_nf4_dev_t *w, int32_t n_mats, int32_t kind, int32_t N);
+/* chr_dv2_gemm_qkv / chr_dv2_gemm_add without a residual (up to three matrices side by side, w an
+ * array, y rows [M0 | M1 | M2]) or, with swiglu, chr_dv2_gemm_swiglu. */
+int chr_dv2_prompt_gemm(const chr_nf4_dev_t *w, int32_t n_mats, int32_t swiglu, const void *x,
+                        int32_t N, void *y, float *ws, int64_t ws_floats, const void *bias,
+                        void *stream);
+/* chr_dv2_gemm_add_sq in place on residual, then, with norm_w, chr_dv2_rms_cols_sq into h. */
+int chr_dv2_prompt_add_rms(const chr_nf4_dev_t *w, const void *x, int32_t N, void *residual,
+                           const void *bias, const void *norm_w, float eps, void *h, float *ws,
+                           int64_t ws_floats, void *stream);
+/* chr_dv2_rms_cols of whole 64-token windows. */
+int chr_dv2_prompt_rms(const void *x, const void *w, void *h, int32_t N, int32_t M, float eps,
+                       void *stream);
+/* chr_dv2_rope_kv_cols on rows [q | k | v] of any N tokens at positions start .. (-3 past the cache). */
+int chr_dv2_rope_kv_rows(const void *qkv, void *q_out, int32_t N, int32_t n_q, int32_t n_kv,
+                         int32_t hd, int32_t start, int32_t max_seq, void *k_cache, void *v_cache,
+                         const void *cos, const void *sin, void *stream);
+
 /* Library version, for the loader's sanity check. */
 int chr_nf4_abi_version(void);
 
