@@ -491,6 +491,67 @@ __device__ __forceinline__ bool x_item(int N, int I, int lane, int &kp, int &q) 
   return I < N / 4;  // 128 k pairs x N/8 vectors = 16 N items = N/4 instructions
 }
 
+// ---- activations of any column count ---------------------------------------------------------
+// The rows of a K tile are one contiguous span of x, whatever N is, and start 16-byte aligned (k0 is
+// a multiple of 256, x aligned): they are fetched as 16-byte pieces and taken apart on the way into
+// LDS.  Element by element, each load waited for before the next, a tile of 63 columns took four
+// times one of 64 (27648x5120: 239 us against 58; as pieces 82, and 23 columns 40 for 61).  P pieces a thread of THREADS; the last elements,
+// short of a piece, are loaded where they are stored (they end x: nothing may be read behind them).
+template <int P, int THREADS>
+__device__ __forceinline__ void fetch_flat(uint32_t *d, const uint16_t *__restrict__ x, int k0, int span, int K,
+                                           int N, int tid) {
+  const int full = (min(span, K - k0) * N) >> 3;
+  if (full == 0) {
+    return;
+  }
+  const uint4 *src = reinterpret_cast<const uint4 *>(x + static_cast<size_t>(k0) * N);
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    const uint4 t = src[min(tid + u * THREADS, full - 1)];
+    d[4 * u + 0] = t.x;
+    d[4 * u + 1] = t.y;
+    d[4 * u + 2] = t.z;
+    d[4 * u + 3] = t.w;
+  }
+}
+
+// Element f of the span is row f / N, column f % N; rows from K on are zeros.
+template <int P, int THREADS, int XS>
+__device__ __forceinline__ void scatter_flat(const uint32_t *d, const uint16_t *__restrict__ x, uint16_t *xs, int k0,
+                                             int span, int K, int N, int tid) {
+  const int rows = min(span, K - k0);
+  const int count = rows * N;
+  const int full = count >> 3;
+  // exact for f < 2^21: the quotient is off by f * (magic * N - 2^32) / 2^32 < 1 / N
+  const uint32_t magic = static_cast<uint32_t>(((1ull << 32) + static_cast<uint32_t>(N) - 1) / static_cast<uint32_t>(N));
+#pragma unroll
+  for (int u = 0; u < P; ++u) {
+    const int piece = tid + u * THREADS;
+    if (piece < full) {
+      const int f = 8 * piece;
+      int kk = static_cast<int>(__umulhi(static_cast<uint32_t>(f), magic));
+      int n = f - kk * N;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        xs[n * XS + kk] = static_cast<uint16_t>(d[4 * u + (e >> 1)] >> (16 * (e & 1)));
+        ++n;
+        const bool wrap = n == N;
+        n = wrap ? 0 : n;
+        kk += wrap ? 1 : 0;
+      }
+    }
+  }
+  const int f = 8 * full + tid;
+  if (f < count) {
+    const int kk = static_cast<int>(__umulhi(static_cast<uint32_t>(f), magic));
+    xs[(f - kk * N) * XS + kk] = x[static_cast<size_t>(k0) * N + f];
+  }
+  for (int i = tid; i < (span - rows) * N; i += THREADS) {
+    const int kk = static_cast<int>(__umulhi(static_cast<uint32_t>(i), magic));
+    xs[(i - kk * N) * XS + rows + kk] = 0;
+  }
+}
+
 template <bool VEC, int NB>
 __device__ __forceinline__ void fetch_x(XRegs<NB> &r, const uint16_t *__restrict__ x, int k0, int K,
                                         int N, int tid) {
@@ -524,7 +585,7 @@ __device__ __forceinline__ void fetch_x(XRegs<NB> &r, const uint16_t *__restrict
       r.d[8 * rep + 7] = b.w;
     }
   } else {
-    (void)r;
+    fetch_flat<4 * NB, kGroupThreads>(r.d, x, k0, kBK, K, N, tid);
   }
 }
 
@@ -548,13 +609,7 @@ __device__ __forceinline__ void scatter_x(const XRegs<NB> &r, const uint16_t *__
       }
     }
   } else {
-    // any N, any alignment: element by element
-    for (int i = tid; i < kBK * N; i += kGroupThreads) {
-      const int kk = i / N;
-      const int n = i - kk * N;
-      const int k = k0 + kk;
-      xs[n * kXStride + kk] = k < K ? x[static_cast<size_t>(k) * N + n] : static_cast<uint16_t>(0);
-    }
+    scatter_flat<4 * NB, kGroupThreads, kXStride>(r.d, x, xs, k0, kBK, K, N, tid);
   }
 }
 
@@ -845,6 +900,12 @@ __global__ __launch_bounds__(kRowsBlock) void gemm_rows(const GemmSegs segs,
     }
   }
 
+  constexpr int FP = NC * TPS;  // 16-byte pieces of a slice of 16 NC columns, a thread
+  uint32_t xf[VEC ? 1 : 4 * FP];
+  if constexpr (!VEC) {
+    fetch_flat<FP, kRowsBlock>(xf, x, k0, SK, K, N, tid);
+  }
+
   // 2. weight and scale requests, the whole slice of this lane's row
   const int row_bytes = K_pad >> 1;
   const int groups = K_pad >> 6;
@@ -891,13 +952,7 @@ __global__ __launch_bounds__(kRowsBlock) void gemm_rows(const GemmSegs segs,
       }
     }
   } else {
-    // any N, any alignment: element by element
-    for (int i = tid; i < SK * N; i += kRowsBlock) {
-      const int kk = i / N;
-      const int n = i - kk * N;
-      const int k = k0 + kk;
-      xs[n * XS + kk] = k < K ? x[static_cast<size_t>(k) * N + n] : static_cast<uint16_t>(0);
-    }
+    scatter_flat<FP, kRowsBlock, XS>(xf, x, xs, k0, SK, K, N, tid);
   }
   __syncthreads();
 
