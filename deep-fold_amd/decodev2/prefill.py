@@ -85,6 +85,12 @@ def _gemm_cols(mat: DeviceLinear, x: torch.Tensor, residual: torch.Tensor | None
     return False if colsq is not None else y
 
 
+def _plain(mats) -> bool:
+    """Blobs laid out and aligned as the several-window products read them."""
+    return all(m.packed.is_contiguous() and m.scale.is_contiguous() and m.packed.data_ptr() % 16 == 0
+               and m.scale.data_ptr() % 8 == 0 for m in mats)
+
+
 class ChunkPrefill:
     """Feature-major prefill of one request's prompt chunks.
 
@@ -134,18 +140,16 @@ class ChunkPrefill:
                     for m in mats]).contiguous())
 
     def _serves_windows(self) -> bool:
-        """Whether every product of the model is one the pass over several windows repeats (asked
-        once per distinct shape)."""
+        """Whether the products of the model are ones the pass over several windows repeats (asked
+        once per distinct shape); gate and up may also go through it window by window."""
         spec = self.state.spec
         kinds = {}
         for ly in self.weights.layers:
             if ly.gate.bias is not None or ly.up.bias is not None or (ly.wqkv is not None and ly.wqkv.bias is not None):
                 return False
             qkv = (ly.wqkv,) if ly.wqkv is not None else (ly.q, ly.k, ly.v)
-            for kind, mats in ((0, qkv), (2, (ly.o,)), (1, (ly.gate, ly.up)), (2, (ly.down,))):
-                plain = all(m.packed.is_contiguous() and m.scale.is_contiguous() and m.packed.data_ptr() % 16 == 0
-                            and m.scale.data_ptr() % 8 == 0 for m in mats)
-                kinds.setdefault((kind, mats[0].K, tuple(m.M for m in mats), plain), mats)
+            for kind, mats in ((0, qkv), (2, (ly.o,)), (2, (ly.down,))):
+                kinds.setdefault((kind, mats[0].K, tuple(m.M for m in mats), _plain(mats)), mats)
         return (spec.hidden % 16 == 0 and spec.hidden <= 16384
                 and all(plain and dv2_prompt_serves([(m.packed, m.scale, m.M) for m in mats], k, kind)
                         for (kind, k, _, plain), mats in kinds.items()))
@@ -164,6 +168,7 @@ class ChunkPrefill:
         x = gather_embed(weights.embed, ids)                                        # [n, hidden]
         attn = torch.empty((n, spec.q_dim), dtype=torch.bfloat16, device=x.device)
         h = dv2_prompt_rms(x, weights.layers[0].norm1, spec.rms_eps)
+        together: dict = {}  # gate and up by shape: whether a launch takes all windows of them
         for li, layer in enumerate(weights.layers):
             qkv = (layer.wqkv,) if layer.wqkv is not None else (layer.q, layer.k, layer.v)
             y = dv2_prompt_gemm([(m.packed, m.scale, m.M) for m in qkv], h, spec.hidden, bias=self._qkv_bias[li])
@@ -172,7 +177,17 @@ class ChunkPrefill:
             dv2_attn_chunk(q, k_cache, v_cache, attn, self.first_len, spec.attn_scale, feature_major=False)
             h = dv2_prompt_add_rms(layer.o.packed, layer.o.scale, attn, layer.o.M, layer.o.K, x, bias=layer.o.bias,
                                    norm_w=layer.norm2, eps=spec.rms_eps)
-            act = dv2_prompt_gemm([(m.packed, m.scale, m.M) for m in (layer.gate, layer.up)], h, spec.hidden, swiglu=True)
+            gate, up = ((m.packed, m.scale, m.M) for m in (layer.gate, layer.up))
+            shape = (layer.gate.M, layer.up.M, _plain((layer.gate, layer.up)))
+            if shape not in together:
+                together[shape] = shape[-1] and dv2_prompt_serves([gate, up], spec.hidden, 1)
+            if together[shape]:
+                act = dv2_prompt_gemm([gate, up], h, spec.hidden, swiglu=True)
+            else:
+                act = torch.empty((n, layer.gate.M), dtype=torch.bfloat16, device=x.device)
+                for lo in range(0, n, self.MAX_WIDTH):
+                    at = slice(lo, lo + self.MAX_WIDTH)
+                    act[at] = dv2_gemm_swiglu(gate, up, h[at].t().contiguous()).t()
             last = li + 1 == len(weights.layers)
             h = dv2_prompt_add_rms(layer.down.packed, layer.down.scale, act, layer.down.M, layer.down.K, x,
                                    bias=layer.down.bias, norm_w=None if last else weights.layers[li + 1].norm1,

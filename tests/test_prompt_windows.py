@@ -132,8 +132,8 @@ def test_rope_rows_store_what_the_columns_store(n, n_q, n_kv, hd, start):
     assert torch.equal(caches[0], caches[2]) and torch.equal(caches[1], caches[3])
 
 
-#: two layers of the 14B, 20B and 32B decoders (one with fused wqkv, one whose SwiGLU is split)
-SPECS = [(dv2.QWEN25_14B, 200, 0), (dv2.INTERNLM25_20B, 130, 9), (dv2.QWEN25_32B, 128, 70)]
+#: two layers of the decoders: gate and up window by window, plain, with fused wqkv and a split SwiGLU, long K
+SPECS = [(dv2.QWEN25_3B, 192, 5), (dv2.QWEN25_14B, 200, 0), (dv2.INTERNLM25_20B, 130, 9), (dv2.QWEN25_32B, 128, 70)]
 
 
 @pytest.mark.gpu
