@@ -424,3 +424,32 @@ extern "C" int chr_dv2_argmax_commit_ws(const void *logits, int32_t n, void *nex
       static_cast<uint8_t *>(finished), static_cast<const int64_t *>(eos_id), commit);
   return launch_rc();
 }
+
+extern "C" int chr_dv2_step_layer(const chr_dv2_layer_t *layer, const chr_dv2_step_t *step, void *stream) {
+  if (layer == nullptr || step == nullptr) {
+    return -1;
+  }
+  const chr_dv2_layer_t &l = *layer;
+  const chr_dv2_step_t &s = *step;
+  if (l.qkv_rows != 1 && l.qkv_rows != 3) {
+    return -3;
+  }
+  int rc = l.qkv_rows == 1
+               ? chr_dv2_gemv_sumsq(&l.q, s.x, s.q, stream, l.q_bias, l.norm1, s.eps, s.sumsq, nullptr)
+               : chr_dv2_gemv_qkv_sumsq(&l.q, &l.k, &l.v, s.x, s.q, s.k, s.v, l.q_bias, l.k_bias, l.v_bias, stream,
+                                        l.norm1, s.eps, s.sumsq);
+  if (rc == 0) {
+    rc = chr_dv2_attn_parts(s.q, l.k_cache, l.v_cache, s.valid_len, s.state, s.n_q, s.n_kv, s.hd, s.n_parts, s.n_waves,
+                            s.attn_scale, stream, s.k, s.v, s.cos, s.sin, s.position, s.max_seq);
+  }
+  if (rc == 0) {
+    rc = chr_dv2_gemv_attn_sumsq(&l.o, s.state, s.n_q, s.hd, s.n_parts, s.x, s.x, stream, s.sumsq);
+  }
+  if (rc == 0) {
+    rc = chr_dv2_gemv_swiglu_sumsq(&l.gate, &l.up, s.x, s.down_in, stream, l.norm2, s.eps, s.sumsq);
+  }
+  if (rc == 0) {
+    rc = chr_dv2_gemv_sumsq(&l.down, s.down_in, s.x, stream, s.x, nullptr, 0.f, nullptr, s.sumsq);
+  }
+  return rc;
+}

@@ -27,8 +27,8 @@ import os
 
 import torch
 
-from ..nf4 import (ATTN_SPLIT, dv2_attn_parts, dv2_begin_step, dv2_gemv_attn, dv2_sumsq_ok, nf4_attn,
-                   nf4_gemv, nf4_qkv, nf4_rms, nf4_swiglu)
+from ..nf4 import (ATTN_SPLIT, dv2_attn_parts, dv2_begin_step, dv2_gemv_attn, dv2_step_args, dv2_step_layer,
+                   dv2_sumsq_ok, nf4_attn, nf4_gemv, nf4_qkv, nf4_rms, nf4_swiglu)
 from .embed import PackedEmbed, gather_embed
 from .linear import DeviceLayer, DeviceLinear, DeviceWeights
 from .state import DecodeState
@@ -110,6 +110,29 @@ def _attend_into_o(state: DecodeState, li: int, layer: DeviceLayer, q, k, v,
         d.add_(o.bias)
 
 
+def _layers_native(state: DecodeState, weights: DeviceWeights, sq: torch.Tensor) -> None:
+    """The layers of a step whose sums of squares are handed over: the same five launches a layer as
+    the loop of ``_forward_calls``, issued by one library call (a 3B layer took 75 us of host time in
+    separate calls, its launches take the device about 30)."""
+    spec, ar = state.spec, state.arena
+    if weights.layers[0].wqkv is not None:
+        flat = ar.qkv.view(-1)
+        q, k, v = flat[: spec.q_dim], flat[spec.q_dim: spec.q_dim + spec.kv_dim], flat[spec.q_dim + spec.kv_dim:]
+    else:
+        q, k, v = ar.q.view(-1), ar.k.view(-1), ar.v.view(-1)
+    step = dv2_step_args(ar.x, q, k, v, ar.down_in, ar.attn_state, sq, state.valid_len, state.position, state.cos,
+                         state.sin, spec.n_q, spec.n_kv, spec.head_dim, spec.max_seq, spec.attn_scale, spec.rms_eps)
+    hidden, down_elems = ar.x.numel(), ar.down_in.numel()
+    for li, ly in enumerate(weights.layers):
+        kc, vc = state.kv.layer(li)
+        if ly.wqkv is not None:
+            first, biases = (ly.wqkv, None, None), (ly.wqkv.bias, None, None)
+        else:
+            first, biases = (ly.q, ly.k, ly.v), (ly.q.bias, ly.k.bias, ly.v.bias)
+        dv2_step_layer(step, hidden, (*first, ly.o, ly.gate, ly.up, ly.down), biases, ly.norm1, ly.norm2, down_elems,
+                       kc, vc)
+
+
 def _attend(state: DecodeState, li: int, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
     spec = state.spec
     ar = state.arena
@@ -136,7 +159,10 @@ def _forward_calls(state: DecodeState, weights: DeviceWeights, commit: bool, fol
     else:
         gather_embed(emb, state.token.reshape(1), out=ar.x)
         state.kv.mark_written(state.position)
-    for li, layer in enumerate(weights.layers):
+    native = sq is not None and len({ly.wqkv is None for ly in weights.layers}) == 1
+    if native:
+        _layers_native(state, weights, sq)
+    for li, layer in enumerate(() if native else weights.layers):
         if fold:
             q, k, v = _qkv(state, layer, ar.x, layer.norm1, sq)
         else:

@@ -22,7 +22,7 @@ import torch
 from torch import nn
 
 from ..chr0.loader import ChrMatrix
-from ..nf4 import LIVE_MAX_N, nf4_gemm, nf4_wide
+from ..nf4 import LIVE_MAX_N, nf4_gemm, nf4_gemv, nf4_wide
 from ..nf4.plan import k_pad
 from ..ring.host_image import HostImage
 
@@ -47,7 +47,7 @@ def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: in
         raise ValueError(f"x{tuple(x.shape)} holds no token to multiply")
     rows = x.to(torch.bfloat16).reshape(n, K)
     if n == 1:
-        out = nf4_gemm(packed, scale, rows.reshape(K, 1), M, K, K_pad).reshape(1, M)
+        out = nf4_gemv(packed, scale, rows.reshape(K), M, K, K_pad).reshape(1, M)
     elif M * K >= WIDE_MIN_CODES:
         # the launch adds a bias it can add as torch would: bf16, one element a feature, no graph
         folds = (bias is not None and bias.dtype == torch.bfloat16 and tuple(bias.shape) == (M,)

@@ -51,6 +51,8 @@ __all__ = [
     "dv2_sumsq_ok",
     "dv2_sumsq_parts",
     "dv2_attn",
+    "dv2_step_args",
+    "dv2_step_layer",
     "dv2_rms_cols",
     "dv2_sq_blocks",
     "dv2_rope_kv_cols",
@@ -104,6 +106,23 @@ class _Plan(ctypes.Structure):
         ("smem_bytes", ctypes.c_int32),
         ("ws_floats", ctypes.c_int64),
     ]
+
+
+class _Layer(ctypes.Structure):
+    """``chr_dv2_layer_t``."""
+
+    _fields_ = ([(n, _Dev) for n in ("q", "k", "v", "o", "gate", "up", "down")]
+                + [(n, ctypes.c_void_p) for n in ("q_bias", "k_bias", "v_bias", "norm1", "norm2", "k_cache", "v_cache")]
+                + [("qkv_rows", ctypes.c_int32)])
+
+
+class _Step(ctypes.Structure):
+    """``chr_dv2_step_t``."""
+
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "q", "k", "v", "down_in", "state", "sumsq", "valid_len",
+                                                "position", "cos", "sin")]
+                + [(n, ctypes.c_int32) for n in ("n_q", "n_kv", "hd", "n_parts", "n_waves", "max_seq")]
+                + [("attn_scale", ctypes.c_float), ("eps", ctypes.c_float)])
 
 
 _PLAN_KEYS = tuple(name for name, _ in _Plan._fields_)
@@ -160,6 +179,7 @@ EXPORTS = (
     ("chr_dv2_gemm_qkv", ctypes.c_int, [_DP, _DP, _DP, _P, _P, _I, _P, ctypes.c_int64, _P, _P]),
     ("chr_dv2_gemm_swiglu_ws", ctypes.c_int64, [_DP, _DP, _I]),
     ("chr_dv2_gemm_swiglu", ctypes.c_int, [_DP, _DP, _P, _P, _I, _P, ctypes.c_int64, _P]),
+    ("chr_dv2_step_layer", ctypes.c_int, [ctypes.POINTER(_Layer), ctypes.POINTER(_Step), _P]),
     ("chr_dv2_mark_written", ctypes.c_int, [_P, _P, _P]),
     ("chr_dv2_argmax_commit", ctypes.c_int, [_P, _I, _P, _P, _P, _P, _P, _I, _P]),
     ("chr_dv2_argmax_ws_bytes", ctypes.c_int64, []),
@@ -220,7 +240,8 @@ def _check_rc(what: str, rc: int) -> None:
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle alone: a torch.cuda.Stream object around it costs a launch's worth of host time
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -229,6 +250,11 @@ def _need(cond: bool, msg: str) -> None:
 
 
 def _check_packed(packed, scale, M: int, K: int, K_pad: int, name: str = "") -> None:
+    # everything asked for below, without building the messages: a decode step asks 250 times
+    if (packed.dtype is torch.uint8 and scale.dtype is torch.float16 and packed.is_cuda and scale.is_cuda
+            and M >= 1 and K >= 1 and K_pad == (K + 63) // 64 * 64
+            and packed.numel() >= M * (K_pad // 2) and scale.numel() >= M * (K_pad // 64)):
+        return
     pre = f"{name} " if name else ""
     _need(packed.is_cuda and scale.is_cuda, f"{pre}packed/scale must be CUDA tensors")
     _need(packed.dtype == torch.uint8, f"{pre}packed must be uint8")
@@ -262,13 +288,14 @@ def _as_kvec(x: torch.Tensor, K: int) -> torch.Tensor:
 
 def _opt_bf16(t, numel: int, what: str, exact: bool):
     """Optional tensor -> (keepalive, pointer or None)."""
-    if t is None or t.numel() == 0:
+    if t is None or (have := t.numel()) == 0:
         return None, None
-    _need(t.is_cuda, f"{what} must be CUDA")
-    if exact:
-        _need(t.numel() == numel, f"{what} numel must equal {numel}")
-    else:
-        _need(t.numel() >= numel, f"{what} too small")
+    if not t.is_cuda:
+        raise RuntimeError(f"{what} must be CUDA")
+    if exact and have != numel:
+        raise RuntimeError(f"{what} numel must equal {numel}")
+    if have < numel:
+        raise RuntimeError(f"{what} too small")
     keep = t.contiguous()
     if keep.dtype != torch.bfloat16:
         keep = keep.to(torch.bfloat16)
@@ -403,10 +430,12 @@ def _opt_sumsq(t: torch.Tensor | None, what: str):
     """Device pointer of a sum-of-squares hand-over buffer, or None."""
     if t is None:
         return None
-    _need(t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
-          and t.numel() >= dv2_sumsq_parts() and t.data_ptr() % 16 == 0,
-          f"{what} must be a contiguous, 16-byte aligned CUDA float32 tensor of dv2_sumsq_parts() elements")
-    return t.data_ptr()
+    at = t.data_ptr()
+    if not (t.is_cuda and t.dtype == torch.float32 and t.is_contiguous() and t.numel() >= dv2_sumsq_parts()
+            and at % 16 == 0):
+        raise RuntimeError(f"{what} must be a contiguous, 16-byte aligned CUDA float32 tensor of "
+                           "dv2_sumsq_parts() elements")
+    return at
 
 
 def nf4_gemv(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int, K: int,  # noqa: N803
@@ -868,8 +897,8 @@ def dv2_gemv_attn(packed: torch.Tensor, scale: torch.Tensor, state: torch.Tensor
     _need(state.is_cuda and state.dtype == torch.float32 and state.is_contiguous()
           and state.numel() >= int(n_q) * int(n_parts) * (int(hd) + 4), "attention state buffer too small")
     for t, name in ((out, "out"), (add, "add")):
-        _need(t is None or (t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous()
-                            and t.numel() >= M), f"{name} must be contiguous CUDA bf16 with M elements")
+        if not (t is None or (t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() and t.numel() >= M)):
+            raise RuntimeError(f"{name} must be contiguous CUDA bf16 with M elements")
     w = _dev(packed, scale, M, K, K_pad)
     if sumsq_out is None:
         rc = _load_ext().chr_dv2_gemv_attn(ctypes.byref(w), state.data_ptr(), int(n_q), int(hd),
@@ -883,6 +912,63 @@ def dv2_gemv_attn(packed: torch.Tensor, scale: torch.Tensor, state: torch.Tensor
                                                  _opt_sumsq(sumsq_out, "sumsq_out"))
         _check_rc("chr_dv2_gemv_attn_sumsq", rc)
     return out
+
+
+def dv2_step_args(x, q, k, v, down_in, state, sumsq, valid_len, position, cos, sin, n_q: int, n_kv: int, hd: int,
+                  max_seq: int, attn_scale: float, eps: float) -> _Step:
+    """What the layers of one decode step share (``dv2_step_layer``), checked once a step.  Holds
+    addresses: good for the step it was made for."""
+    kv = n_kv * hd
+    for t, name, numel in ((x, "x", 1), (q, "q", n_q * hd), (k, "k", kv), (v, "v", kv), (down_in, "down_in", 1)):
+        if not (t.is_cuda and t.dtype == torch.bfloat16 and t.is_contiguous() and t.numel() >= numel):
+            raise RuntimeError(f"{name} must be contiguous CUDA bf16 of at least {numel} elements")
+    for t in (cos, sin, position):
+        _need(t.is_cuda and t.is_contiguous(), "cos, sin and position must be contiguous CUDA")
+    _need(valid_len.is_cuda and valid_len.dtype == torch.int32 and valid_len.numel() == 1,
+          "valid_len must be a CUDA int32 scalar")
+    _need(state.is_cuda and state.dtype == torch.float32 and state.is_contiguous()
+          and state.numel() >= n_q * ATTN_PARTS * (hd + 4), "attention state buffer too small")
+    return _Step(x.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), down_in.data_ptr(), state.data_ptr(),
+                 _opt_sumsq(sumsq, "sumsq"), valid_len.data_ptr(), position.data_ptr(), cos.data_ptr(), sin.data_ptr(),
+                 n_q, n_kv, hd, ATTN_PARTS, ATTN_PART_WAVES, max_seq, attn_scale, eps)
+
+
+def dv2_step_layer(step: _Step, hidden: int, mats, biases, norm1, norm2, down_elems: int, k_cache, v_cache) -> None:
+    """The five launches of one layer of the folded step in one call.  ``mats``: ``(q, k, v, o, gate,
+    up, down)`` with ``packed``, ``scale``, ``M``, ``K``, ``K_pad`` (``k`` and ``v`` None: ``q`` is the
+    fused matrix); ``hidden`` and ``down_elems``: elements of the step's ``x`` and ``down_in``."""
+    devs, keep = [], []
+    for m in mats:
+        if m is None:
+            devs.append(_Dev())
+            continue
+        packed, scale = m.packed, m.scale
+        _check_packed(packed, scale, m.M, m.K, m.K_pad)
+        if not (packed.is_contiguous() and scale.is_contiguous()):
+            packed, scale = packed.contiguous(), scale.contiguous()
+            keep.append((packed, scale))
+        devs.append(_Dev(m.M, m.K, m.K_pad, packed.data_ptr(), scale.data_ptr()))
+    q, k, v, o, gate, up, down = devs
+    n_q, n_kv, hd = step.n_q, step.n_kv, step.hd
+    fused = mats[1] is None
+    _need(q.K == gate.K == up.K == o.M == down.M == hidden and o.K == n_q * hd and gate.M == up.M == down.K
+          and down_elems >= down.K and (q.M == (n_q + 2 * n_kv) * hd if fused else
+                                        q.M == n_q * hd and k.M == v.M == n_kv * hd and k.K == v.K == hidden),
+          "the layer's matrices do not fit the step's buffers")
+    _need(not fused or (step.k - step.q == 2 * n_q * hd and step.v - step.k == 2 * n_kv * hd),
+          "a fused matrix writes q, k and v side by side")
+    ptrs = []
+    for t, numel, name in ((biases[0], q.M, "bias"), (biases[1], k.M, "bias"), (biases[2], v.M, "bias"),
+                           (norm1, hidden, "rms_w"), (norm2, hidden, "rms_w")):
+        held, ptr = _opt_bf16(t, numel, name, exact=not (fused and name == "bias"))
+        keep.append(held)
+        ptrs.append(ptr)
+    _need(ptrs[3] is not None and ptrs[4] is not None, "both norms are needed")
+    _need(k_cache.is_contiguous() and v_cache.is_contiguous() and k_cache.shape == v_cache.shape
+          and tuple(k_cache.shape) == (step.max_seq, n_kv, hd), "caches must be contiguous [max_seq,n_kv,hd]")
+    layer = _Layer(q, k, v, o, gate, up, down, *ptrs, k_cache.data_ptr(), v_cache.data_ptr(), 1 if fused else 3)
+    _check_rc("chr_dv2_step_layer", _load_ext().chr_dv2_step_layer(ctypes.byref(layer), ctypes.byref(step), _stream()))
+    del keep
 
 
 def _bf16_cuda(t: torch.Tensor, what: str) -> None:

@@ -399,6 +399,28 @@ int64_t chr_dv2_gemm_swiglu_ws(const chr_nf4_dev_t *gate, const chr_nf4_dev_t *u
 int chr_dv2_gemm_swiglu(const chr_nf4_dev_t *gate, const chr_nf4_dev_t *up, const void *x,
                         void *y, int32_t N, float *ws, int64_t ws_floats, void *stream);
 
+/* One layer of the folded decode step, its five launches issued by one call: chr_dv2_gemv_qkv_sumsq
+ * (chr_dv2_gemv_sumsq where qkv_rows == 1: q then describes the fused matrix, bias its bias),
+ * chr_dv2_attn_parts, chr_dv2_gemv_attn_sumsq onto x, chr_dv2_gemv_swiglu_sumsq,
+ * chr_dv2_gemv_sumsq onto x.  Returns the first launch's code that is not 0, later launches are not
+ * issued then.  A step in an interpreter spends more host time on the five calls than the device on
+ * a small model's layer.  No reference counterpart. */
+typedef struct {
+  chr_nf4_dev_t q, k, v, o, gate, up, down;
+  const void *q_bias, *k_bias, *v_bias;
+  const void *norm1, *norm2; /* bf16 [K] of q and of gate */
+  void *k_cache, *v_cache;   /* [max_seq, n_kv, hd] */
+  int32_t qkv_rows;          /* 3: q, k and v; 1: fused, rows [Q | K | V] */
+} chr_dv2_layer_t;
+typedef struct {
+  void *x, *q, *k, *v, *down_in;  /* bf16: the residual stream, this token's q, k, v, silu(g) * u */
+  float *state, *sumsq;           /* attention states; the parts handed from writer to reader of x */
+  const void *valid_len, *position, *cos, *sin;
+  int32_t n_q, n_kv, hd, n_parts, n_waves, max_seq;
+  float attn_scale, eps;
+} chr_dv2_step_t;
+int chr_dv2_step_layer(const chr_dv2_layer_t *layer, const chr_dv2_step_t *step, void *stream);
+
 /* chr_dv2_argmax_commit as two launches for a large vocabulary: 128 workgroups leave the best
  * (value, index) of a slice each in ws, a small launch picks among them and commits; same
  * tie and NaN rules.  ws: chr_dv2_argmax_ws_bytes() bytes of device memory, 8-byte aligned;
