@@ -49,7 +49,7 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
 }
 
 // Bound: the matrix cores and the LDS reads beside them where the launch fills the chip (gate and up
-// of 27648 x 5120 at 1792 tokens 1.49 ms, 0.68 PFLOP/s), the table, first loads and the meeting of
+// of 27648 x 5120 at 1792 tokens 1.42 ms, 0.72 PFLOP/s), the table, first loads and the meeting of
 // the sums where a split is a few chunks (5120 x 5120 at 1792 in 3 splits 270 us, 0.35).  The window
 // launches it stands for took 57 ms for a 14B prompt of 512 tokens and 484 for a 32B one of 1791;
 // with it 32 and 308.
@@ -201,23 +201,29 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
         const Raw16 f = {pair_at<0>(w, lane4), pair_at<1>(w, lane4), pair_at<2>(w, lane4), pair_at<3>(w, lane4)};
         wf[j] = __builtin_bit_cast(Bf16x8, f);
       }
+      // the chains of the two token blocks take turns, ahead of the other wavefront's lookups (1792
+      // tokens through gate and up of 13824 / 27648 x 5120: 786 / 1476 us one after the other at even
+      // priority, 758 / 1418 so)
+      F32x16 d[2];
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        d[0][v] = 0.f;
+        d[1][v] = 0.f;
+      }
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        d[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[0][j], wf[j], d[0], 0, 0, 0);
+        d[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[1][j], wf[j], d[1], 0, 0, 0);
+      }
+      __builtin_amdgcn_s_setprio(0);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
-        F32x16 d;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
-          d[v] = 0.f;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          d = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[t][j], wf[j], d, 0, 0, 0);
-        }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          acc[b][t][v] = fmaf(s, d[v], acc[b][t][v]);
+          acc[b][t][v] = fmaf(s, d[t][v], acc[b][t][v]);
         }
       }
-      asm volatile("" ::: "memory");  // keeps a later block's codes and lookups out of this one's registers
     }
     store_s(buf ^ 1);
     lds_loads_done();
