@@ -8,10 +8,9 @@
 // 102 / 42, 11008x2048 at 333 296 / 47, 5120x13824 at 1024 873 / 166 (872 TFLOP/s; the library's
 // dense bf16 8192^3 product reaches 1150 on this card).
 //
-// Arithmetic: bf16(level) times the bf16 activation in the matrix cores, every 64-wide group's sum
-// times its scale in fp32 (the numerics of the tile that finishes its rows itself in nf4_gemm.hip:
-// 1.4e-3 of weight rounding against 1.7e-3 for bf16(level * scale)), splits added in fp32 in a
-// fixed order, one bf16 rounding.
+// Arithmetic: bf16(kWideUnit * level) times the bf16 activation in the matrix cores, every 64-wide
+// group's sum times its scale / kWideUnit in fp32, splits added in fp32 in a fixed order, one bf16
+// rounding.
 
 #include "nf4_common.h"
 
@@ -23,6 +22,22 @@ namespace {
 typedef __attribute__((ext_vector_type(8))) __bf16 Bf16x8;
 typedef __attribute__((ext_vector_type(4))) float F32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t Raw16;
+
+// The levels as the matrix cores take them.  A level rounded to bf16 is off by the same amount in
+// every weight that has it, so what the sixteen errors leave on average grows with the sum of x: with
+// bf16(level) a product of activations that do not average to zero (behind a relu or a gate) was off
+// by 2e-2 of its norm at K = 5120, 4e-2 at 27648.  The unit and three other roundings were chosen for
+// errors that are small (1.13e-3 of the weights' norm; bf16(level) 1.38e-3, bf16(level * scale)
+// 1.66e-3) and cancel: levels 1, 6 and 10 are rounded to the nearest in lanes of even 16-lane rows
+// and to the neighbour on the other side in odd ones, which take the other half of every group's K.
+// The average left is below 3e-6 of the weights' norm, whether they are normal, Laplace, uniform,
+// triangular or Student-t (bf16(level) 4e-4).  Products of K = 1024 .. 27648 against 64 bits, x of zero
+// mean, of mean 1 and sigma 0.3, and behind a relu or silu: 1.8e-3 .. 2.1e-3 of the norm, the rounding
+// of the result (1.7e-3) included.
+constexpr float kWideUnit = 1.24227f;
+constexpr uint32_t kWideLevel[2][16] = {
+    {0xBF9F, 0xBF5D, 0xBF27, 0xBEFB, 0xBEB5, 0xBE6B, 0xBDE8, 0x0000, 0x3DCA, 0x3E4D, 0x3E9D, 0x3ED7, 0x3F0C, 0x3F33, 0x3F66, 0x3F9F},
+    {0xBF9F, 0xBF5E, 0xBF27, 0xBEFB, 0xBEB5, 0xBE6B, 0xBDE7, 0x0000, 0x3DCA, 0x3E4D, 0x3E9C, 0x3ED7, 0x3F0C, 0x3F33, 0x3F66, 0x3F9F}};
 
 struct WideArgs {
   const uint8_t *packed;
@@ -146,8 +161,8 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
   // a wavefront's scales of two groups, by row: lane i reads the four of its rows 4i .. 4i + 3
   const uint32_t sc_at = static_cast<uint32_t>(kPairTableBytes + 2 * kStageBytes + wave * 512);
   auto store_s = [&]() {
-    *reinterpret_cast<__attribute__((address_space(3))) float *>(sc_at + lane * 4) = f16_to_f32(static_cast<uint16_t>(ns01));
-    *reinterpret_cast<__attribute__((address_space(3))) float *>(sc_at + 256 + lane * 4) = f16_to_f32(static_cast<uint16_t>(ns01 >> 16));
+    *reinterpret_cast<__attribute__((address_space(3))) float *>(sc_at + lane * 4) = f16_to_f32(static_cast<uint16_t>(ns01)) * (1.f / kWideUnit);
+    *reinterpret_cast<__attribute__((address_space(3))) float *>(sc_at + 256 + lane * 4) = f16_to_f32(static_cast<uint16_t>(ns01 >> 16)) * (1.f / kWideUnit);
   };
   auto read_s = [&](int half) {
     return __builtin_bit_cast(F32x4, lds0_u128(sc_at + half * 256 + li * 16));
@@ -156,8 +171,9 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
   load_x(g_lo, 0);
   load_w(g_lo, cw);
   for (int b = wave; b < 256; b += NW) {
-    const uint32_t lo = kLutBits[b & 15], hi = kLutBits[b >> 4];
-    smem[b * 64 + lane] = bf16_bits_rne(lo) | (bf16_bits_rne(hi) << 16);
+    const uint32_t even = kWideLevel[0][b & 15] | (kWideLevel[0][b >> 4] << 16);
+    const uint32_t odd = kWideLevel[1][b & 15] | (kWideLevel[1][b >> 4] << 16);
+    smem[b * 64 + lane] = (lane & 16) == 0 ? even : odd;
   }
   store_s();
   lds_loads_done();

@@ -440,8 +440,8 @@ int chr_dv2_argmax_commit_ws(const void *logits, int32_t n, void *next_token, vo
  *   - x 16-byte and y 8-byte aligned (-5); x_stride % 8 == 0 and x_stride >= K_pad (-3): where K is
  *     not a multiple of 64 the caller's rows are K_pad long, with zeros behind K
  *   - ws: chr_nf4_wide_ws floats (0: none; -1: bad arguments), 16-byte aligned (-5; too few: -7)
- *   - weights enter as bf16(level) and every 64-wide group's sum takes its scale in fp32, as in the
- *     tile of chr_nf4_gemm that finishes its rows itself */
+ *   - weights enter the matrix cores as bf16 levels chosen so that their roundings cancel, every
+ *     64-wide group's sum takes its scale in fp32 */
 int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y,
                  float *ws, int64_t ws_floats, const void *bias, void *stream);
 int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N);

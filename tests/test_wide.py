@@ -82,6 +82,23 @@ def test_product(n, m, k, bias):
         assert torch.equal(nf4.nf4_wide(*mat[:2], wide[:, off:off + k], m, k, k_pad(k), bias=b), got)
 
 
+# activations whose sum does not vanish meet the average of the levels' roundings: it must not grow with K.
+# Bound: the rounding of the result (2^-9 of it at most: 1.7e-3 of the norm) and of the levels (1.15e-3) make 2.1e-3
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k", [(512, 5120), (256, 27648)])
+@pytest.mark.parametrize("weights", ["normal", "uniform"])
+@pytest.mark.parametrize("acts", ["mean one", "relu", "zero mean"])
+def test_roundings_of_the_levels_cancel(m, k, weights, acts):
+    g = torch.Generator(device="cuda").manual_seed(m + len(weights))
+    w = torch.randn(m, k, generator=g, device="cuda") if weights == "normal" else torch.rand(m, k, generator=g, device="cuda") * 2 - 1
+    packed, scale = nf4.nf4_quantize(w * 0.02)
+    x = torch.randn(40, k, generator=g, device="cuda")
+    x = {"mean one": 1 + 0.3 * x, "relu": x.relu(), "zero mean": x}[acts].to(BF16)
+    want = x.double() @ nf4.nf4_dequant(packed, scale, m, k, k).double().t()
+    got = nf4.nf4_wide(packed, scale, x, m, k, k).double()
+    assert float((got - want).norm()) <= 2.4e-3 * float(want.norm())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [2, 16, 17, 32, 33, 64, 65, 257])
 @pytest.mark.parametrize("dtype", [BF16, torch.float32])
