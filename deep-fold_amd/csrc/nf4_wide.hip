@@ -47,7 +47,7 @@ struct WideArgs {
   float *part;  // fp32 partials [splits][N][M], or null
   const uint16_t *bias;
   int64_t x_stride;
-  int N, M;
+  int N, M, K;
   int groups, split_groups;
   int tiles_m, tiles_n;
 };
@@ -69,7 +69,13 @@ struct WideArgs {
 //
 // x goes from global memory straight to LDS one stage of two groups ahead, 128-byte rows whose 16-byte
 // pieces are XORed with the row's low bits: the 16-lane reads of a fragment touch all banks once.
-template <int WM, int WN, int TT>
+//
+// WHOLE: the rows of x are whole 16-byte pieces of whole groups.  Otherwise (a ragged K, rows at any
+// 2-byte boundary) the pieces pass through registers, what lies behind K as zeros: a padded copy is two
+// launches (at 8 tokens 320x500 17.1 us, 12.7 so; 16384x6100 34.8, 29.3), but the 512 x 128 tile spills
+// five registers and runs a tenth longer, so large calls bring one (16384x6100 at 1024 tokens 215 us,
+// 235 so).
+template <int WM, int WN, int TT, bool WHOLE>
 __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
   constexpr int NW = WM * WN;
   constexpr int BN = WN * TT * 16;
@@ -125,14 +131,38 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
     xp[p] = a.x + static_cast<int64_t>(min(tok0 + row, a.N - 1)) * a.x_stride + sub * kGroup + piece * 8;
   }
 
+  uint4 xr[WHOLE ? 1 : kPass];
   auto load_x = [&](int g, int buf) {
 #pragma unroll
     for (int p = 0; p < kPass; ++p) {
       // the second half of a last, odd stage is not multiplied: it reads its first half again
       const int sub = (wave + p * NW) / (BN / 8);
       const int off = (sub == 1 && g + 1 >= g_hi) ? (g - 1) * kGroup : g * kGroup;
-      const uint32_t at = static_cast<uint32_t>(kPairTableBytes + buf * kStageBytes + (wave + p * NW) * 1024);
-      load_to_lds16(xp[p] + off, at);
+      if constexpr (WHOLE) {
+        const uint32_t at = static_cast<uint32_t>(kPairTableBytes + buf * kStageBytes + (wave + p * NW) * 1024);
+        load_to_lds16(xp[p] + off, at);
+      } else if ((g + 2) * kGroup <= a.K) {
+        __builtin_memcpy(&xr[p], xp[p] + off, 16);
+      } else {
+        const int left = a.K - off - sub * kGroup - ((lane & 7) ^ (lane >> 3)) * 8;
+        uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          if (e < left) {
+            w[e >> 1] |= static_cast<uint32_t>(xp[p][off + e]) << (16 * (e & 1));
+          }
+        }
+        xr[p] = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+    }
+  };
+  auto store_x = [&](int buf) {
+    if constexpr (!WHOLE) {
+#pragma unroll
+      for (int p = 0; p < kPass; ++p) {
+        const uint32_t at = static_cast<uint32_t>(kPairTableBytes + buf * kStageBytes + (wave + p * NW) * 1024 + lane * 16);
+        *reinterpret_cast<__attribute__((address_space(3))) Raw16 *>(at) = __builtin_bit_cast(Raw16, xr[p]);
+      }
     }
   };
   auto from_loader = [&](uint32_t v) {
@@ -175,6 +205,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
     smem[b * 64 + lane] = (lane & 16) == 0 ? even : odd;
   }
   store_s();
+  store_x(0);
   lds_loads_done();
   __syncthreads();
 
@@ -251,6 +282,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
     }
     if (more) {
       store_s();
+      store_x(buf ^ 1);
     }
     lds_loads_done();
     __syncthreads();
@@ -384,11 +416,11 @@ __global__ __launch_bounds__(256) void wide_reduce(const float *__restrict__ par
   store_bf16<W>(y + at, o);
 }
 
-template <int WM, int WN, int TT>
+template <int WM, int WN, int TT, bool WHOLE>
 int wide_launch(WideArgs &a, int splits, hipStream_t st) {
   constexpr int BN = WN * TT * 16;
   constexpr int kLds = kPairTableBytes + 4 * BN * 128 + WM * WN * 512;
-  if (hipFuncSetAttribute(reinterpret_cast<const void *>(&wide_gemm<WM, WN, TT>),
+  if (hipFuncSetAttribute(reinterpret_cast<const void *>(&wide_gemm<WM, WN, TT, WHOLE>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, kLds) != hipSuccess) {
     (void)hipGetLastError();
     return -6;
@@ -400,7 +432,7 @@ int wide_launch(WideArgs &a, int splits, hipStream_t st) {
   if (grid > INT32_MAX) {
     return -3;
   }
-  wide_gemm<WM, WN, TT><<<dim3(static_cast<unsigned>(grid)), dim3(WM * WN * kWave), kLds, st>>>(a);
+  wide_gemm<WM, WN, TT, WHOLE><<<dim3(static_cast<unsigned>(grid)), dim3(WM * WN * kWave), kLds, st>>>(a);
   return launch_rc();
 }
 
@@ -451,13 +483,14 @@ WidePlan wide_plan(int M, int N, int groups) {
   return best;
 }
 
+template <bool WHOLE>
 int wide_dispatch(int tile, WideArgs &a, int splits, hipStream_t st) {
   switch (tile) {
-    case 0: return wide_launch<8, 1, 8>(a, splits, st);
-    case 1: return wide_launch<4, 2, 4>(a, splits, st);
-    case 2: return wide_launch<4, 1, 4>(a, splits, st);
-    case 3: return wide_launch<4, 1, 2>(a, splits, st);
-    default: return wide_launch<4, 1, 1>(a, splits, st);
+    case 0: return wide_launch<8, 1, 8, WHOLE>(a, splits, st);
+    case 1: return wide_launch<4, 2, 4, WHOLE>(a, splits, st);
+    case 2: return wide_launch<4, 1, 4, WHOLE>(a, splits, st);
+    case 3: return wide_launch<4, 1, 2, WHOLE>(a, splits, st);
+    default: return wide_launch<4, 1, 1, WHOLE>(a, splits, st);
   }
 }
 
@@ -482,6 +515,7 @@ int wide_args(const chr_nf4_dev_t *w, int32_t N, WideArgs &a) {
   a.packed = w->packed;
   a.scale = w->scale;
   a.M = w->M;
+  a.K = w->K;
   a.N = N;
   a.groups = w->K_pad / kGroup;
   return 0;
@@ -491,21 +525,10 @@ int64_t wide_ws(const WideArgs &a, const WidePlan &p) {
   return p.splits == 1 ? 0 : static_cast<int64_t>(p.splits) * a.N * a.M;
 }
 
-}  // namespace
-}  // namespace chr
-
-using namespace chr;
-
-extern "C" int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N) {
-  WideArgs a{};
-  if (wide_args(w, N, a) != 0) {
-    return -1;
-  }
-  return wide_ws(a, wide_plan(a.M, N, a.groups));
-}
-
-extern "C" int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y, float *ws,
-                            int64_t ws_floats, const void *bias, void *stream) {
+// rows: x at any 2-byte boundary, its rows x_stride >= K apart.  Otherwise whole 16-byte pieces of
+// whole groups, a ragged K padded by the caller.
+int wide_entry(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y, float *ws, int64_t ws_floats,
+               const void *bias, void *stream, bool rows) {
   if (x == nullptr || y == nullptr) {
     return -1;
   }
@@ -513,13 +536,12 @@ extern "C" int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_str
   if (const int rc = wide_args(w, N, a)) {
     return rc;
   }
-  // whole 16-byte pieces of whole groups: a ragged K is the caller's to pad
-  if (x_stride < w->K_pad || (x_stride & 7) != 0) {
+  if (rows ? x_stride < w->K : (x_stride < w->K_pad || (x_stride & 7) != 0)) {
     return -3;
   }
   const WidePlan p = wide_plan(a.M, N, a.groups);
   const int64_t need = wide_ws(a, p);
-  if (!aligned16(x) || (reinterpret_cast<uintptr_t>(y) & 7u) != 0 || (need > 0 && !aligned16(ws))) {
+  if (!(rows ? aligned2(x) : aligned16(x)) || (reinterpret_cast<uintptr_t>(y) & 7u) != 0 || (need > 0 && !aligned16(ws))) {
     return -5;
   }
   if (need > 0 && (ws == nullptr || ws_floats < need)) {
@@ -538,7 +560,8 @@ extern "C" int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_str
   a.part = need > 0 ? ws : nullptr;
   a.split_groups = p.split_groups;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int rc = wide_dispatch(p.tile, a, p.splits, st);
+  const bool whole = !rows || (w->K == w->K_pad && (x_stride & 7) == 0 && aligned16(x));
+  const int rc = whole ? wide_dispatch<true>(p.tile, a, p.splits, st) : wide_dispatch<false>(p.tile, a, p.splits, st);
   if (rc != 0 || a.part == nullptr) {
     return rc;
   }
@@ -549,4 +572,27 @@ extern "C" int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_str
     wide_reduce<1><<<grid, block, 0, st>>>(a.part, p.splits, count, a.M, a.bias, a.y);
   }
   return launch_rc();
+}
+
+}  // namespace
+}  // namespace chr
+
+using namespace chr;
+
+extern "C" int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N) {
+  WideArgs a{};
+  if (wide_args(w, N, a) != 0) {
+    return -1;
+  }
+  return wide_ws(a, wide_plan(a.M, N, a.groups));
+}
+
+extern "C" int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y, float *ws,
+                            int64_t ws_floats, const void *bias, void *stream) {
+  return wide_entry(w, x, x_stride, N, y, ws, ws_floats, bias, stream, false);
+}
+
+extern "C" int chr_nf4_wide_rows(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y, float *ws,
+                                 int64_t ws_floats, const void *bias, void *stream) {
+  return wide_entry(w, x, x_stride, N, y, ws, ws_floats, bias, stream, true);
 }

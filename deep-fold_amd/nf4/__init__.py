@@ -185,6 +185,7 @@ EXPORTS = (
     ("chr_dv2_argmax_ws_bytes", ctypes.c_int64, []),
     ("chr_dv2_argmax_commit_ws", ctypes.c_int, [_P, _I, _P, _P, _P, _P, _P, _I, _P, ctypes.c_int64, _P]),
     ("chr_nf4_wide", ctypes.c_int, [_DP, _P, ctypes.c_int64, _I, _P, _P, ctypes.c_int64, _P, _P]),
+    ("chr_nf4_wide_rows", ctypes.c_int, [_DP, _P, ctypes.c_int64, _I, _P, _P, ctypes.c_int64, _P, _P]),
     ("chr_nf4_wide_ws", ctypes.c_int64, [_DP, _I]),
     ("chr_dv2_prompt_ws", ctypes.c_int64, [_DP, _I, _I, _I]),
     ("chr_dv2_prompt_gemm", ctypes.c_int, [_DP, _I, _I, _P, _I, _P, _P, ctypes.c_int64, _P, _P]),
@@ -1144,22 +1145,29 @@ def dv2_gemm_swiglu(gate, up, x: torch.Tensor) -> torch.Tensor:
     return y
 
 
+#: Products of this many weights x tokens take a ragged K from a padded copy: the copy (two launches,
+#: 3 to 8 us) costs less there than passing x through registers in the product (a tenth of it).  In
+#: the product / from a copy, us: 1000x1111 at 33 tokens 11.9 / 15.8, 8192x8200 at 33 32.5 / 36.4 and at
+#: 512 108.8 / 109.4, 27648x5000 at 33 63.5 / 60.8 and at 1024 387 / 349, 2048x11000 at 1024 78.9 / 87.6.
+PAD_MACS = 1 << 34
+
+
 def nf4_wide(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int, K: int,  # noqa: N803
              K_pad: int, *, bias: torch.Tensor | None = None) -> torch.Tensor:  # noqa: N803
     """``x [N, K]`` bf16, any N, times the transpose of the packed matrix: ``[N, M]`` (+ ``bias``,
-    one bf16 element a feature).  A ragged K is padded with zeros into a copy, rows that are not
-    contiguous in whole 16-byte pieces are copied."""
+    one bf16 element a feature).  Rows may lie any distance apart; rows whose elements are not
+    contiguous are copied."""
     M, K, K_pad = int(M), int(K), int(K_pad)
     _need(packed.is_cuda and scale.is_cuda and x.is_cuda, "packed, scale, and x must be CUDA tensors")
     _need(x.dtype == torch.bfloat16 and x.dim() == 2 and int(x.size(1)) == K and int(x.size(0)) >= 1,
           f"x must be bfloat16 [N, {K}]")
     _check_packed(packed, scale, M, K, K_pad)
     packed, scale = packed.contiguous(), scale.contiguous()
-    if K != K_pad:
-        x = torch.nn.functional.pad(x, (0, K_pad - K))
-    elif x.stride(1) != 1 or x.stride(0) % 8 != 0 or x.stride(0) < K or x.data_ptr() % 16 != 0:
-        x = x.clone(memory_format=torch.contiguous_format)
     n = int(x.size(0))
+    if K != K_pad and M * K * n >= PAD_MACS:
+        x, K = torch.nn.functional.pad(x, (0, K_pad - K)), K_pad
+    elif (x.stride(1) != 1 and K > 1) or x.stride(0) < K:
+        x = x.clone(memory_format=torch.contiguous_format)
     _need(bias is None or (bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
                            and bias.numel() == M), f"bias must be contiguous CUDA bf16 of {M} elements")
     lib = _load_ext()
@@ -1167,10 +1175,10 @@ def nf4_wide(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int,
     floats = int(lib.chr_nf4_wide_ws(ctypes.byref(w), n))
     ws = torch.empty(floats, dtype=torch.float32, device=x.device) if floats > 0 else None
     y = torch.empty((n, M), dtype=torch.bfloat16, device=x.device)
-    rc = lib.chr_nf4_wide(ctypes.byref(w), x.data_ptr(), int(x.stride(0)), n, y.data_ptr(),
-                          None if ws is None else ws.data_ptr(), floats, None if bias is None else bias.data_ptr(),
-                          _stream())
-    _check_rc("chr_nf4_wide", rc)
+    rc = lib.chr_nf4_wide_rows(ctypes.byref(w), x.data_ptr(), int(x.stride(0)), n, y.data_ptr(),
+                               None if ws is None else ws.data_ptr(), floats, None if bias is None else bias.data_ptr(),
+                               _stream())
+    _check_rc("chr_nf4_wide_rows", rc)
     return y
 
 

@@ -37,6 +37,29 @@ def test_arguments_are_refused_before_any_launch():
     assert lib.chr_nf4_wide(ctypes.byref(w), p, 13824, 128, p, p + 4, need, None, None) == -5
     assert lib.chr_nf4_wide_ws(ctypes.byref(w), 0) == -1
 
+    def rows_rc(k=250, kp=256, x=p, stride=250, y=p):
+        w = nf4._Dev(128, k, kp, 0x1000, 0x2000)
+        return lib.chr_nf4_wide_rows(ctypes.byref(w), x, stride, 65, y, None, 0, None, None)
+
+    assert rows_rc(x=None) == -1 and rows_rc(stride=249) == -3 and rows_rc(kp=320) == -4
+    assert rows_rc(x=p + 1) == -5 and rows_rc(y=p + 2) == -5
+
+
+# the padded copy of a ragged K and the rows as they are: one result, and what lies behind a row is not multiplied
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,k", [(2, 300, 1), (5, 64, 63), (33, 256, 65), (70, 1030, 200), (130, 512, 1111), (520, 5000, 1090)])
+def test_rows_of_a_ragged_k(n, m, k):
+    mat, w = matrix(m, k, seed=k)
+    kp = k_pad(k)
+    clean = rand(n, k, seed=n)
+    want = nf4.nf4_wide(*mat[:2], torch.nn.functional.pad(clean, (0, kp - k)), m, kp, kp)
+    close(want, clean.double() @ w.t())
+    for before, behind in ((0, 1), (3, 6), (8, 8)):
+        room = torch.full((n, before + k + behind), float("nan"), dtype=BF16, device="cuda")
+        x = room[:, before:before + k]
+        x.copy_(clean)
+        assert torch.equal(nf4.nf4_wide(*mat[:2], x, m, k, kp), want)
+
 
 def matrix(m, k, seed, sigma=0.05):
     w = np.random.default_rng(seed).standard_normal((m, k)).astype(np.float32) * sigma
