@@ -3,10 +3,12 @@
 // columns (nf4_gemm.hip) read and decode the whole matrix once per window; here a workgroup keeps
 // 256 or 512 weight rows against up to 128 tokens, so a matrix is decoded once per 128 tokens.
 // Bound: up to about 64 tokens the bytes of the weights and a workgroup's fixed start, above the
-// matrix cores and the LDS reads beside them.  Whole calls through the linear seat, windows of 32
-// before and this after (us): 5120x5120 at 17 tokens 27 / 18, 13824x5120 at 64 50 / 36, at 100
-// 102 / 42, 11008x2048 at 333 296 / 47, 5120x13824 at 1024 873 / 166 (872 TFLOP/s; the library's
-// dense bf16 8192^3 product reaches 1150 on this card).
+// matrix cores and the LDS reads beside them.  Whole calls through the linear seat from a graph, windows
+// of 32 before and this after (us): 512x512 at 8 tokens 11.2 / 8.0, 5120x5120 at 17 27.4 / 14.9 and at
+// 32 19.2 / 16.7, 13824x5120 at 64 47 / 33, 11008x2048 at 333 189 / 43, 5120x13824 at 1024 797 / 167 (870
+// TFLOP/s; the library's dense bf16 8192^3 product reaches 1150 on this card).  A window of whole vectors
+// is still the faster through some matrices of 10^8 codes and more: 16384x6144 at 8 / 32 tokens 24.7 / 27.7
+// and 25.9 / 29.5, 27648x5184 at 8 37.5 and 42.4, a ragged 16384x6100 at 32 27.7 and 33.6.
 //
 // Arithmetic: bf16(kWideUnit * level) times the bf16 activation in the matrix cores, every 64-wide
 // group's sum times its scale / kWideUnit in fp32, splits added in fp32 in a fixed order, one bf16
@@ -35,9 +37,9 @@ typedef __attribute__((ext_vector_type(4))) uint32_t Raw16;
 // mean, of mean 1 and sigma 0.3, and behind a relu or silu: 1.8e-3 .. 2.1e-3 of the norm, the rounding
 // of the result (1.7e-3) included.
 constexpr float kWideUnit = 1.24227f;
-constexpr uint32_t kWideLevel[2][16] = {
-    {0xBF9F, 0xBF5D, 0xBF27, 0xBEFB, 0xBEB5, 0xBE6B, 0xBDE8, 0x0000, 0x3DCA, 0x3E4D, 0x3E9D, 0x3ED7, 0x3F0C, 0x3F33, 0x3F66, 0x3F9F},
-    {0xBF9F, 0xBF5E, 0xBF27, 0xBEFB, 0xBEB5, 0xBE6B, 0xBDE7, 0x0000, 0x3DCA, 0x3E4D, 0x3E9C, 0x3ED7, 0x3F0C, 0x3F33, 0x3F66, 0x3F9F}};
+constexpr uint32_t kWideLevel[16] = {0xBF9F, 0xBF5D, 0xBF27, 0xBEFB, 0xBEB5, 0xBE6B, 0xBDE8, 0x0000,
+                                     0x3DCA, 0x3E4D, 0x3E9D, 0x3ED7, 0x3F0C, 0x3F33, 0x3F66, 0x3F9F};
+constexpr int kWideOther[16] = {0, 1, 0, 0, 0, 0, -1, 0, 0, 0, -1};  // to the neighbour in odd 16-lane rows
 
 struct WideArgs {
   const uint8_t *packed;
@@ -72,7 +74,7 @@ struct WideArgs {
 //
 // WHOLE: the rows of x are whole 16-byte pieces of whole groups.  Otherwise (a ragged K, rows at any
 // 2-byte boundary) the pieces pass through registers, what lies behind K as zeros: a padded copy is two
-// launches (at 8 tokens 320x500 17.1 us, 12.7 so; 16384x6100 34.8, 29.3), but the 512 x 128 tile spills
+// launches (at 8 tokens 320x500 17.1 us, 12.7 so; 16384x6100 34.8, 29.3, each with a slower table fill), but the 512 x 128 tile spills
 // five registers and runs a tenth longer, so large calls bring one (16384x6100 at 1024 tokens 215 us,
 // 235 so).
 template <int WM, int WN, int TT, bool WHOLE>
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
     }
     // both scales in one load, at whatever 2-byte boundary the row puts them: each of its 64 lanes
     // reads a line of its own, and as two loads an odd group count cost a third more than its even
-    // neighbour (16 tokens, 16384x6208 42.7 us against 30.8 at 6272; 31.8 so)
+    // neighbour (16 tokens, 16384x6208 42.6 us against 30.8 at 6272; 29.8 and 28.4 so)
     if (odd) {
       ns01 = sp[g];
     } else {
@@ -199,10 +201,22 @@ __global__ __launch_bounds__(WM *WN *kWave) void wide_gemm(const WideArgs a) {
 
   load_x(g_lo, 0);
   load_w(g_lo, cw);
-  for (int b = wave; b < 256; b += NW) {
-    const uint32_t even = kWideLevel[0][b & 15] | (kWideLevel[0][b >> 4] << 16);
-    const uint32_t odd = kWideLevel[1][b & 15] | (kWideLevel[1][b >> 4] << 16);
-    smem[b * 64 + lane] = (lane & 16) == 0 ? even : odd;
+  // The table, sixteen bytes of one high code at a time, their low levels literals: an instruction and
+  // half a store a byte.  One byte a turn, its two levels loaded, took 4 us of every workgroup's start (from
+  // a graph 512x512 at 8 tokens 12.0 us, 8.0 so; 5120x5120 at 17 18.1 and 14.9).
+  const uint32_t odd_row = (lane >> 4) & 1;
+  uint32_t hi[16 / NW];
+#pragma unroll
+  for (int i = 0; i < 16 / NW; ++i) {
+    hi[i] = (kWideLevel[wave + i * NW] + static_cast<uint32_t>(kWideOther[wave + i * NW]) * odd_row) << 16;
+  }
+#pragma unroll
+  for (int i = 0; i < 16 / NW; ++i) {
+#pragma unroll
+    for (int l = 0; l < 16; ++l) {
+      smem[(16 * (wave + i * NW) + l) * 64 + lane] =
+          hi[i] | (kWideLevel[l] + static_cast<uint32_t>(kWideOther[l]) * odd_row);
+    }
   }
   store_s();
   store_x(0);
@@ -442,7 +456,10 @@ int wide_launch(WideArgs &a, int splits, hipStream_t st) {
 // splits add 3.5 and the writing and reading of their fp32 partials at 3.4 TB/s together.  Unsplit
 // 8 / 32 / 80 / 216 groups took 11 / 26 / 54 / 132 us on 256 x 16, 17 / 42 / 92 / 230 on 256 x 64 and
 // 18 / 48 / 111 / 285 on 256 x 128; 80 groups 161 on 512 x 128, which does the most a us where it fills
-// the chip.  At 5120 x 5120: 17 tokens 17.7 us on 256 x 32 in 10 splits (23.8 on 256 x 64), 128 tokens
+// the chip.  (All with a table fill that took 4 us longer.  The fixed parts stand as they were: taken off,
+// they send 512x512 at 8 tokens to splits and a second launch, 6.3 us from a graph instead of 8.0 but 19.8
+// instead of 15.8 in a program that calls it launch by launch, and change no larger call by more than 3%.)
+// At 5120 x 5120, then: 17 tokens 17.7 us on 256 x 32 in 10 splits (23.8 on 256 x 64), 128 tokens
 // 32 us on 256 x 64 in 6 (44 on 512 x 128), 512 tokens 57 on 512 x 128 in 6 (100 on 256 x 64).
 struct WideTile {
   int wm, bn;
