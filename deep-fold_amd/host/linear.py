@@ -20,6 +20,7 @@ import math
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 
 from ..chr0.loader import ChrMatrix
 from ..nf4 import LIVE_MAX_N, nf4_gemm, nf4_gemv, nf4_wide
@@ -36,6 +37,14 @@ GROUP_SIZE = 64
 WIDE_MIN_CODES = 1 << 17
 
 
+def _values_alone(t: torch.Tensor) -> bool:
+    """Whether ``t`` is no more than its elements: no gradient, tangent or batch rides on it that an
+    addition by torch would carry on into the answer."""
+    return (type(t) in (torch.Tensor, nn.Parameter) and not t.requires_grad
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t)
+            and (forward_ad._current_level < 0 or forward_ad.unpack_dual(t).tangent is None))
+
+
 def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: int, K: int,  # noqa: N803
                K_pad: int, bias: torch.Tensor | None = None) -> torch.Tensor:  # noqa: N803
     """``y[..., M] = x[..., K] @ dequant(packed, scale).T (+ bias)`` in bf16."""
@@ -49,9 +58,9 @@ def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: in
     if n == 1:
         out = nf4_gemv(packed, scale, rows.reshape(K), M, K, K_pad).reshape(1, M)
     elif M * K >= WIDE_MIN_CODES:
-        # the launch adds a bias it can add as torch would: bf16, one element a feature, no graph
+        # the launch adds a bias it can add as torch would: bf16, one element a feature, values alone
         folds = (bias is not None and bias.dtype == torch.bfloat16 and tuple(bias.shape) == (M,)
-                 and bias.is_contiguous() and bias.device == rows.device and not bias.requires_grad)
+                 and bias.is_contiguous() and bias.device == rows.device and _values_alone(bias))
         out = nf4_wide(packed, scale, rows, M, K, K_pad, bias=bias if folds else None)
         if folds:
             bias = None

@@ -127,3 +127,31 @@ def test_forward_matches_linear_on_the_decoded_matrix(lead, bias):
     assert torch.equal(y, y2)
     ref = F.linear(x.float(), w, None if b is None else b.float())
     assert float((y.float() - ref).abs().max()) <= 1e-2 * float(ref.abs().max()) + 1e-3
+
+
+def test_what_rides_on_a_bias_reaches_the_answer(monkeypatch):
+    """A gradient, a tangent or a batch of biases is added by torch, not by the launch."""
+    from deepfold_amd.host import linear as mod
+
+    def product(packed, scale, x, m, k, k_pad, *, bias=None):
+        y = torch.zeros(x.shape[0], m, dtype=torch.bfloat16)
+        return y if bias is None else y + bias.detach()
+
+    monkeypatch.setattr(mod, "nf4_wide", product)
+    m, k = 512, 512
+    p, s = blobs(m, k)
+    x, b, t = torch.zeros(4, k), torch.randn(m).bfloat16(), torch.randn(m).bfloat16()
+
+    def f(bias):
+        return nf4_linear(x, p, s, m, k, k, bias)
+
+    assert torch.equal(f(b), b.expand(4, m))
+    y, dy = torch.func.jvp(f, (b,), (t,))
+    assert torch.equal(y, b.expand(4, m)) and torch.equal(dy, t.expand(4, m))
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(b, t)
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(f(dual)).tangent, t.expand(4, m))
+    assert torch.equal(torch.func.vmap(f)(torch.stack([b, t])), torch.stack([b.expand(4, m), t.expand(4, m)]))
+    g = b.clone().requires_grad_()
+    f(g).float().sum().backward()
+    assert torch.equal(g.grad, torch.full_like(b, 4.0))
