@@ -8,7 +8,7 @@ nothing registers one, ``weight`` is a read-only 0-element stand-in, so neither
 Layout glue lives here: callers hand ``[..., K]`` activations, the kernels take ``[K, N]``
 (token index fastest) and answer ``[M, N]``.  One token is a view (no copy) and goes to the
 GEMV; more tokens go to the token-major product, which takes and leaves rows as they are, or,
-through a small matrix, to the MFMA GEMM in windows of at most 32, each window's answer
+a few through a small matrix, to the MFMA GEMM in windows of at most 32, each window's answer
 written straight into its rows of the one output buffer.  The bias is added after the
 product's bf16 rounding, as the reference does (``linear.py:62-63,79-80``), so all seats
 round alike.
@@ -30,11 +30,12 @@ from ..ring.host_image import HostImage
 __all__ = ["CompressedLinear", "nf4_linear", "k_pad"]
 
 GROUP_SIZE = 64
-#: Matrices of fewer codes stay in windows of 32 tokens: launches of a few us either way
-#: (512x512 at 32 tokens 12.7 us in a window, 10.0 token-major), and their windows multiply
-#: bf16(level * scale), not the level and the scale apart, which callers of small seats see in
-#: the last bit.
+#: Matrices of fewer codes keep up to WINDOW_TOKENS tokens in windows of 32.  Not for speed: 256x256
+#: takes 10.4 us from a graph at 32 tokens and 39 at 128 that way, 5.7 and 5.8 token-major.  Callers of
+#: small seats hold such answers to the last bit of bf16(level * scale), which the windows multiply and
+#: the token-major product does not.  Above (2000 tokens: 63 windows, 603 us against 6.1) it serves them too.
 WIDE_MIN_CODES = 1 << 17
+WINDOW_TOKENS = 128
 
 
 def _values_alone(t: torch.Tensor) -> bool:
@@ -57,7 +58,7 @@ def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: in
     rows = x.to(torch.bfloat16).reshape(n, K)
     if n == 1:
         out = nf4_gemv(packed, scale, rows.reshape(K), M, K, K_pad).reshape(1, M)
-    elif M * K >= WIDE_MIN_CODES:
+    elif M * K >= WIDE_MIN_CODES or n > WINDOW_TOKENS:
         # the launch adds a bias it can add as torch would: bf16, one element a feature, values alone
         folds = (bias is not None and bias.dtype == torch.bfloat16 and tuple(bias.shape) == (M,)
                  and bias.is_contiguous() and bias.device == rows.device and _values_alone(bias))

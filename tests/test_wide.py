@@ -136,3 +136,15 @@ def test_linear_seat_across_the_window(n, dtype):
     assert y.dtype == dtype                        # a wider bias still widens the answer
     close(y, x.double() @ w.t() + lin.bias.double())
     assert torch.equal(lin(x.t().contiguous().t()), y)   # K not the fastest axis
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [128, 129, 700])
+def test_many_tokens_through_a_small_seat(n):
+    m, k = 96, 200
+    (p, s, _), w = matrix(m, k, seed=4)
+    lin = CompressedLinear(k, m, device="cuda")
+    lin.attach(ChrMatrix("t", m, k, k_pad(k), p, s))
+    x = rand(n, k, seed=2)
+    close(lin(x), x.double() @ w.t())
+    assert torch.equal(lin(x), nf4.nf4_wide(p, s, x, m, k, k_pad(k))) == (n > 128)
