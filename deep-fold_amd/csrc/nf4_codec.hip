@@ -31,6 +31,10 @@ __device__ __forceinline__ void load_lut_lds(float *lut) {
 }
 
 // ---- codec twins -------------------------------------------------------------
+// A grid holds fewer than 2^32 threads: more workgroups of 256 than this go in several launches, which
+// take their blocks from `first` on.
+constexpr int64_t kLaunchBlocks = int64_t{1} << 23;
+
 // out is [M, K] fp32, four weights a thread and kDequantQuads such quads, a workgroup's quads
 // back to back: every store is a 16-byte piece of a wavefront's whole kilobyte, and the loads (two
 // bytes a quad) are all issued before the first store.  Bound by the fp32 it writes, past the caches
@@ -42,11 +46,11 @@ constexpr int kDequantQuads = 4;
 template <typename Index>
 __global__ __launch_bounds__(256) void dequant_f32(const uint8_t *__restrict__ packed,
                                                    const uint16_t *__restrict__ scale,
-                                                   float *__restrict__ out, Index quads, int K4,
-                                                   int K_pad) {
+                                                   float *__restrict__ out, Index first, Index quads,
+                                                   int K4, int K_pad) {
   __shared__ float lut[16];
   load_lut_lds(lut);
-  const Index q0 = static_cast<Index>(blockIdx.x) * (256 * kDequantQuads) + threadIdx.x;
+  const Index q0 = (first + blockIdx.x) * (256 * kDequantQuads) + threadIdx.x;
   uint32_t w[kDequantQuads];
   uint16_t s[kDequantQuads];
 #pragma unroll
@@ -77,11 +81,11 @@ constexpr int64_t kManyWeights = int64_t{1} << 23;
 template <typename Index, int Q>
 __global__ __launch_bounds__(256) void dequant_f32_ragged(const uint8_t *__restrict__ packed,
                                                           const uint16_t *__restrict__ scale,
-                                                          float *__restrict__ out, Index count, int K,
-                                                          int K_pad) {
+                                                          float *__restrict__ out, Index first, Index count,
+                                                          int K, int K_pad) {
   __shared__ float lut[16];
   load_lut_lds(lut);
-  const Index i0 = static_cast<Index>(blockIdx.x) * (256 * Q) + threadIdx.x;
+  const Index i0 = (first + blockIdx.x) * (256 * Q) + threadIdx.x;
   uint8_t w[Q];
   uint16_t s[Q];
   bool odd[Q];
@@ -220,8 +224,8 @@ template <bool VEC>
 __global__ __launch_bounds__(256) void quantize_groups(const float *__restrict__ src,
                                                        uint8_t *__restrict__ packed,
                                                        uint16_t *__restrict__ scale,
-                                                       int32_t *status, int64_t groups, int K,
-                                                       int ng) {
+                                                       int32_t *status, int64_t first, int64_t groups,
+                                                       int K, int ng) {
   __shared__ float cross[kCells];
   __shared__ uint32_t below[kCells];
   if (threadIdx.x < kCells) {
@@ -230,7 +234,7 @@ __global__ __launch_bounds__(256) void quantize_groups(const float *__restrict__
   }
   __syncthreads();
   const int lane = threadIdx.x & 15;
-  const int64_t g0 = static_cast<int64_t>(blockIdx.x) * (16 * kQuantUnroll) + (threadIdx.x >> 4);
+  const int64_t g0 = (first + blockIdx.x) * (16 * kQuantUnroll) + (threadIdx.x >> 4);
   F32x4 v[kQuantUnroll];
 #pragma unroll
   for (int n = 0; n < kQuantUnroll; ++n) {
@@ -327,15 +331,14 @@ extern "C" int chr_nf4_dequant(const chr_nf4_dev_t *w, float *out, void *stream)
   const int64_t items = whole ? count / 4 : count;
   const int per = 256 * (whole || count < kManyWeights ? kDequantQuads : 8);
   const int64_t blocks = (items + per - 1) / per;
-  if (blocks > INT32_MAX) {
-    return -3;
-  }
-  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
   hipStream_t st = static_cast<hipStream_t>(stream);
   // 32-bit indexes (and divisions) unless the last workgroup's would pass 2^32
   const bool narrow = items < (int64_t{1} << 32) - per;
   auto run = [&](auto kernel, auto n, int row) {
-    kernel<<<grid, block, 0, st>>>(w->packed, w->scale, out, n, row, w->K_pad);
+    for (int64_t b = 0; b < blocks; b += kLaunchBlocks) {
+      const dim3 grid(static_cast<unsigned>(blocks - b < kLaunchBlocks ? blocks - b : kLaunchBlocks));
+      kernel<<<grid, dim3(256), 0, st>>>(w->packed, w->scale, out, static_cast<decltype(n)>(b), n, row, w->K_pad);
+    }
   };
   if (whole && narrow) {
     run(dequant_f32<uint32_t>, static_cast<uint32_t>(items), w->K / 4);
@@ -382,17 +385,16 @@ extern "C" int chr_nf4_quantize(const float *src, const chr_nf4_dev_t *dst, int3
   const int ng = dst->K_pad >> 6;
   const int64_t groups = static_cast<int64_t>(dst->M) * ng;
   const int64_t blocks = (groups + 16 * kQuantUnroll - 1) / (16 * kQuantUnroll);
-  if (blocks > INT32_MAX) {
-    return -3;
-  }
-  const dim3 grid(static_cast<unsigned>(blocks)), block(256);
   hipStream_t st = static_cast<hipStream_t>(stream);
   uint8_t *packed = const_cast<uint8_t *>(dst->packed);
   uint16_t *scale = const_cast<uint16_t *>(dst->scale);
-  if ((dst->K & 3) == 0 && aligned16(src)) {
-    quantize_groups<true><<<grid, block, 0, st>>>(src, packed, scale, status, groups, dst->K, ng);
-  } else {
-    quantize_groups<false><<<grid, block, 0, st>>>(src, packed, scale, status, groups, dst->K, ng);
+  for (int64_t b = 0; b < blocks; b += kLaunchBlocks) {
+    const dim3 grid(static_cast<unsigned>(blocks - b < kLaunchBlocks ? blocks - b : kLaunchBlocks)), block(256);
+    if ((dst->K & 3) == 0 && aligned16(src)) {
+      quantize_groups<true><<<grid, block, 0, st>>>(src, packed, scale, status, b, groups, dst->K, ng);
+    } else {
+      quantize_groups<false><<<grid, block, 0, st>>>(src, packed, scale, status, b, groups, dst->K, ng);
+    }
   }
   return launch_rc();
 }
