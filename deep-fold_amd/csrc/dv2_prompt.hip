@@ -168,8 +168,10 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
   }
   int buf = 0;
   for (int c = c_lo; c < c_hi; ++c) {
-    // the requests of the next chunk (the last one asks for its own again: the waits below count
-    // requests); a row block's codes are asked for where the block's own are read
+    // The requests of the next chunk; a row block's codes are asked for where the block's own are read.
+    // The last chunk asks for its own again and drops it: with the requests behind a branch the loop
+    // took two to five times as long (1792 tokens through gate and up of 27648 x 5120 1.43 ms, 5.60; o of
+    // 5120 x 5120, where it is one chunk in seven, 255 us, 644).
     const int next = min(c + 1, c_hi - 1);
     load_x(next, buf ^ 1);
     load_s(next);

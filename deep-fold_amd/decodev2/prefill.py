@@ -87,8 +87,11 @@ def _gemm_cols(mat: DeviceLinear, x: torch.Tensor, residual: torch.Tensor | None
 
 def _plain(mats) -> bool:
     """Blobs laid out and aligned as the several-window products read them."""
-    return all(m.packed.is_contiguous() and m.scale.is_contiguous() and m.packed.data_ptr() % 16 == 0
-               and m.scale.data_ptr() % 8 == 0 for m in mats)
+    for m in mats:
+        packed, scale = m.packed, m.scale
+        if packed.data_ptr() & 15 or scale.data_ptr() & 7 or not (packed.is_contiguous() and scale.is_contiguous()):
+            return False
+    return True
 
 
 class ChunkPrefill:
@@ -140,19 +143,27 @@ class ChunkPrefill:
                     for m in mats]).contiguous())
 
     def _serves_windows(self) -> bool:
-        """Whether the products of the model are ones the pass over several windows repeats (asked
-        once per distinct shape); gate and up may also go through it window by window."""
+        """Whether the products of the model are ones the pass over several windows repeats; gate and
+        up may also go through it window by window.  The library is asked once per distinct shape, every
+        layer's blobs are looked at (weights may be exchanged between prompts)."""
         spec = self.state.spec
-        kinds = {}
+        if spec.hidden % 16 != 0 or spec.hidden > 16384:
+            return False
+        seen = set()
         for ly in self.weights.layers:
+            qkv = (ly.q, ly.k, ly.v) if ly.wqkv is None else (ly.wqkv,)
             if ly.gate.bias is not None or ly.up.bias is not None or (ly.wqkv is not None and ly.wqkv.bias is not None):
                 return False
-            qkv = (ly.wqkv,) if ly.wqkv is not None else (ly.q, ly.k, ly.v)
-            for kind, mats in ((0, qkv), (2, (ly.o,)), (2, (ly.down,))):
-                kinds.setdefault((kind, mats[0].K, tuple(m.M for m in mats), _plain(mats)), mats)
-        return (spec.hidden % 16 == 0 and spec.hidden <= 16384
-                and all(plain and dv2_prompt_serves([(m.packed, m.scale, m.M) for m in mats], k, kind)
-                        for (kind, k, _, plain), mats in kinds.items()))
+            mats = (*qkv, ly.o, ly.down)
+            if not _plain(mats):
+                return False
+            shape = tuple([(m.M, m.K) for m in mats])
+            if shape not in seen:
+                seen.add(shape)
+                if not all(dv2_prompt_serves([(m.packed, m.scale, m.M) for m in of], of[0].K, kind)
+                           for kind, of in ((2, (ly.o,)), (0, qkv), (2, (ly.down,)))):
+                    return False
+        return True
 
     def whole_windows(self, n: int) -> int:
         """Tokens in front of an ``n``-token prompt that go through together: its whole windows,
@@ -251,10 +262,15 @@ class ChunkPrefill:
         self._finish(start + n, logits)
 
     def run_windows(self, token_ids: torch.Tensor, start: int, *, logits: bool = True) -> None:
-        ids, start = self._checked(token_ids, start)
-        n = int(ids.numel())
+        n = int(token_ids.numel())
         if self.whole_windows(n) != n:
             raise ValueError(f"{n} tokens are not two or more whole windows this model takes together")
+        self._run_windows(token_ids, start, logits=logits)
+
+    def _run_windows(self, token_ids: torch.Tensor, start: int, *, logits: bool) -> None:
+        """``run_windows`` of as many tokens as ``whole_windows`` has just named."""
+        ids, start = self._checked(token_ids, start)
+        n = int(ids.numel())
         for first in range(0, n, self.PASS_MAX):
             part = ids[first:first + self.PASS_MAX]
             self.first_len.fill_(start + first + 1)

@@ -59,7 +59,7 @@ def consume_prompt(state: DecodeState, weights: DeviceWeights, token_ids: Sequen
         # the whole windows in front go through together, with the bits of one after the other
         first_window = prefill.whole_windows(len(ids))
         if first_window:
-            prefill.run_windows(on_device[:first_window], slot0, logits=first_window == len(ids))
+            prefill._run_windows(on_device[:first_window], slot0, logits=first_window == len(ids))
     for first, past, final in _windows(len(ids), _window_width(state, chunk, prefill)):
         if past <= first_window:
             continue
