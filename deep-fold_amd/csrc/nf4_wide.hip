@@ -604,6 +604,21 @@ extern "C" int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N) {
   return wide_ws(a, wide_plan(a.M, N, a.groups));
 }
 
+extern "C" int chr_nf4_wide_plan(const chr_nf4_dev_t *w, int32_t N, int32_t *rows, int32_t *tokens, int32_t *splits) {
+  WideArgs a{};
+  if (rows == nullptr || tokens == nullptr || splits == nullptr) {
+    return -1;
+  }
+  if (const int rc = wide_args(w, N, a)) {
+    return rc;
+  }
+  const WidePlan p = wide_plan(a.M, N, a.groups);
+  *rows = kWideTiles[p.tile].wm * 64;
+  *tokens = kWideTiles[p.tile].bn;
+  *splits = p.splits;
+  return 0;
+}
+
 extern "C" int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y, float *ws,
                             int64_t ws_floats, const void *bias, void *stream) {
   return wide_entry(w, x, x_stride, N, y, ws, ws_floats, bias, stream, false);

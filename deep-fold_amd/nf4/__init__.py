@@ -187,6 +187,7 @@ EXPORTS = (
     ("chr_nf4_wide", ctypes.c_int, [_DP, _P, ctypes.c_int64, _I, _P, _P, ctypes.c_int64, _P, _P]),
     ("chr_nf4_wide_rows", ctypes.c_int, [_DP, _P, ctypes.c_int64, _I, _P, _P, ctypes.c_int64, _P, _P]),
     ("chr_nf4_wide_ws", ctypes.c_int64, [_DP, _I]),
+    ("chr_nf4_wide_plan", ctypes.c_int, [_DP, _I, *[ctypes.POINTER(ctypes.c_int32)] * 3]),
     ("chr_dv2_prompt_ws", ctypes.c_int64, [_DP, _I, _I, _I]),
     ("chr_dv2_prompt_gemm", ctypes.c_int, [_DP, _I, _I, _P, _I, _P, _P, ctypes.c_int64, _P, _P]),
     ("chr_dv2_prompt_add_rms", ctypes.c_int, [_DP, _P, _I, _P, _P, _P, _F, _P, _P, ctypes.c_int64, _P]),

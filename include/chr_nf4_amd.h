@@ -445,6 +445,8 @@ int chr_dv2_argmax_commit_ws(const void *logits, int32_t n, void *next_token, vo
 int chr_nf4_wide(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y,
                  float *ws, int64_t ws_floats, const void *bias, void *stream);
 int64_t chr_nf4_wide_ws(const chr_nf4_dev_t *w, int32_t N);
+/* The tile a launch would take (weight rows x tokens of a workgroup) and the splits of K.  No launch. */
+int chr_nf4_wide_plan(const chr_nf4_dev_t *w, int32_t N, int32_t *rows, int32_t *tokens, int32_t *splits);
 /* chr_nf4_wide on rows as they are: x 2-byte aligned (-5), x_stride >= K (-3), nothing read behind
  * element K of a row.  Same bits, same workspace. */
 int chr_nf4_wide_rows(const chr_nf4_dev_t *w, const void *x, int64_t x_stride, int32_t N, void *y,

@@ -87,3 +87,19 @@ def test_a_group_that_is_not_finite_is_left_alone(bad):
     s.reshape(5, 3)[3, 1] = np.float16(7.0)
     assert np.array_equal(packed.cpu().numpy(), p.reshape(5, 96))
     assert np.array_equal(scale.cpu().numpy().view(np.uint16), s.view(np.uint16).reshape(5, 3))
+
+
+# from 2^23 weights on the ragged decoder takes eight a thread, 2048 a workgroup: none of these counts is a multiple,
+# one is a single weight above the line
+@pytest.mark.parametrize("m,k,shift", [(1, (1 << 23) + 1, 0), (2100, 4003, 0), (2100, 4003, 1), (2050, 4096, 1)])
+def test_ragged_decoder_of_many_weights(m, k, shift):
+    kp = oc.k_pad(k)
+    rng = np.random.default_rng(m)
+    p = rng.integers(0, 256, size=(m, kp // 2), dtype=np.uint8)
+    s = (rng.random((m, kp // 64)).astype(np.float16) * np.float16(0.1)).view(np.uint16)
+    assert m * k >= 1 << 23 and (k % 4 != 0 or shift) and (m * k % 2048 != 0 or shift)
+    room = torch.full((m * k + shift + 1,), float("nan"), device="cuda")
+    out = room[shift:shift + m * k]
+    got = nf4.nf4_dequant(torch.from_numpy(p).cuda(), torch.from_numpy(s.view(np.float16)).cuda(), m, k, kp, out=out)
+    assert np.array_equal(got.cpu().numpy().view(np.uint32), oc.c_decode(p, s, m, k).reshape(-1).view(np.uint32))
+    assert bool(torch.isnan(room[shift + m * k:]).all()) and bool(torch.isnan(room[:shift]).all())

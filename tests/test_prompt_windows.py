@@ -158,3 +158,50 @@ def test_a_prompt_repeats_its_windows(spec, n, start):
     assert int(a.position.item()) == int(b.position.item()) == start + n
     assert torch.equal(a.kv.k, b.kv.k) and torch.equal(a.kv.v, b.kv.v)
     assert torch.equal(a.arena.logits, b.arena.logits) and int(a.next_token.item()) == int(b.next_token.item())
+
+
+@pytest.mark.gpu
+def test_a_prompt_of_several_passes(monkeypatch):
+    """More tokens than one pass takes: two whole passes, one of a single window, and a remainder."""
+    spec = dataclasses.replace(dv2.QWEN25_14B, n_layers=2, vocab=512, max_seq=384, eos_id=2)
+    weights = dv2.DeviceWeights.random(spec, seed=3)
+    ids = [int(t) for t in np.random.default_rng(2).integers(0, spec.vocab, size=347)]
+    states = []
+    for per_pass in (128, 2048):
+        monkeypatch.setattr(dv2.ChunkPrefill, "PASS_MAX", per_pass)
+        state = dv2.DecodeState.allocate(spec, device="cuda")
+        pre = dv2.ChunkPrefill(state, weights)
+        assert pre.whole_windows(340) == 320
+        dv2.consume_prompt(state, weights, ids[:7], prefill=pre)
+        dv2.consume_prompt(state, weights, ids[7:], start=7, prefill=pre)
+        states.append(state)
+    a, b = states
+    assert int(a.position.item()) == int(b.position.item()) == 347
+    assert torch.equal(a.kv.k, b.kv.k) and torch.equal(a.kv.v, b.kv.v) and torch.equal(a.arena.logits, b.arena.logits)
+
+
+# the sizes of a long prompt: 28 token tiles, splits and none, three matrices
+@pytest.mark.gpu
+@pytest.mark.parametrize("ms,k,kind", [((5120, 1024, 1024), 5120, 0), ((5120,), 5120, 2), ((2048,), 11008, 2), ((13824, 13824), 5120, 1)])
+def test_products_of_a_long_prompt(ms, k, kind):
+    n = 1792
+    mats = [matrix(m, k, i) for i, m in enumerate(ms)]
+    x = rand(n, k, seed=5).to(BF16)
+    assert nf4.dv2_prompt_serves(mats, k, kind)
+    if kind == 0:
+        assert torch.equal(nf4.dv2_prompt_gemm(mats, x, k), windows(lambda at: nf4.dv2_gemm_qkv(*mats, cols(x[at])), n))
+    elif kind == 1:
+        assert torch.equal(nf4.dv2_prompt_gemm(mats, x, k, swiglu=True),
+                           windows(lambda at: nf4.dv2_gemm_swiglu(*mats, cols(x[at])), n))
+    else:
+        m = ms[0]
+        res, g = rand(n, m, seed=3).to(BF16), rand(m, seed=4).to(BF16)
+        sums, norms = [], []
+        for lo in range(0, n, 64):
+            sq = torch.zeros(nf4.dv2_sq_blocks(m, 64) * 64, device="cuda")
+            y, written = nf4.nf4_gemm(*mats[0][:2], cols(x[lo:lo + 64]), m, k, k, 64, residual=cols(res[lo:lo + 64]), colsq=sq)
+            assert written
+            sums.append(y.t())
+            norms.append(nf4.dv2_rms_cols(y, g, 1e-6, colsq=sq).t())
+        h = nf4.dv2_prompt_add_rms(*mats[0][:2], x, m, k, res, norm_w=g)
+        assert torch.equal(res, torch.cat(sums)) and torch.equal(h, torch.cat(norms))

@@ -36,6 +36,11 @@ def test_arguments_are_refused_before_any_launch():
     assert lib.chr_nf4_wide(ctypes.byref(w), p, 13824, 128, p, p, need - 1, None, None) == -7
     assert lib.chr_nf4_wide(ctypes.byref(w), p, 13824, 128, p, p + 4, need, None, None) == -5
     assert lib.chr_nf4_wide_ws(ctypes.byref(w), 0) == -1
+    out = [ctypes.c_int32() for _ in range(3)]
+    refs = [ctypes.byref(o) for o in out]
+    assert lib.chr_nf4_wide_plan(ctypes.byref(w), 128, *refs) == 0 and out[2].value == need // (128 * 5120)
+    assert lib.chr_nf4_wide_plan(None, 128, *refs) == -1 and lib.chr_nf4_wide_plan(ctypes.byref(w), 128, None, *refs[1:]) == -1
+    assert lib.chr_nf4_wide_plan(ctypes.byref(w), 0, *refs) == -2
 
     def rows_rc(k=250, kp=256, x=p, stride=250, y=p):
         w = nf4._Dev(128, k, kp, 0x1000, 0x2000)
@@ -43,6 +48,47 @@ def test_arguments_are_refused_before_any_launch():
 
     assert rows_rc(x=None) == -1 and rows_rc(stride=249) == -3 and rows_rc(kp=320) == -4
     assert rows_rc(x=p + 1) == -5 and rows_rc(y=p + 2) == -5
+
+
+# (tile, splits or not) -> shapes just past its edges: rows and tokens that end inside it, rows that are no whole
+# vectors and some that are, odd group counts (a last half stage), a ragged K
+TILES = [((512, 128), True, (513, 7169, 2050)), ((512, 128), False, (257, 22017, 200)), ((256, 128), True, (513, 257, 1990)),
+         ((256, 128), True, (513, 260, 2112)), ((256, 128), False, (385, 5121, 320)), ((256, 128), False, (385, 5124, 300)),
+         ((256, 64), True, (33, 11009, 2050)), ((256, 64), True, (33, 11012, 2112)), ((256, 64), False, (385, 5121, 576)),
+         ((256, 64), False, (385, 5124, 570)), ((256, 32), True, (300, 257, 832)), ((256, 32), True, (385, 260, 1990)),
+         ((256, 32), False, (513, 2049, 320)), ((256, 32), False, (513, 2052, 300)), ((256, 16), True, (2, 255, 2050)),
+         ((256, 16), True, (16, 256, 2048)), ((256, 16), False, (2, 255, 320)), ((256, 16), False, (385, 1537, 1111))]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,split,shape", TILES, ids=[f"{t[0]}x{t[1]}-{'split' if p else 'whole'}-{s}" for t, p, s in TILES])
+@pytest.mark.parametrize("bias", [False, True])
+def test_every_tile(tile, split, shape, bias):
+    n, m, k = shape
+    kp = k_pad(k)
+    g = torch.Generator(device="cuda").manual_seed(m + k)
+    packed, scale = nf4.nf4_quantize(torch.randn(m, k, generator=g, device="cuda") * 0.05)
+    plan = [ctypes.c_int32() for _ in range(3)]
+    w = nf4._Dev(m, k, kp, packed.data_ptr(), scale.data_ptr())
+    assert nf4._load_ext().chr_nf4_wide_plan(ctypes.byref(w), n, *map(ctypes.byref, plan)) == 0
+    rows, tokens, splits = (p.value for p in plan)
+    assert ((rows, tokens), splits > 1) == (tile, split)      # a refit that moves a shape needs another one here
+    x = rand(n, k, seed=n)
+    b = rand(m, seed=5) if bias else None
+    want = x.double() @ nf4.nf4_dequant(packed, scale, m, k, kp).double().t()
+    want = want + b.double() if bias else want
+    got = nf4.nf4_wide(packed, scale, x, m, k, kp, bias=b)
+    close(got, want)
+    # a row or a token left out or taken twice hides in the norm of a large result: no element is far off.  Its
+    # error is the rounding of the result and a sum of k independent roundings of the levels, 1.15e-3 of the
+    # norm: six of their deviations
+    far = (got.double() - want).abs() - 2.0 ** -7 * want.abs()
+    assert float(far.max()) <= 6 * 1.15e-3 * float(want.pow(2).mean().sqrt()) + (2.0 ** -7 * float(b.abs().max()) if bias else 0)
+    # whole pieces and rows as they are: the same bits
+    padded = nf4.nf4_wide(packed, scale, torch.nn.functional.pad(x, (0, kp - k)), m, kp, kp, bias=b)
+    room = torch.full((n, k + 3), float("nan"), dtype=BF16, device="cuda")
+    room[:, 1:1 + k] = x
+    assert torch.equal(padded, got) and torch.equal(nf4.nf4_wide(packed, scale, room[:, 1:1 + k], m, k, kp, bias=b), got)
 
 
 # the padded copy of a ragged K and the rows as they are: one result, and what lies behind a row is not multiplied
@@ -82,8 +128,8 @@ def close(got, want):
     assert float((got - want).abs().max()) <= 2e-2 * max(float(want.abs().max()), 1e-3)
 
 
-# tile edges (16, 32, 64, 128 tokens; 256, 512 rows), odd group counts (a last half stage), ragged K (padded
-# copy), rows that are no whole vectors, few tokens over a long K (splits)
+# few tokens and many, odd group counts (a last half stage), ragged K, rows that are no whole vectors, few tokens
+# over a long K (splits); all but one take the 256 x 16 tile: test_every_tile has the others
 SHAPES = [(1, 64, 64), (2, 300, 128), (17, 5120, 1088), (33, 256, 576), (65, 256, 64), (63, 255, 192), (129, 513, 320), (70, 1030, 200), (128, 130, 2048),
           (257, 77, 1111), (66, 5120, 4160), (520, 512, 640)]
 
