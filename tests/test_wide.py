@@ -194,3 +194,29 @@ def test_many_tokens_through_a_small_seat(n):
     x = rand(n, k, seed=2)
     close(lin(x), x.double() @ w.t())
     assert torch.equal(lin(x), nf4.nf4_wide(p, s, x, m, k, k_pad(k))) == (n > 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,m,k", [(17, 2048, 2048), (5, 300, 500), (129, 96, 200), (8, 40, 72)])
+def test_the_seat_in_a_graph(n, m, k):
+    """Split and not, whole and ragged, and a small seat's window: replays with eager calls between them."""
+    (p, s, _), _ = matrix(m, k, seed=6)
+    lin = CompressedLinear(k, m, bias=True, device="cuda")
+    lin.attach(ChrMatrix("t", m, k, k_pad(k), p, s))
+    lin.set_bias(rand(m, seed=1))
+    x = rand(n, k, seed=2)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        lin(x)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = lin(x)
+    for i in range(4):
+        x.copy_(rand(n, k, seed=10 + i))
+        want = lin(x)
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
