@@ -50,7 +50,7 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
 
 // Bound: the matrix cores and the LDS reads beside them where the launch fills the chip (gate and up
 // of 27648 x 5120 at 1792 tokens 1.42 ms, 0.72 PFLOP/s), the table, first loads and the meeting of
-// the sums where a split is a few chunks (5120 x 5120 at 1792 in 3 splits 270 us, 0.35).  The window
+// the sums where a split is a few chunks (5120 x 5120 at 1792 in 3 splits 202 us, 0.46).  The window
 // launches it stands for took 54 ms for a 14B prompt of 512 tokens and 467 for a 32B one of 1791;
 // with it 30 and 266 (the 32B one with its remainder of 63 tokens staged as flat spans).
 //

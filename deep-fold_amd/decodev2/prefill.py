@@ -108,7 +108,8 @@ class ChunkPrefill:
 
     ``run_windows`` takes several whole windows in one token-major pass, layer by layer, with
     the bits ``run`` leaves on one after the other; ``whole_windows(n)`` says how many of ``n``
-    tokens ``consume_prompt`` sends there."""
+    tokens ``consume_prompt`` sends there.  Such a pass is launched eagerly (``use_graph`` or not)
+    and holds the activations of all its tokens."""
 
     MAX_WIDTH = int(PLAN_MAX_N)
     #: tokens of one pass over several windows: bounds its activations and partials
@@ -167,7 +168,8 @@ class ChunkPrefill:
 
     def whole_windows(self, n: int) -> int:
         """Tokens in front of an ``n``-token prompt that go through together: its whole windows,
-        where there are two or more of the default width."""
+        where there are two or more of the default width.  Two, as two graph replays and as one pass
+        (ms): 3B 8.45 / 6.96, 14B 12.7 / 10.7, 32B 24.9 / 17.9, two layers of the 3B 0.58 / 0.50."""
         whole = int(n) - int(n) % self.MAX_WIDTH
         if self.width != self.MAX_WIDTH or whole < 2 * self.MAX_WIDTH or not self._serves_windows():
             return 0
