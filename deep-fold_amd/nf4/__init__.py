@@ -1146,9 +1146,9 @@ def dv2_gemm_swiglu(gate, up, x: torch.Tensor) -> torch.Tensor:
     return y
 
 
-#: Products of this many weights x tokens take a ragged K from a padded copy: the copy (two launches,
-#: 3 to 8 us) costs less there than passing x through registers in the product (a tenth of it).  In
-#: the product / from a copy, us: 1000x1111 at 33 tokens 11.9 / 15.8, 8192x8200 at 33 32.5 / 36.4 and at
+#: Products of this many weights x tokens take a ragged K, or rows off the 16-byte grid, from a copy: it
+#: (padded, two launches, 3 to 8 us) costs less there than passing x through registers in the product (a
+#: tenth of it).  In the product / from a copy, us: 1000x1111 at 33 tokens 11.9 / 15.8, 8192x8200 at 33 32.5 / 36.4 and at
 #: 512 108.8 / 109.4, 27648x5000 at 33 63.5 / 60.8 and at 1024 387 / 349, 2048x11000 at 1024 78.9 / 87.6.
 PAD_MACS = 1 << 34
 
@@ -1165,8 +1165,10 @@ def nf4_wide(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int,
     _check_packed(packed, scale, M, K, K_pad)
     packed, scale = packed.contiguous(), scale.contiguous()
     n = int(x.size(0))
-    if K != K_pad and M * K * n >= PAD_MACS:
+    if M * K * n >= PAD_MACS and K != K_pad:
         x, K = torch.nn.functional.pad(x, (0, K_pad - K)), K_pad
+    elif M * K * n >= PAD_MACS and (x.stride(0) % 8 != 0 or x.data_ptr() % 16 != 0):
+        x = x.clone(memory_format=torch.contiguous_format)
     elif (x.stride(1) != 1 and K > 1) or x.stride(0) < K:
         x = x.clone(memory_format=torch.contiguous_format)
     _need(bias is None or (bias.is_cuda and bias.dtype == torch.bfloat16 and bias.is_contiguous()
