@@ -87,6 +87,7 @@ struct AttnArgs {
   // q + t*q_tok_stride, sees *valid_len + t cache rows, and writes dim d of a head to
   // out[t*out_tok_stride + (head*hd + d)*out_dim_stride]
   int q_tok_stride, out_tok_stride, out_dim_stride;
+  int n_tok;
   // one-workgroup forms: workgroups are dealt to the eight dies of the chip in turn (workgroup
   // b runs on die b % 8, each with its own L2).  With xcd_map the (head, part) of a workgroup
   // follows from b so that the query heads of one KV head that walk the same cache rows (the
@@ -618,6 +619,246 @@ __global__ __launch_bounds__(kWave * kMaxGqaWaves) void attn_chunk_gqa(const Att
   }
 }
 
+// The chunk attention on the matrix cores, 16 queries a workgroup, with the bits of attn_flash.
+//
+// attn_chunk_gqa is bound by its vector instructions: per (query, row) 128 products of q.k, 2 x 128 of the
+// rescale and the update, and a softmax that all 16 lanes of a row repeat.  The single-product fp32 matrix
+// instruction (16x16x1, four blocks) does the same multiply-adds in the same order, one fused multiply-add per
+// element and instruction, at twice the vector rate; a lane owns a (query, chain) pair, so the softmax is done
+// once.  Bound here: the fp32 matrix instructions and the vector ones, which take turns on one pipe (bf16
+// matrix instructions run beside vector ones, fp32 ones do not): a tile of 16 queries x 64 rows is 2048 clocks
+// of 64 matrix instructions a wavefront, some 190 vector ones, and the rescale where a maximum moves (a quarter
+// of the time on random scores).  40 query heads on 8: 1728 tokens 1085 -> 496 us, 512 tokens 126 -> 62, 63
+// behind 1728 95 -> 67; 16 on 2: 512 tokens 63 -> 31, 2 to 32 tokens behind 1000 59 -> 43.
+//
+// Queries: 16 consecutive ones of a KV head, (token, head of the group) flattened, heads fastest.  Rows: as
+// attn_chunk_gqa's four wavefronts of four lane groups, row t belongs to chain t % 16, wavefront w takes
+// chains w, w + 4, w + 8, w + 12, each walked in row order.
+//  q.k  The 16 lanes of a row there each sum 8 dims by fused multiply-adds and are added pairwise: blocks
+//       of the instruction are such 8-dim pieces, eight instructions a piece; the 16 sums of a (query, row)
+//       end in one lane and are added in the same tree.  Row i of the tile is step i % 4 of chain i / 4, so a
+//       lane ends with four successive rows of one chain of one query.
+//  p.v  Blocks are the chains, the weight goes in as it left the softmax; result row i of block dt is dim
+//       8 i + dt, so that a lane's operand is one 16-byte load of a row.
+// acc * alpha is left out where no query of a chain moves its maximum (alpha is 1: exact).  Votes by 4 queries
+// instead of 16 (the sums transposed) save two thirds of these products and lose it to the branches (520 us).
+typedef __attribute__((ext_vector_type(16))) float F32x16;
+constexpr int kMfmaWaves = 4;
+constexpr int kMfmaQueries = 16;
+
+__global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const AttnArgs a) {
+  constexpr int HD = 128;
+  constexpr int kTile = 64;                              // rows of a step of the workgroup
+  constexpr int kStateStride = kMfmaWaves * HD + 4;      // floats of a query's states: the pad spreads the banks
+  __shared__ float sm[kMfmaQueries][kMfmaWaves], sl[kMfmaQueries][kMfmaWaves];
+  __shared__ __align__(16) float so[kMfmaQueries * kStateStride];
+  __shared__ float4 sq[4][2][kWave];
+
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int lane = threadIdx.x & (kWave - 1);
+  const int li = lane & 15, lg = lane >> 4;
+  const int rep = a.n_rep;
+  // the longest tiles first; neighbouring workgroups take different KV heads, so a KV head stays on a die
+  const int kv_head = static_cast<int>(blockIdx.x) % a.n_kv;
+  const int q0 = (static_cast<int>(gridDim.x) / a.n_kv - 1 - static_cast<int>(blockIdx.x) / a.n_kv) * kMfmaQueries;
+  const int n_queries = a.n_tok * rep;
+  const int first_len = *a.valid_len;
+  const int tok = min(q0 + li, n_queries - 1) / rep;
+  const int head = kv_head * rep + min(q0 + li, n_queries - 1) - tok * rep;
+  const int vl = min(first_len + tok, a.max_seq);
+  const int vl_min = min(first_len + q0 / rep, a.max_seq);
+  const int vl_max = min(first_len + min(q0 + kMfmaQueries - 1, n_queries - 1) / rep, a.max_seq);
+
+  // byte offsets in 32 bits (the host looks at the cache's size); rows past the last one read it again
+  const uint32_t row_bytes = static_cast<uint32_t>(a.n_kv) * HD * 2;
+  const uint32_t k_lane = static_cast<uint32_t>(kv_head) * HD * 2 + lg * 16;
+  const uint32_t v_lane = static_cast<uint32_t>(kv_head) * HD * 2 + li * 16;
+  const uint32_t last = static_cast<uint32_t>(max(vl_max - 1, 0)) * row_bytes;
+  const uint32_t k_last = last + k_lane, v_last = last + v_lane;
+  uint32_t k_at = static_cast<uint32_t>(16 * (li & 3) + wave + 4 * (li >> 2)) * row_bytes + k_lane;  // step li % 4 of chain li / 4
+  const int v_row = wave + 4 * lg;
+  uint32_t v_at = static_cast<uint32_t>(v_row) * row_bytes + v_lane;
+  uint4 kr[4], vr[4];
+  auto load_k = [&]() {
+    const char *src = reinterpret_cast<const char *>(a.k_cache) + min(k_at, k_last);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      kr[g] = *reinterpret_cast<const uint4 *>(src + g * 64);
+    }
+    k_at += kTile * row_bytes;
+  };
+  auto load_v = [&]() {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      vr[r] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(a.v_cache) +
+                                               min(v_at + 16 * r * row_bytes, v_last));
+    }
+    v_at += kTile * row_bytes;
+  };
+  load_k();
+  load_v();
+  // the queries as every wavefront reads them back a tile, widened: wavefront g brings pieces 4 g .. 4 g + 3
+  {
+    float qf[8];
+    widen8(*reinterpret_cast<const uint4 *>(a.q + static_cast<size_t>(tok) * a.q_tok_stride +
+                                            static_cast<size_t>(head) * HD + wave * 32 + lg * 8), qf);
+    sq[wave][0][lane] = make_float4(qf[0], qf[1], qf[2], qf[3]);
+    sq[wave][1][lane] = make_float4(qf[4], qf[5], qf[6], qf[7]);
+  }
+
+  F32x16 acc[8];
+#pragma unroll
+  for (int dt = 0; dt < 8; ++dt) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      acc[dt][e] = 0.f;
+    }
+  }
+  float m = kNegBig, l = 0.f;
+
+  __syncthreads();
+  auto from_lane = [](float v, int lane) {
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(lane * 4, __float_as_int(v)));
+  };
+  for (int base = 0; base < vl_max; base += kTile) {
+    const bool all = base + kTile <= vl_min;  // every row of the tile is live for every query
+    // pieces 4 g .. 4 g + 3 of the 16 rows, each result row's four added pairwise
+    float part[2][4];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      F32x16 d;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        d[i] = 0.f;
+      }
+      asm volatile("" ::: "memory");  // (read a tile: kept across the loop they take registers the sums need)
+      const float4 qa = sq[g][0][lane], qb = sq[g][1][lane];
+      const float qf[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+      float kf[8];
+      widen8(kr[g], kf);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        d = __builtin_amdgcn_mfma_f32_16x16x1f32(kf[s], qf[s], d, 0, 0, 0);
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float quad = (d[v] + d[4 + v]) + (d[8 + v] + d[12 + v]);
+        part[g >> 1][v] = (g & 1) != 0 ? part[g >> 1][v] + quad : quad;
+      }
+    }
+    load_k();
+    float sum[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      sum[r] = part[0][r] + part[1][r];
+    }
+    if (!all) {
+      // a row past a query's own: a score of -inf (scale > 0) leaves m, l and, with a weight of 0, the sums
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        sum[r] = base + 16 * r + v_row < vl ? sum[r] : -__builtin_inff();
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float dot = sum[r] * a.scale;
+      const uint64_t moved = __ballot(dot > m);
+      const float m2 = fmaxf(m, dot);
+      const float e = __expf(fmaf(a.scale, sum[r], -m2));  // as attn_flash's scaling and difference are contracted
+      float alpha = 1.f;
+      if (moved != 0) {
+        alpha = __expf(m - m2);
+        float f[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          f[b] = from_lane(alpha, 16 * b + li);
+        }
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          if ((static_cast<uint32_t>(moved >> (b < 2 ? 0 : 32)) & (0xFFFFu << (16 * (b & 1)))) != 0) {
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+#pragma unroll
+              for (int v = 0; v < 4; ++v) {
+                acc[dt][4 * b + v] *= f[b];
+              }
+            }
+          }
+        }
+        m = m2;
+      }
+      l = fmaf(l, alpha, e);
+      float vf[8];
+      widen8(vr[r], vf);
+      if (!all) {
+        // A query whose rows have ended has a weight of 0, which leaves its sums as they are unless the
+        // row holds an infinity or a NaN: those go in as 0 and are added below where the query is live.
+        bool odd = false;
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+          odd |= !(fabsf(vf[dt]) < __builtin_inff());
+        }
+        if (__ballot(odd) != 0) {
+#pragma unroll
+          for (int dt = 0; dt < 8; ++dt) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+              const float x = from_lane(vf[dt], 16 * (i >> 2) + 4 * lg + (i & 3)), f = from_lane(e, 16 * (i >> 2) + li);
+              if (!(fabsf(x) < __builtin_inff()) && base + 16 * r + wave + 4 * (i >> 2) < vl) {
+                acc[dt][i] = fmaf(f, x, acc[dt][i]);
+              }
+              __builtin_amdgcn_sched_barrier(0);  // one at a time: the registers are full
+            }
+            vf[dt] = fabsf(vf[dt]) < __builtin_inff() ? vf[dt] : 0.f;
+          }
+        }
+      }
+#pragma unroll
+      for (int dt = 0; dt < 8; ++dt) {
+        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x1f32(vf[dt], e, acc[dt], 0, 0, 0);
+      }
+    }
+    load_v();
+  }
+
+  // fold_lane_groups: the four chains of the wavefront, (0 1) (2 3) as the compiler contracts it there
+  float mg = fmaxf(m, __shfl_xor(m, 16, kWave));
+  mg = fmaxf(mg, __shfl_xor(mg, 32, kWave));
+  const float w = __expf(m - mg);
+  float wb[4], lb[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    wb[b] = from_lane(w, 16 * b + li);
+    lb[b] = from_lane(l, 16 * b + li);
+  }
+  if (lg == 0) {
+    sm[li][wave] = mg;
+    sl[li][wave] = fmaf(lb[0], wb[0], __fmul_rn(lb[1], wb[1])) + fmaf(lb[2], wb[2], __fmul_rn(lb[3], wb[3]));
+  }
+  float *dst = so + li * kStateStride + wave * HD + lg * 32;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    float o[8];
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+      o[dt] = fmaf(acc[dt][v], wb[0], __fmul_rn(acc[dt][4 + v], wb[1])) +
+              fmaf(acc[dt][8 + v], wb[2], __fmul_rn(acc[dt][12 + v], wb[3]));
+    }
+    *reinterpret_cast<float4 *>(dst + v * 8) = make_float4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<float4 *>(dst + v * 8 + 4) = make_float4(o[4], o[5], o[6], o[7]);
+  }
+  __syncthreads();
+  for (int item = threadIdx.x; item < kMfmaQueries * HD; item += kMfmaWaves * kWave) {
+    const int j = item / HD, d = item - j * HD;
+    if (q0 + j < n_queries) {
+      const int t = (q0 + j) / rep, h = kv_head * rep + (q0 + j) - t * rep;
+      merge_wg<kMfmaWaves>(sm[j], sl[j], so + j * kStateStride,
+                           a.out + static_cast<size_t>(t) * a.out_tok_stride + static_cast<size_t>(h) * HD * a.out_dim_stride,
+                           HD, kMfmaWaves, d, nullptr, a.out_dim_stride);
+    }
+  }
+}
+
 template <int LPT>
 bool launch_chunk_gqa(const AttnArgs &a, int n_rep, int n_waves, int n_tok, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(n_tok));
@@ -944,6 +1185,7 @@ int attn_common(const void *q, const void *k, const void *v, void *out, const vo
   a.scale = scale;
   a.out = static_cast<uint16_t *>(out);
   a.q_tok_stride = n_q * hd;
+  a.n_tok = n_tok;
   a.out_tok_stride = out_tok_stride;
   a.out_dim_stride = out_dim_stride;
   // heads that share cache rows on one die, where the (KV head, part) pairs deal out evenly
@@ -969,7 +1211,15 @@ int attn_common(const void *q, const void *k, const void *v, void *out, const vo
   bool shared = false;
   if (mode == 1 && n_tok > 1 && !rope && vec_ok && n_split <= kMaxGqaWaves) {
     const int n_rep = n_q / n_kv;
-    if (hd == 128) {
+    // the matrix cores' form from two tokens on: at 40 query heads on 8 with one tile a KV head (2 tokens behind
+    // 1000 rows) 39.7 us without, 38 to 40 with it, more of either in the comment at the kernel; it takes byte
+    // offsets of 32 bits and leaves rows out by a score of -inf, so scale > 0
+    if (hd == 128 && n_split == kMfmaWaves && scale > 0.f &&
+        static_cast<int64_t>(max_seq) * n_kv * hd < (int64_t{1} << 30)) {
+      const int64_t tiles = (static_cast<int64_t>(n_tok) * n_rep + kMfmaQueries - 1) / kMfmaQueries;
+      attn_chunk_mfma<<<dim3(static_cast<unsigned>(tiles * n_kv)), dim3(kWave * kMfmaWaves), 0, st>>>(a);
+      shared = true;
+    } else if (hd == 128) {
       shared = launch_chunk_gqa<16>(a, n_rep, n_split, n_tok, st);
     } else if (hd == 64) {
       shared = launch_chunk_gqa<8>(a, n_rep, n_split, n_tok, st);

@@ -141,6 +141,36 @@ def test_attn_chunk(n_q, n_kv, hd, max_seq, first, n, waves):
         assert (bf16_bits(one) == bf16_bits(out_t[t])).all(), t
 
 
+@pytest.mark.parametrize("n_q,n_kv,max_seq,first,n,odd", [
+    (8, 8, 96, 40, 33, False),    # one query head a KV head: 16 tokens a tile, two tiles and one query
+    (6, 2, 130, 1, 64, False),    # three: a tile begins inside a token; rows end on and around whole tiles of 64
+    (40, 8, 200, 0, 2, False),    # the first token sees nothing
+    (40, 8, 200, 63, 5, False), (16, 2, 200, 126, 4, False), (34, 2, 80, 30, 9, False), (4, 4, 64, 60, 9, False),
+    (40, 8, 320, 250, 70, True), (6, 2, 150, 20, 40, True), (1, 1, 70, 30, 17, True)])
+def test_attn_chunk_on_the_matrix_cores(n_q, n_kv, max_seq, first, n, odd):
+    """Four wavefronts, 128 dims: every token has the bits of the decode step's kernel, also where rows behind a
+    token's own (``odd``: and rows it sees) hold infinities and NaN."""
+    say("attn_chunk_mfma", n_q, n_kv, max_seq, first, n, odd)
+    q, kc, vc = rnd((n, n_q * 128), 31, 2.0), rnd((max_seq, n_kv, 128), 32), rnd((max_seq, n_kv, 128), 33)
+    last = min(first + n - 1, max_seq)
+    kc[last:], vc[last:] = np.nan, np.inf
+    if odd:
+        vc[first + n // 2, :, 5], vc[first + n // 2 + 1, 0, 7], vc[first - 3, 0, 100:103] = np.nan, np.inf, -np.inf
+        kc[last - 2] = np.nan
+    dq, dk, dv = bf16_tensor(q), bf16_tensor(kc), bf16_tensor(vc)
+    out = torch.zeros((n, n_q * 128), dtype=torch.bfloat16, device=DEV)
+    nf4.dv2_attn_chunk(dq, dk, dv, out, torch.tensor(first, dtype=torch.int32, device=DEV), 128 ** -0.5, n_waves=4,
+                       feature_major=False)
+    one = torch.zeros(n_q * 128, dtype=torch.bfloat16, device=DEV)
+    for t in range(n):
+        nf4.dv2_attn(dq[t].view(n_q, 128), dk, dv, one, torch.tensor(first + t, dtype=torch.int32, device=DEV),
+                     128 ** -0.5, n_waves=4)
+        nan = torch.isnan(one)
+        assert odd or not nan.any(), t
+        assert torch.equal(nan, torch.isnan(out[t])), t
+        assert (bf16_bits(one.masked_fill(nan, 0)) == bf16_bits(out[t].masked_fill(nan, 0))).all(), t
+
+
 def test_attn_chunk_clamps_to_the_cache():
     n_q, n_kv, hd, max_seq, n = 2, 1, 16, 8, 4
     q, kc, vc = rnd((n, n_q * hd), 1), rnd((max_seq, n_kv, hd), 2), rnd((max_seq, n_kv, hd), 3)
