@@ -24,7 +24,7 @@ constexpr int kChunk = 256;       // K of a stage: four groups, as in the 64-col
 constexpr int kBlocks = 4;        // 32-row blocks of a wavefront
 constexpr int kTileRows = 2 * kBlocks * 32;
 constexpr int kXStage = kWindow * kChunk * 2;
-constexpr int kScaleStage = 4 * kTileRows * 4;
+constexpr int kScaleStage = 4 * kTileRows * 2;
 constexpr int kXAddr = kPairTableBytes;
 constexpr int kScaleAddr = kXAddr + 2 * kXStage;
 constexpr int kPromptLds = kScaleAddr + 2 * kScaleStage;
@@ -48,11 +48,12 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
   return f32_to_bf16(act * bf16_to_f32(f32_to_bf16(up)));
 }
 
-// Bound: the matrix cores and the LDS reads beside them where the launch fills the chip (gate and up
-// of 27648 x 5120 at 1792 tokens 1.42 ms, 0.72 PFLOP/s), the table, first loads and the meeting of
-// the sums where a split is a few chunks (5120 x 5120 at 1792 in 3 splits 202 us, 0.46).  The window
-// launches it stands for took 54 ms for a 14B prompt of 512 tokens and 467 for a 32B one of 1791;
-// with it 30 and 266 (the 32B one with its remainder of 63 tokens staged as flat spans).
+// Bound: a chunk of 256 K takes 4050 clocks of which the matrix cores work 2048; the rest is the vector
+// instructions that do not fit beside them (a scaling per product and token, an address per two weights), LDS
+// and the start of a chunk; 18 000 clocks a workgroup lie outside the loop.  Gate and up of 27648 x 5120 at
+// 1792 tokens 1.38 ms (0.74 PFLOP/s; 1.70 with every block's lookups, products and scaling one after the
+// other), down 5120 x 27648 0.70 (0.89), at 512 tokens 13824 x 5120 207 us (263), 5120 x 13824 104 (132),
+// 5120 x 5120 55 (69), 7168 x 5120 68 (86); the clock is at 1.9 to 2.3 GHz in these launches.
 //
 // 256 rows x 64 tokens.  As in the 64-column tile a wavefront sums group w % 4 of every chunk of
 // 256, four 16-wide products a group in the same order of k, scaled into its accumulators group by
@@ -61,10 +62,18 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
 // wavefront between barriers.  Tokens are the rows of the result: a lane holds one weight row's column
 // and its scale.  PAIR: row blocks alternate between gate and up.
 //
-// Codes: a lane pair fetches the 32 bytes of a row's group, ds_bpermute hands them to the lanes that
-// multiply them; x straight to LDS in 128-byte rows (a token's group), 16-byte pieces XORed with the
-// row's low bits; scales through LDS; all one chunk ahead.  At the end the four wavefronts' sums of
-// an output meet in LDS in group order.
+// Order inside a chunk: vector instructions run beside a matrix instruction if they stand between two of them
+// (up to six cost nothing; eight products in a row and then their scaling cost both times).  A unit is
+// the four products of 32 rows x 32 tokens; between them stand the scaling of the unit before and, in every
+// second unit, the lookups of the next row block, each into the operand register its product has just read
+// for the last time.  The order is pinned (sched_barrier): the compiler pulls the units apart again.
+//
+// Codes: a lane pair fetches the 32 bytes of a row's group; two neighbouring rows' fetches are handed to the
+// lanes that multiply them by two lane exchanges (hand_over; ds_bpermute, 6 clocks of LDS each, took a third
+// of its time).  x straight to LDS in 128-byte rows (a token's group), 16-byte pieces XORed with the row's low
+// bits, and so the scales.  Flat loads to LDS in flight turn every wait for a register into a wait for all of
+// them: codes, x and scales have half a chunk or more to arrive, which no launch here was seen to wait for
+// (without any of the loads the loop takes as long).
 template <bool PAIR>
 __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a) {
   extern __shared__ __align__(16) uint32_t smem[];
@@ -110,7 +119,7 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
 #pragma unroll
   for (int b = 0; b < kBlocks; ++b) {
     int mat;
-    const int row = locate(half * (kTileRows / 2) + b * 32 + (lane >> 1), mat);
+    const int row = locate(half * (kTileRows / 2) + (b >> 1) * 64 + (lane & ~1) + (b & 1), mat);
     const uint8_t *base = mat == 0 ? a.packed[0] : (mat == 1 ? a.packed[1] : a.packed[2]);
     wp[b] = base + static_cast<size_t>(row) * groups * 32 + g * 32 + (lane & 1) * 16;
   }
@@ -121,37 +130,50 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
     const uint16_t *base = mat == 0 ? a.scale[0] : (mat == 1 ? a.scale[1] : a.scale[2]);
     sp = base + static_cast<size_t>(row) * groups + (tid & 1) * 2;
   }
-  const int from_lane4 = (2 * r + h) * 4;
-  const uint16_t *xp =
-      a.x + static_cast<size_t>(tok0 + wave * 8 + (lane >> 3)) * a.K + ((lane & 7) ^ (lane >> 3)) * 8;
+  const bool odd = (lane & 1) != 0;
+  const char *xp = reinterpret_cast<const char *>(a.x + static_cast<size_t>(tok0) * a.K);
+  const uint32_t x_lane = (static_cast<uint32_t>(wave * 8 + (lane >> 3)) * a.K + ((lane & 7) ^ (lane >> 3)) * 8) * 2;
 
   auto load_x = [&](int c, int buf) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {  // group p of the chunk, tokens 8 wave .. + 8
-      load_to_lds16(xp + c * kChunk + p * kGroup,
+      load_to_lds16(reinterpret_cast<const uint16_t *>(xp + static_cast<size_t>(c) * (kChunk * 2) + x_lane + p * (kGroup * 2)),
                     static_cast<uint32_t>(kXAddr + buf * kXStage + p * (kWindow * 128) + wave * 1024));
     }
   };
-  uint4 cw[kBlocks];
-  uint32_t ns;
-  auto load_w = [&](int c, int b) { cw[b] = *reinterpret_cast<const uint4 *>(wp[b] + static_cast<size_t>(c) * 128); };
-  auto load_s = [&](int c) { ns = *reinterpret_cast<const uint32_t *>(sp + c * 4); };
-  auto store_s = [&](int buf) {
-    const uint32_t at = static_cast<uint32_t>(kScaleAddr + buf * kScaleStage + ((tid & 1) * 2 * kTileRows + (tid >> 1)) * 4);
-    *reinterpret_cast<__attribute__((address_space(3))) float *>(at) = f16_to_f32(static_cast<uint16_t>(ns));
-    *reinterpret_cast<__attribute__((address_space(3))) float *>(at + kTileRows * 4) = f16_to_f32(static_cast<uint16_t>(ns >> 16));
+  uint4 cw[2];
+  auto load_w = [&](int c, int b) { cw[b & 1] = *reinterpret_cast<const uint4 *>(wp[b] + static_cast<size_t>(c) * 128); };
+  auto load_s = [&](int c, int buf) {
+    load_to_lds4(sp + c * 4, static_cast<uint32_t>(kScaleAddr + buf * kScaleStage + wave * 256));
   };
-
+  // x of row 2 i and y of row 2 i + 1 hold half `lane & 1` of their rows' groups; afterwards lane (r, h) has half
+  // h of row r in lo and of row 32 + r in hi
+  auto hand_over = [&](uint32_t x, uint32_t y, uint32_t &lo, uint32_t &hi) {
+    const uint32_t xn = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), kDppQuadXor1, 0xF, 0xF, true));
+    const uint32_t yn = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(y), kDppQuadXor1, 0xF, 0xF, true));
+    const auto p = __builtin_amdgcn_permlane32_swap(odd ? yn : x, odd ? y : xn, false, false);
+    lo = p[0];
+    hi = p[1];
+  };
   load_x(c_lo, 0);
-  load_s(c_lo);
+  load_s(c_lo, 0);
+  load_w(c_lo, 0);
+  load_w(c_lo, 1);
+  // the table, its low levels literals (a byte a turn with two loads each, 4 us a workgroup)
+  {
+    uint32_t hi[2];
 #pragma unroll
-  for (int b = 0; b < kBlocks; ++b) {
-    load_w(c_lo, b);
+    for (int i = 0; i < 2; ++i) {
+      hi[i] = bf16_bits_rne(kLutBits[wave + i * 8]) << 16;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+#pragma unroll
+      for (int l = 0; l < 16; ++l) {
+        smem[(16 * (wave + i * 8) + l) * 64 + lane] = hi[i] | bf16_bits_rne(kLevelBits[l]);
+      }
+    }
   }
-  for (int b = wave; b < 256; b += kPromptThreads / kWave) {
-    smem[b * 64 + lane] = bf16_bits_rne(kLutBits[b & 15]) | (bf16_bits_rne(kLutBits[b >> 4]) << 16);
-  }
-  store_s(0);
   lds_loads_done();
   __syncthreads();
 
@@ -166,15 +188,48 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
       }
     }
   }
+  uint32_t codes[2][4];
+  Bf16x8 wf[4];
+  auto hand_over_pair = [&]() {
+    hand_over(cw[0].x, cw[1].x, codes[0][0], codes[1][0]);
+    hand_over(cw[0].y, cw[1].y, codes[0][1], codes[1][1]);
+    hand_over(cw[0].z, cw[1].z, codes[0][2], codes[1][2]);
+    hand_over(cw[0].w, cw[1].w, codes[0][3], codes[1][3]);
+  };
+  uint32_t at[4];  // table addresses of one of a block's four operands
+  auto address = [&](int b, int j, int k) {
+    constexpr uint32_t sel = 0x0C0C0400u;
+    at[k] = __builtin_amdgcn_perm(codes[b & 1][j], lane4, sel + (static_cast<uint32_t>(k) << 8));
+  };
+  auto look_up = [&](int j) {
+    const Raw16 f = {lds0_u32(at[0]), lds0_u32(at[1]), lds0_u32(at[2]), lds0_u32(at[3])};
+    wf[j] = __builtin_bit_cast(Bf16x8, f);
+  };
+  // the first block's operands, as every block before leaves them
+  hand_over_pair();
+  load_w(c_lo, 2);
+  load_w(c_lo, 3);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      address(0, j, k);
+    }
+    look_up(j);
+  }
+  F32x16 d[2];
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    d[1][v] = 0.f;
+  }
+  float s_old = 0.f;
   int buf = 0;
   for (int c = c_lo; c < c_hi; ++c) {
-    // The requests of the next chunk; a row block's codes are asked for where the block's own are read.
-    // The last chunk asks for its own again and drops it: with the requests behind a branch the loop
-    // took two to five times as long (1792 tokens through gate and up of 27648 x 5120 1.43 ms, 5.60; o of
-    // 5120 x 5120, where it is one chunk in seven, 255 us, 644).
+    // the last chunk asks for its own x again and drops it: requests behind a branch are waited for
     const int next = min(c + 1, c_hi - 1);
+    asm volatile("" ::: "memory");
     load_x(next, buf ^ 1);
-    load_s(next);
+    load_s(next, buf ^ 1);
     asm volatile("" ::: "memory");
     Bf16x8 xf[2][4];
 #pragma unroll
@@ -186,58 +241,85 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
         xf[t][j] = __builtin_bit_cast(Bf16x8, lds0_u128(at));
       }
     }
+    const uint32_t s_at = static_cast<uint32_t>(kScaleAddr + buf * kScaleStage + (half * (kTileRows / 2) + r) * 8 + g * 2);
 #pragma unroll
     for (int b = 0; b < kBlocks; ++b) {
-      uint32_t code[4] = {cw[b].x, cw[b].y, cw[b].z, cw[b].w};
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        code[j] = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(from_lane4, static_cast<int>(code[j])));
+      const float s_now = f16_to_f32(*reinterpret_cast<const __attribute__((address_space(3))) uint16_t *>(s_at + b * 256));
+      if (b & 1) {  // the codes of the next two blocks; their registers are asked for again behind it
+        __builtin_amdgcn_sched_barrier(0);
+        hand_over_pair();
+        __builtin_amdgcn_sched_barrier(0);
+        load_w(next, b == 1 ? 0 : 2);
+        load_w(next, b == 1 ? 1 : 3);
       }
-      load_w(next, b);
-      const float s = *reinterpret_cast<const __attribute__((address_space(3))) float *>(
-          static_cast<uint32_t>(kScaleAddr + buf * kScaleStage + (g * kTileRows + half * (kTileRows / 2) + b * 32 + r) * 4));
-      Bf16x8 wf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t w = code[j];
-        const Raw16 f = {pair_at<0>(w, lane4), pair_at<1>(w, lane4), pair_at<2>(w, lane4), pair_at<3>(w, lane4)};
-        wf[j] = __builtin_bit_cast(Bf16x8, f);
-      }
-      // the chains of the two token blocks take turns, ahead of the other wavefront's lookups (1792
-      // tokens through gate and up of 13824 / 27648 x 5120: 786 / 1476 us one after the other at even
-      // priority, 758 / 1418 so)
-      F32x16 d[2];
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        d[0][v] = 0.f;
-        d[1][v] = 0.f;
-      }
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        d[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[0][j], wf[j], d[0], 0, 0, 0);
-        d[1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[1][j], wf[j], d[1], 0, 0, 0);
-      }
-      __builtin_amdgcn_s_setprio(0);
 #pragma unroll
       for (int t = 0; t < 2; ++t) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          acc[b][t][v] = fmaf(s, d[t][v], acc[b][t][v]);
+        for (int j = 0; j < 4; ++j) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (j == 0) {
+            F32x16 z;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+              z[v] = 0.f;
+            }
+            d[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[t][j], wf[j], z, 0, 0, 0);
+          } else {
+            d[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xf[t][j], wf[j], d[t], 0, 0, 0);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          const int nb = (b + 1) & 3;
+          if (t == 0 && j == 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              address(nb, 0, k);
+            }
+          }
+          if (t == 1) {
+            look_up(j);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          if (t == 1 && j < 3) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+              address(nb, j + 1, k);
+            }
+          }
+          // unit before: (b, 0) beside (b, 1), (b - 1, 1) beside (b, 0)
+          const int pb = t == 1 ? b : (b + 3) & 3, pt = t ^ 1;
+          const float s = t == 1 ? s_now : s_old;
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            if (v * 3 / 16 == j - 1) {
+              acc[pb][pt][v] = fmaf(s, d[pt][v], acc[pb][pt][v]);
+            }
+          }
         }
       }
+      s_old = s_now;
     }
-    store_s(buf ^ 1);
-    lds_loads_done();
+    __builtin_amdgcn_sched_barrier(0);
+    // the next chunk's x and scales are the oldest requests but the four of codes since
+    asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     __syncthreads();
     buf ^= 1;
   }
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    acc[kBlocks - 1][1][v] = fmaf(s_old, d[1][v], acc[kBlocks - 1][1][v]);
+  }
+  lds_loads_done();
+  __syncthreads();
 
-  // the four wavefronts' sums of every output meet in LDS (the table and x are done with), two row
-  // blocks at a time; wavefront (half, g) finishes result rows 8g .. 8g + 7 of each 32 tokens
+  // The four wavefronts' sums of every output meet in LDS (the table and x are done with), two row blocks at
+  // a time.  There lanes 4 i .. 4 i + 3 of a result register are four successive rows of one token: a thread
+  // adds the four sums of these, in group order, and stores them as one vector (a row of one token a lane and
+  // four bytes a store, the stores took as long as two chunks).
   float *sums = reinterpret_cast<float *>(smem);
   static_assert(2 * 2 * 8 * 16 * kWave * 4 <= kScaleAddr, "the sums of two row blocks fit");
   const size_t row_floats = static_cast<size_t>(PAIR ? 2 * a.M : a.M);
+  const int quad = (tid & 7) * 4, at_h = (tid >> 3) & 1, at_v = (tid >> 4) & 15;  // rows, and the token's place
+  const int at_half = tid >> 8;
 #pragma unroll
   for (int pass = 0; pass < kBlocks / 2; ++pass) {
     if (pass > 0) {
@@ -254,49 +336,56 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
       }
     }
     __syncthreads();
-    int row[2];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      row[b] = out_row(half * (kTileRows / 2) + (2 * pass + b) * 32 + r);
-    }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      F32x4 o[2];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int v = 4 * g + u;
-        float o[2];
+      for (int b = 0; b < 2; ++b) {
+        o[b] = F32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          o[b] = 0.f;
+        for (int q = 0; q < 4; ++q) {
+          const F32x4 part = *reinterpret_cast<const F32x4 *>(
+              sums + (((b * 2 + t) * 8 + 4 * at_half + q) * 16 + at_v) * kWave + at_h * 32 + quad);
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            o[b] += sums[(((b * 2 + t) * 8 + 4 * half + q) * 16 + v) * kWave + lane];
+          for (int e = 0; e < 4; ++e) {
+            o[b][e] += part[e];
           }
         }
-        const size_t tok = static_cast<size_t>(tok0 + t * 32 + 8 * g + 4 * h + u);
-        if constexpr (PAIR) {
-          if (row[0] < a.M) {
-            if (a.part != nullptr) {
-              float *dst = a.part + (static_cast<size_t>(split) * a.N + tok) * row_floats + row[0];
-              dst[0] = o[0];
-              dst[a.M] = o[1];
-            } else {
-              a.y[tok * a.M + row[0]] = swiglu_bf16(o[0], o[1]);
-            }
-          }
-        } else {
+      }
+      const size_t tok = static_cast<size_t>(tok0 + t * 32 + 8 * (at_v >> 2) + 4 * at_h + (at_v & 3));
+      if constexpr (PAIR) {
+        const int row = out_row(at_half * (kTileRows / 2) + 2 * pass * 32 + quad);
+        if (row < a.M) {
+          if (a.part != nullptr) {
+            float *dst = a.part + (static_cast<size_t>(split) * a.N + tok) * row_floats + row;
+            *reinterpret_cast<F32x4 *>(dst) = o[0];
+            *reinterpret_cast<F32x4 *>(dst + a.M) = o[1];
+          } else {
+            uint32_t out[4];
 #pragma unroll
-          for (int b = 0; b < 2; ++b) {
-            if (row[b] < a.M) {
-              if (a.part != nullptr) {
-                a.part[(static_cast<size_t>(split) * a.N + tok) * row_floats + row[b]] = o[b];
-              } else {
-                uint16_t out = f32_to_bf16(o[b]);
+            for (int e = 0; e < 4; ++e) {
+              out[e] = swiglu_bf16(o[0][e], o[1][e]);
+            }
+            *reinterpret_cast<uint2 *>(a.y + tok * a.M + row) = make_uint2(out[0] | (out[1] << 16), out[2] | (out[3] << 16));
+          }
+        }
+      } else {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const int row = out_row(at_half * (kTileRows / 2) + (2 * pass + b) * 32 + quad);
+          if (row < a.M) {
+            if (a.part != nullptr) {
+              *reinterpret_cast<F32x4 *>(a.part + (static_cast<size_t>(split) * a.N + tok) * row_floats + row) = o[b];
+            } else {
+              uint32_t out[4];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                out[e] = f32_to_bf16(o[b][e]);
                 if (a.bias != nullptr) {
-                  out = f32_to_bf16(bf16_to_f32(out) + bf16_to_f32(a.bias[row[b]]));
+                  out[e] = f32_to_bf16(bf16_to_f32(static_cast<uint16_t>(out[e])) + bf16_to_f32(a.bias[row + e]));
                 }
-                a.y[tok * a.M + row[b]] = out;
               }
+              *reinterpret_cast<uint2 *>(a.y + tok * a.M + row) = make_uint2(out[0] | (out[1] << 16), out[2] | (out[3] << 16));
             }
           }
         }
@@ -530,7 +619,8 @@ int prompt_args(const chr_nf4_dev_t *w, int32_t n_mats, bool pair, int32_t N, Pr
     rows += w[i].M;
   }
   a.split_chunks = window64_chunks(w, n_mats);
-  if (a.split_chunks < 1 || w[0].K % kChunk != 0 || rows > INT32_MAX / 2 || rows % 4 != 0 || w[0].M % 4 != 0) {
+  constexpr int kMostK = 1 << 24;  // a workgroup's rows of x lie within 32-bit byte offsets
+  if (a.split_chunks < 1 || w[0].K > kMostK || w[0].K % kChunk != 0 || rows > INT32_MAX / 2 || rows % 4 != 0 || w[0].M % 4 != 0) {
     return -3;
   }
   for (int i = n_mats; i <= kPromptMats; ++i) {

@@ -312,6 +312,11 @@ __device__ __forceinline__ void load_to_lds16(const uint16_t *src, uint32_t at) 
   __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint16_t *)src,
                                    reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(at), 16, 0, 0);
 }
+// The same with 4 bytes a lane: LDS at `at` + 4 * lane.
+__device__ __forceinline__ void load_to_lds4(const uint16_t *src, uint32_t at) {
+  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) uint16_t *)src,
+                                   reinterpret_cast<__attribute__((address_space(3))) uint32_t *>(at), 4, 0, 0);
+}
 __device__ __forceinline__ void lds_loads_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Compute units of the current device (256 on an MI355X), cached after the first call.

@@ -205,3 +205,18 @@ def test_products_of_a_long_prompt(ms, k, kind):
             norms.append(nf4.dv2_rms_cols(y, g, 1e-6, colsq=sq).t())
         h = nf4.dv2_prompt_add_rms(*mats[0][:2], x, m, k, res, norm_w=g)
         assert torch.equal(res, torch.cat(sums)) and torch.equal(h, torch.cat(norms))
+
+
+# rows 2 i and 2 i + 1 of a tile in two matrices, workgroups of a single chunk of K and of two
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,ms,k", [(64, (5120, 1021, 1027), 5120), (128, (4100,), 256), (64, (2048,), 1024),
+                                    (64, (4100,), 1280)])
+def test_products_at_the_ends_of_the_pipeline(n, ms, k):
+    mats = [matrix(m, k, i) for i, m in enumerate(ms)]
+    x = rand(n, k, seed=5).to(BF16)
+    assert nf4.dv2_prompt_serves(mats, k, 0)
+    if len(ms) == 3:
+        want = windows(lambda at: nf4.dv2_gemm_qkv(*mats, cols(x[at])), n)
+    else:
+        want = windows(lambda at: nf4.nf4_gemm(*mats[0][:2], cols(x[at]), ms[0], k, k, 64), n)
+    assert torch.equal(nf4.dv2_prompt_gemm(mats, x, k), want)
