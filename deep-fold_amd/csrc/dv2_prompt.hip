@@ -440,61 +440,90 @@ __global__ __launch_bounds__(256) void prompt_reduce(const float *__restrict__ p
       make_uint2(o[0] | (static_cast<uint32_t>(o[1]) << 16), o[2] | (static_cast<uint32_t>(o[3]) << 16));
 }
 
-// One workgroup a token, a thread 16 consecutive features: x += bf16(sum of the splits) (+ bias), and
-// with norm_w h = RMSNorm(x).  The squares are added as the 64-column tile's column sums and rms_cols
-// add them: a block of 16 rows in the order 0 4 1 5 2 6 3 7 8 12 9 13 10 14 11 15, sixteen chains of
-// every sixteenth block, the chains in order.
+// lane Q of every four
+template <int Q>
+__device__ __forceinline__ float of_quad(float v) {
+  return dpp_f32<Q * 0x55>(v);
+}
+
+// One workgroup a token: x += bf16(sum of the splits) (+ bias), and with norm_w h = RMSNorm(x).  Bound: the
+// partials it reads.  A thread takes four neighbouring features in each of four passes, so a wavefront's
+// requests are whole lines and all of a split's leave together (with 16 neighbouring features a thread 1728
+// tokens of 5120 behind three splits and behind six took 59 + 121 us, 83 in all so; 512 tokens 13, 11).  The
+// squares are added as the 64-column tile's column sums and rms_cols add them: a block of 16 rows in the order 0 4 1 5 2 6 3 7 8 12 9 13 10 14 11 15 (four lanes hold it, each
+// adds all of it), sixteen chains of every sixteenth block, the chains in order.
 __global__ __launch_bounds__(1024) void prompt_add_rms(const float *__restrict__ part, int splits, size_t stride, int M,
                                                        const uint16_t *__restrict__ bias, uint16_t *__restrict__ x,
                                                        const uint16_t *__restrict__ norm_w, float eps,
                                                        uint16_t *__restrict__ h) {
   __shared__ float block_sum[1024], chain[16];
-  const int b = threadIdx.x, blocks = M / 16;
-  const size_t at = static_cast<size_t>(blockIdx.x) * M + b * 16;
-  float f[16];
-  if (b < blocks) {
-    uint32_t packed[8];
-    *reinterpret_cast<uint4 *>(packed) = *reinterpret_cast<const uint4 *>(x + at);
-    *reinterpret_cast<uint4 *>(packed + 4) = *reinterpret_cast<const uint4 *>(x + at + 8);
+  const int tid = threadIdx.x, threads = blockDim.x, blocks = M / 16;
+  const size_t row = static_cast<size_t>(blockIdx.x) * M;
+  float f[4][4];
+  F32x4 s[4];
+  uint2 packed[4];
+  // requests without a branch: features past the last are its again, and dropped
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const F32x4 s = sum_in_order(part + at + 4 * q, splits, stride);
+  for (int p = 0; p < 4; ++p) {
+    const int m = min((p * threads + tid) * 4, M - 4);
+    packed[p] = *reinterpret_cast<const uint2 *>(x + row + m);
+    s[p] = *reinterpret_cast<const F32x4 *>(part + row + m);
+  }
+#pragma unroll 4
+  for (int j = 1; j < splits; ++j) {
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int m = min((p * threads + tid) * 4, M - 4);
+      const F32x4 v = *reinterpret_cast<const F32x4 *>(part + j * stride + row + m);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int i = 4 * q + e;
-        float t = bf16_to_f32(f32_to_bf16(s[e]));
-        if (bias != nullptr) {
-          t = bf16_to_f32(f32_to_bf16(t + bf16_to_f32(bias[b * 16 + i])));
-        }
-        const float was = (i & 1) != 0 ? bf16_hi(packed[i >> 1]) : bf16_lo(packed[i >> 1]);
-        f[i] = bf16_to_f32(f32_to_bf16(was + t));
+        s[p][e] += v[e];
       }
     }
+  }
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      packed[q] = f32x2_to_bf16x2(f[2 * q], f[2 * q + 1]);
+  for (int p = 0; p < 4; ++p) {
+    const int quad = p * threads + tid, m = quad * 4;  // (whole blocks of four quads are in or out)
+    if (m >= M) {
+      continue;
     }
-    *reinterpret_cast<uint4 *>(x + at) = *reinterpret_cast<const uint4 *>(packed);
-    *reinterpret_cast<uint4 *>(x + at + 8) = *reinterpret_cast<const uint4 *>(packed + 4);
+    const float was[4] = {bf16_lo(packed[p].x), bf16_hi(packed[p].x), bf16_lo(packed[p].y), bf16_hi(packed[p].y)};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float t = bf16_to_f32(f32_to_bf16(s[p][e]));
+      if (bias != nullptr) {
+        t = bf16_to_f32(f32_to_bf16(t + bf16_to_f32(bias[m + e])));
+      }
+      f[p][e] = bf16_to_f32(f32_to_bf16(was[e] + t));
+    }
+    *reinterpret_cast<uint2 *>(x + row + m) = make_uint2(f32x2_to_bf16x2(f[p][0], f[p][1]), f32x2_to_bf16x2(f[p][2], f[p][3]));
     float sum = 0.f;
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const int lo = 8 * (v >> 2) + (v & 3);
-      sum = __fadd_rn(sum, __fmul_rn(f[lo], f[lo]));
-      sum = __fadd_rn(sum, __fmul_rn(f[lo + 4], f[lo + 4]));
+    for (int e = 0; e < 4; ++e) {
+      const float a = of_quad<0>(f[p][e]), b = of_quad<1>(f[p][e]);
+      sum = __fadd_rn(sum, __fmul_rn(a, a));
+      sum = __fadd_rn(sum, __fmul_rn(b, b));
     }
-    block_sum[b] = sum;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float a = of_quad<2>(f[p][e]), b = of_quad<3>(f[p][e]);
+      sum = __fadd_rn(sum, __fmul_rn(a, a));
+      sum = __fadd_rn(sum, __fmul_rn(b, b));
+    }
+    if ((tid & 3) == 0) {
+      block_sum[quad >> 2] = sum;
+    }
   }
   if (norm_w == nullptr) {
     return;
   }
   __syncthreads();
-  if (b < 16) {
+  if (tid < 16) {
     float t = 0.f;
-    for (int i = b; i < blocks; i += 16) {
+    for (int i = tid; i < blocks; i += 16) {
       t += block_sum[i];
     }
-    chain[b] = t;
+    chain[tid] = t;
   }
   __syncthreads();
   float t = 0.f;
@@ -503,15 +532,18 @@ __global__ __launch_bounds__(1024) void prompt_add_rms(const float *__restrict__
     t += chain[i];
   }
   const float inv = rsqrtf(t / static_cast<float>(M) + eps);
-  if (b < blocks) {
-    uint32_t out[8];
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      out[q] = f32x2_to_bf16x2((bf16_to_f32(norm_w[b * 16 + 2 * q]) * f[2 * q]) * inv,
-                               (bf16_to_f32(norm_w[b * 16 + 2 * q + 1]) * f[2 * q + 1]) * inv);
+  for (int p = 0; p < 4; ++p) {
+    const int m = (p * threads + tid) * 4;
+    if (m >= M) {
+      continue;
     }
-    *reinterpret_cast<uint4 *>(h + at) = *reinterpret_cast<const uint4 *>(out);
-    *reinterpret_cast<uint4 *>(h + at + 8) = *reinterpret_cast<const uint4 *>(out + 4);
+    float out[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      out[e] = (bf16_to_f32(norm_w[m + e]) * f[p][e]) * inv;
+    }
+    *reinterpret_cast<uint2 *>(h + row + m) = make_uint2(f32x2_to_bf16x2(out[0], out[1]), f32x2_to_bf16x2(out[2], out[3]));
   }
 }
 
