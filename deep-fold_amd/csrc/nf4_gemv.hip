@@ -91,6 +91,8 @@ struct StreamArgs {
   // its y; sq_in (with rms_w): this launch takes mean(x^2) from them instead of summing x.
   float *sq_out;
   const float *sq_in;
+  // plain kernel: add meets the sum rounded to bf16, as an addition behind the launch would
+  int add_rounded;
 };
 
 // Sum of a value over a workgroup of kStagedThreads threads, the same in every thread.
@@ -825,6 +827,9 @@ __global__ __launch_bounds__(256) void gemv_stream(const StreamArgs a) {
       if (writer && lane == u && r < M) {
         float v = sv;
         if (add != nullptr) {
+          if (a.add_rounded != 0) {
+            v = bf16_to_f32(f32_to_bf16(v));
+          }
           v += bf16_to_f32(add[r]);
         }
         y[r] = f32_to_bf16(v);
@@ -2044,9 +2049,11 @@ int launch_pairs(StreamArgs &a, int m_pairs, hipStream_t st) {
 
 }  // namespace
 
-// Shared with the GEMM entry points, which route N == 1 here.
+// Shared with the GEMM entry points, which route N == 1 here.  `rounded`: add is a bias that meets the
+// product's bf16.  The plain kernel adds it (2048 x 2048 through the linear seat 22.3 -> 17.0 us); the staged
+// ones, whose launches are that much longer, leave it to a launch behind them.
 int gemv_entry(const chr_nf4_dev_t *w, const void *x, void *y, void *stream, const void *add,
-               const void *rms_w, float rms_eps, const float *sq_in, float *sq_out) {
+               const void *rms_w, float rms_eps, const float *sq_in, float *sq_out, bool rounded) {
   if (w == nullptr || x == nullptr || y == nullptr) {
     return -1;
   }
@@ -2075,6 +2082,12 @@ int gemv_entry(const chr_nf4_dev_t *w, const void *x, void *y, void *stream, con
   a.rms_eps = rms_eps;
   a.sq_in = sq_in;
   a.sq_out = sq_out;
+  a.add_rounded = rounded ? 1 : 0;
+  if (rounded && pick_family(a, w->M) != 0) {
+    a.add[0] = nullptr;
+    const int rc = launch_rows(a, 1, w->M, static_cast<hipStream_t>(stream));
+    return rc != 0 ? rc : chr_dv2_add_cols(y, nullptr, add, w->M, 1, stream);
+  }
   return launch_rows(a, 1, w->M, static_cast<hipStream_t>(stream));
 }
 
@@ -2167,13 +2180,20 @@ using namespace chr;
 
 extern "C" int chr_nf4_gemv(const chr_nf4_dev_t *w, const void *x, void *y, void *stream,
                             const void *add, const void *rms_w, float rms_eps) {
-  return gemv_entry(w, x, y, stream, add, rms_w, rms_eps, nullptr, nullptr);
+  return gemv_entry(w, x, y, stream, add, rms_w, rms_eps, nullptr, nullptr, false);
+}
+
+extern "C" int chr_nf4_gemv_bias(const chr_nf4_dev_t *w, const void *x, void *y, const void *bias, void *stream) {
+  if (bias == nullptr) {
+    return -1;
+  }
+  return gemv_entry(w, x, y, stream, bias, nullptr, 0.f, nullptr, nullptr, true);
 }
 
 extern "C" int chr_dv2_gemv_sumsq(const chr_nf4_dev_t *w, const void *x, void *y, void *stream,
                                   const void *add, const void *rms_w, float rms_eps,
                                   const float *sumsq_in, float *sumsq_out) {
-  return gemv_entry(w, x, y, stream, add, rms_w, rms_eps, sumsq_in, sumsq_out);
+  return gemv_entry(w, x, y, stream, add, rms_w, rms_eps, sumsq_in, sumsq_out, false);
 }
 
 extern "C" int32_t chr_dv2_sumsq_parts(void) { return kSumsqParts; }

@@ -56,12 +56,14 @@ def nf4_linear(x: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, M: in
     if n < 1:
         raise ValueError(f"x{tuple(x.shape)} holds no token to multiply")
     rows = x.to(torch.bfloat16).reshape(n, K)
+    # a launch adds a bias it can add as torch would: bf16, one element a feature, values alone
+    folds = (bias is not None and bias.dtype == torch.bfloat16 and tuple(bias.shape) == (M,)
+             and bias.is_contiguous() and bias.device == rows.device and _values_alone(bias))
     if n == 1:
-        out = nf4_gemv(packed, scale, rows.reshape(K), M, K, K_pad).reshape(1, M)
+        out = nf4_gemv(packed, scale, rows.reshape(K), M, K, K_pad, bias=bias if folds else None).reshape(1, M)
+        if folds:
+            bias = None
     elif M * K >= WIDE_MIN_CODES or n > WINDOW_TOKENS:
-        # the launch adds a bias it can add as torch would: bf16, one element a feature, values alone
-        folds = (bias is not None and bias.dtype == torch.bfloat16 and tuple(bias.shape) == (M,)
-                 and bias.is_contiguous() and bias.device == rows.device and _values_alone(bias))
         out = nf4_wide(packed, scale, rows, M, K, K_pad, bias=bias if folds else None)
         if folds:
             bias = None

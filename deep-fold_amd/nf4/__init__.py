@@ -142,6 +142,7 @@ EXPORTS = (
     ("chr_nf4_set_tuning", None, [_I, _I, _I]),
     ("chr_nf4_gemm_stream_policy", None, [_I]),
     ("chr_nf4_gemv", ctypes.c_int, [_DP, _P, _P, _P, _P, _P, _F]),
+    ("chr_nf4_gemv_bias", ctypes.c_int, [_DP, _P, _P, _P, _P]),
     ("chr_nf4_gemv_qkv", ctypes.c_int, [_DP, _DP, _DP, _P, _P, _P, _P, _P, _P, _P, _P, _P, _F]),
     ("chr_nf4_gemv_swiglu", ctypes.c_int, [_DP, _DP, _P, _P, _P, _P, _F]),
     ("chr_nf4_rope_kv", ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _P]),
@@ -443,7 +444,8 @@ def _opt_sumsq(t: torch.Tensor | None, what: str):
 def nf4_gemv(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int, K: int,  # noqa: N803
              K_pad: int, out: torch.Tensor | None = None, add: torch.Tensor | None = None,  # noqa: N803
              rms_w: torch.Tensor | None = None, rms_eps: float = 1e-6,
-             sumsq_in: torch.Tensor | None = None, sumsq_out: torch.Tensor | None = None) -> torch.Tensor:
+             sumsq_in: torch.Tensor | None = None, sumsq_out: torch.Tensor | None = None,
+             bias: torch.Tensor | None = None) -> torch.Tensor:
     """N=1 GEMV.  ``x`` is bf16 ``[K, 1]`` or ``[K]``; ``y`` is ``[M, 1]``.
 
     Optional ``out`` is the destination (numel >= M).  Optional ``add`` is a
@@ -454,7 +456,9 @@ def nf4_gemv(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int,
     ``sumsq_out``: the launch also leaves the sum of squares of what it stored, in parts, for
     the launch that normalises ``y``; ``sumsq_in`` (with ``rms_w``): mean(x^2) comes from the
     parts the writer of ``x`` left instead of a sum over ``x`` (``chr_dv2_gemv_sumsq``; no
-    reference counterpart)."""
+    reference counterpart).
+
+    ``bias`` (alone): one bf16 element a row, added to the rounded product as ``y + bias`` would."""
     n = 1 if x.dim() == 1 else int(x.size(-1))
     if n != 1:
         raise RuntimeError(f"chr_nf4_gemv is N=1 only, got N={n}")
@@ -480,7 +484,13 @@ def nf4_gemv(packed: torch.Tensor, scale: torch.Tensor, x: torch.Tensor, M: int,
     add_keep, add_ptr = _opt_bf16(add, M, "add", exact=False)
     rms_keep, rms_ptr = _opt_bf16(rms_w, K, "rms_w", exact=True)
     w = _dev(packed, scale, M, K, K_pad)
-    if sumsq_in is None and sumsq_out is None:
+    if bias is not None:
+        _need(add is None and rms_w is None and sumsq_in is None and sumsq_out is None, "bias goes alone")
+        bias_keep, bias_ptr = _opt_bf16(bias, M, "bias", exact=True)
+        rc = _load_ext().chr_nf4_gemv_bias(ctypes.byref(w), x.data_ptr(), y.data_ptr(), bias_ptr, _stream())
+        _check_rc("chr_nf4_gemv_bias", rc)
+        del bias_keep
+    elif sumsq_in is None and sumsq_out is None:
         rc = _load_ext().chr_nf4_gemv(ctypes.byref(w), x.data_ptr(), y.data_ptr(), _stream(), add_ptr,
                                       rms_ptr, float(rms_eps))
         _check_rc("chr_nf4_gemv", rc)

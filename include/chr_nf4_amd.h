@@ -142,6 +142,11 @@ void chr_nf4_gemm_stream_policy(int32_t policy);
 int chr_nf4_gemv(const chr_nf4_dev_t *w, const void *x, void *y, void *stream,
                  const void *add, const void *rms_w, float rms_eps);
 
+/* y = bf16(W x) + bias[M], the sum rounded to bf16 once more: what an addition behind chr_nf4_gemv gives
+ * (gpu/host/linear.py:62-63), in its launch where that is below 16M codes, in a second one otherwise.
+ * -1 without a bias; otherwise chr_nf4_gemv's return codes. */
+int chr_nf4_gemv_bias(const chr_nf4_dev_t *w, const void *x, void *y, const void *bias, void *stream);
+
 /* One launch over q.M + k.M + v.M rows sharing x; optional bf16 biases are
  * added in fp32 before the single bf16 rounding.
  * Replaces chr_nf4_gemv_qkv (chr_gpu.h:99-103; nf4_gemv.cu:836-874). */

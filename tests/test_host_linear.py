@@ -155,3 +155,17 @@ def test_what_rides_on_a_bias_reaches_the_answer(monkeypatch):
     g = b.clone().requires_grad_()
     f(g).float().sum().backward()
     assert torch.equal(g.grad, torch.full_like(b, 4.0))
+
+
+# the plain kernel with whole, odd and K-split rows; kernels that leave the bias to a second launch
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,k", [(2048, 2048), (1001, 2560), (7, 64), (300, 16384), (4100, 1000), (5120, 5120)])
+def test_one_token_adds_its_bias_behind_the_rounding(m, k):
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    packed, scale = nf4.nf4_quantize(torch.randn(m, k, generator=gen, device="cuda") * 0.05)
+    x = torch.randn(1, 1, k, generator=gen, device="cuda").to(torch.bfloat16)
+    b = torch.randn(m, generator=gen, device="cuda").to(torch.bfloat16)
+    b[0] = float("-inf")
+    want = nf4_linear(x, packed, scale, m, k, k_pad(k)) + b
+    assert torch.equal(nf4_linear(x, packed, scale, m, k, k_pad(k), b), want)
+    assert nf4._load_ext().chr_nf4_gemv_bias(None, None, None, None, None) == -1
