@@ -19,7 +19,10 @@ constexpr int kMaxCols = 64;
 //   sq == nullptr: the workgroup reads the whole tile itself (a few hundred KB, in L2; all
 //                  workgroups add in one order, so all hold the same bits);
 //   sq != nullptr: the launch that stored x left sums per block of rows, sq[sq_blocks][N]
-//                  (chr_dv2_gemm_add_sq), and only those are added.  N divides 1024 then.
+//                  (chr_dv2_gemm_add_sq), and only those are added.  N divides 1024 then;
+//   chains != nullptr (not VEC, N > 16): cols_chains left the sums a thread's rows have here, one launch
+//                  for all workgroups (their additions, repeated by 64 workgroups, were the launch's time:
+//                  5120 rows of 17 to 31 columns 13.9 us, of 33 to 63 columns 25; 8.6 and 13 so, in two).
 //
 // Thread t owns column t % CP of rows t / CP, t / CP + 1024 / CP, ..; CP is N rounded up to a
 // power of two, threads whose column is >= N idle.  VEC: N is 8, 16, 32 or 64 and rows are 16-byte
@@ -30,7 +33,7 @@ __global__ __launch_bounds__(kColsBlock) void rms_cols(const uint16_t *__restric
                                                        uint16_t *__restrict__ y, int rows, int N,
                                                        int cp, float eps, int rows_per_wg,
                                                        const float *__restrict__ sq,
-                                                       int sq_blocks) {
+                                                       int sq_blocks, const float *__restrict__ chains) {
   __shared__ float part[kColsWaves][kMaxCols];
   __shared__ float inv[kMaxCols];
   const int lane = threadIdx.x & (kWave - 1);
@@ -87,6 +90,14 @@ __global__ __launch_bounds__(kColsBlock) void rms_cols(const uint16_t *__restric
       }
       __syncthreads();
     }
+  } else if (!VEC && chains != nullptr) {
+    // one or two rows of a step to a wavefront, as their lanes are folded below
+    const int c = lane, per = rstep / kColsWaves;
+    if (c < N) {
+      const float *from = chains + wave * per * kMaxCols + c;
+      part[wave][c] = per == 1 ? from[0] : from[0] + from[kMaxCols];
+    }
+    __syncthreads();
   } else {
     float ss[W];
 #pragma unroll
@@ -160,6 +171,32 @@ __global__ __launch_bounds__(kColsBlock) void rms_cols(const uint16_t *__restric
       const uint16_t xv = pre ? static_cast<uint16_t>(x0.x) : x[at];
       y[at] = f32_to_bf16((wk * bf16_to_f32(xv)) * inv[col]);
     }
+  }
+}
+
+// The chains of rms_cols<false> at more than 16 columns: chains[r][col] the squares of rows r, r + steps, .. of
+// column col, added in that order.  A wavefront a chain of rows, 32 of them in flight.
+__global__ __launch_bounds__(kWave) void cols_chains(const uint16_t *__restrict__ x, int rows, int N, int steps,
+                                                     float *__restrict__ chains) {
+  const int col = min(static_cast<int>(threadIdx.x), N - 1), r = blockIdx.x;
+  const int count = (rows - r + steps - 1) / steps;
+  float ss = 0.f;
+  constexpr int kBatch = 32;
+  for (int i0 = 0; i0 < count; i0 += kBatch) {
+    uint16_t v[kBatch];
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {  // (rows past the last are it again, and dropped)
+      v[u] = x[static_cast<size_t>(r + min(i0 + u, count - 1) * steps) * N + col];
+    }
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      if (i0 + u < count) {
+        ss = fmaf(bf16_to_f32(v[u]), bf16_to_f32(v[u]), ss);
+      }
+    }
+  }
+  if (static_cast<int>(threadIdx.x) < N) {
+    chains[r * kMaxCols + threadIdx.x] = ss;
   }
 }
 
@@ -306,8 +343,10 @@ using namespace chr;
 namespace chr {
 namespace {
 
+constexpr int kChainFloats = 32 * kMaxCols;
+
 int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps,
-                    const float *sq, int32_t sq_blocks, void *stream) {
+                    const float *sq, int32_t sq_blocks, void *stream, float *chains = nullptr) {
   if (x == nullptr || w == nullptr || y == nullptr) {
     return -1;
   }
@@ -333,11 +372,21 @@ int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t
   if (vec) {
     rms_cols<true><<<grid, dim3(kColsBlock), 0, st>>>(
         static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w),
-        static_cast<uint16_t *>(y), rows, N, cp, eps, rows_per_wg, sq, sq_blocks);
+        static_cast<uint16_t *>(y), rows, N, cp, eps, rows_per_wg, sq, sq_blocks, nullptr);
   } else {
+    // from a thousand rows on the second launch costs less than what it saves (1000 rows of 17 columns 5.3 us
+    // in one launch, of 33 columns 7.7)
+    const int steps = kColsBlock / cp;
+    if (sq != nullptr || cp < 32 || rows < 1024) {
+      chains = nullptr;
+    }
+    if (chains != nullptr) {
+      cols_chains<<<dim3(static_cast<unsigned>(steps)), dim3(kWave), 0, st>>>(static_cast<const uint16_t *>(x), rows, N, steps,
+                                                                              chains);
+    }
     rms_cols<false><<<grid, dim3(kColsBlock), 0, st>>>(
         static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w),
-        static_cast<uint16_t *>(y), rows, N, cp, eps, rows_per_wg, sq, sq_blocks);
+        static_cast<uint16_t *>(y), rows, N, cp, eps, rows_per_wg, sq, sq_blocks, chains);
   }
   return launch_rc();
 }
@@ -348,6 +397,16 @@ int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t
 extern "C" int chr_dv2_rms_cols(const void *x, const void *w, void *y, int32_t rows, int32_t N,
                                 float eps, void *stream) {
   return rms_cols_launch(x, w, y, rows, N, eps, nullptr, 0, stream);
+}
+
+extern "C" int32_t chr_dv2_rms_cols_ws_floats(void) { return kChainFloats; }
+
+extern "C" int chr_dv2_rms_cols_ws(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps, float *ws,
+                                   void *stream) {
+  if (ws == nullptr) {
+    return -1;
+  }
+  return rms_cols_launch(x, w, y, rows, N, eps, nullptr, 0, stream, ws);
 }
 
 extern "C" int chr_dv2_rms_cols_sq(const void *x, const void *w, void *y, int32_t rows, int32_t N,

@@ -168,6 +168,8 @@ EXPORTS = (
      [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _P, _P, _P, _P, _P, _I]),
     ("chr_dv2_gemv_attn", ctypes.c_int, [_DP, _P, _I, _I, _I, _P, _P, _P]),
     ("chr_dv2_rms_cols", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P]),
+    ("chr_dv2_rms_cols_ws_floats", ctypes.c_int32, []),
+    ("chr_dv2_rms_cols_ws", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P, _P]),
     ("chr_dv2_rope_kv_cols", ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     ("chr_dv2_attn_chunk", ctypes.c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I]),
     ("chr_dv2_swiglu_elems", ctypes.c_int, [_P, _P, _P, ctypes.c_int64, _P]),
@@ -1008,8 +1010,13 @@ def dv2_rms_cols(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor
                                              int(x.size(1)), float(eps), colsq.data_ptr(), blocks, _stream())
         _check_rc("chr_dv2_rms_cols_sq", rc)
         return out
-    rc = _load_ext().chr_dv2_rms_cols(x.data_ptr(), w.data_ptr(), out.data_ptr(), int(x.size(0)),
-                                      int(x.size(1)), float(eps), _stream())
+    lib, n = _load_ext(), int(x.size(1))
+    if n > 16 and n not in (32, 64):
+        ws = torch.empty(int(lib.chr_dv2_rms_cols_ws_floats()), dtype=torch.float32, device=x.device)
+        rc = lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), out.data_ptr(), int(x.size(0)), n, float(eps),
+                                     ws.data_ptr(), _stream())
+    else:
+        rc = lib.chr_dv2_rms_cols(x.data_ptr(), w.data_ptr(), out.data_ptr(), int(x.size(0)), n, float(eps), _stream())
     _check_rc("chr_dv2_rms_cols", rc)
     return out
 

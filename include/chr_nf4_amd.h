@@ -313,6 +313,12 @@ int chr_dv2_begin_step_sumsq(const chr_nf4_dev_t *table, const void *token, cons
 int chr_dv2_rms_cols(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps,
                      void *stream);
 
+/* chr_dv2_rms_cols, the same bits, with chr_dv2_rms_cols_ws_floats() fp32 elements of workspace: a tall tile
+ * whose columns are no whole vectors has its squares added once, in a launch of its own.  -1 without ws. */
+int32_t chr_dv2_rms_cols_ws_floats(void);
+int chr_dv2_rms_cols_ws(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps, float *ws,
+                        void *stream);
+
 /* chr_dv2_rms_cols with the column sums of squares supplied (what chr_dv2_gemm_add_sq left for
  * this x: sq[sq_blocks * N]) instead of read from the tile.  N must divide 1024.
  * No reference counterpart. */

@@ -51,6 +51,18 @@ def test_rms_cols(rows, n):
     assert np.abs(got - t.cpu().numpy().T).max() <= 2 ** -7 * max(1.0, np.abs(ref).max())
 
 
+# 32 and 16 chains a column, rows that end inside a step and inside a batch of 32, just above and below the line
+@pytest.mark.parametrize("rows,n", [(5120, 17), (1024, 31), (1025, 24), (5120, 63), (1039, 33), (4099, 50), (1023, 40)])
+def test_rms_cols_in_two_launches(rows, n):
+    say("rms_cols two launches", rows, n)
+    x, w = bf16_tensor(rnd((rows, n), rows + n, 1.5)), bf16_tensor(rnd((rows,), 3, 1.0))
+    one = torch.empty_like(x)
+    lib = nf4._load_ext()
+    assert lib.chr_dv2_rms_cols(x.data_ptr(), w.data_ptr(), one.data_ptr(), rows, n, 1e-6, nf4._stream()) == 0
+    assert torch.equal(nf4.dv2_rms_cols(x, w, 1e-6), one)
+    assert lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), one.data_ptr(), rows, n, 1e-6, None, None) == -1
+
+
 def test_rms_cols_rejects_wide_chunks():
     x = torch.zeros((64, 65), dtype=torch.bfloat16, device=DEV)
     with pytest.raises(RuntimeError):
