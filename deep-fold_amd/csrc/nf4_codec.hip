@@ -218,8 +218,9 @@ __device__ __constant__ const CellTable kCellTable = make_cells();
 // pieces and the four are loaded one by one), kQuantUnroll groups a lane with all loads first.
 // Steps are those of the CPU encoder: absmax, binary16 scale, divide by the widened scale, clip,
 // nearest level.  Bound by reading the fp32; one weight a lane, a wavefront a group and fifteen
-// squared distances a weight took 302 us at 13824x5120 (vector arithmetic), so 71 (4.5 TB/s; 68 with
-// four or eight groups a lane, which take 7 and 8 us at 1000x1111 against 5).
+// squared distances a weight took 302 us at 13824x5120 (vector arithmetic), dividing every weight 90,
+// so 72 (4 TB/s, launches back to back; 25 and 29 at 5120x5120).  Four groups a lane, or loads past the
+// caches, are no faster.
 constexpr int kQuantUnroll = 2;
 
 template <bool VEC>
@@ -283,13 +284,29 @@ __global__ __launch_bounds__(256) void quantize_groups(const float *__restrict__
       s16 = s32 > 65504.f ? 0x7BFFu : 0x3C00u;  // the largest finite scale, or one
       s = f16_to_f32(s16);
     }
+    // v / s decides nothing but the side of a crossing: the product with the reciprocal (an ulp off, as its
+    // product: 2^-22 at most) decides the same wherever it is further from it.  Nearer, one weight in 10^5, the
+    // wavefront divides.
+    const float inv = __builtin_amdgcn_rcpf(s);
     uint32_t codes = 0;
+    bool near = false;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float u = v[n][e] / s;
-      u = u > 1.f ? 1.f : (u < -1.f ? -1.f : u);
+      const float u = fminf(fmaxf(v[n][e] * inv, -1.f), 1.f);
       const int cell = static_cast<int>((u + 1.f) * 16.f);
-      codes |= (below[cell] + (u >= cross[cell] ? 1u : 0u)) << (4 * e);
+      const float past = u - cross[cell];
+      near |= fabsf(past) < 0x1p-21f;
+      codes |= (below[cell] + (past >= 0.f ? 1u : 0u)) << (4 * e);
+    }
+    if (__builtin_expect(__any(near), 0)) {
+      codes = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        float u = v[n][e] / s;
+        u = u > 1.f ? 1.f : (u < -1.f ? -1.f : u);
+        const int cell = static_cast<int>((u + 1.f) * 16.f);
+        codes |= (below[cell] + (u >= cross[cell] ? 1u : 0u)) << (4 * e);
+      }
     }
     if (aligned2(packed)) {
       reinterpret_cast<uint16_t *>(packed)[gi * 16 + lane] = static_cast<uint16_t>(codes);

@@ -69,6 +69,25 @@ def test_every_change_of_level():
         assert np.array_equal(gs.cpu().numpy().view(np.uint16), np.asarray(s).view(np.uint16)), f
 
 
+# the quantiser divides only where the reciprocal's product lies within 2^-21 of a change of level: weights on both
+# sides of that band, and within it, at scales whose reciprocal is rounded, at subnormal and at the largest ones
+@pytest.mark.parametrize("lo,hi", [(1, 1024), (1024, 0x3C00), (0x3C00, 0x7C00)])
+def test_the_reciprocal_and_the_division_choose_one_code(lo, hi):
+    levels = oc.LUT.astype(np.float64)
+    mids = (levels[1:] + levels[:-1]) / 2
+    steps = np.array([0, 1, 2, 3, 7, 15, 29, 31, 32, 33, 35, 63]) * 2.0 ** -26
+    u = (mids[:, None] + np.concatenate([steps, -steps])[None, :]).reshape(-1)
+    u = np.concatenate([u, np.zeros(-len(u) % 63)]).reshape(-1, 63)
+    rng = np.random.default_rng(lo)
+    scales = np.concatenate([[lo, hi - 1], rng.integers(lo, hi, 62)]).astype(np.uint16).view(np.float16).astype(np.float64)
+    w = np.concatenate([np.ones((len(u), 1)), u], axis=1)[None] * scales[:, None, None]
+    w = w.reshape(-1, 64).astype(np.float32)
+    p, s = oc.c_encode(w)
+    gp, gs = nf4.nf4_quantize(torch.from_numpy(w).cuda())
+    assert np.array_equal(gs.cpu().numpy().view(np.uint16), np.asarray(s).view(np.uint16).reshape(gs.shape))
+    assert np.array_equal(gp.cpu().numpy(), np.asarray(p).reshape(gp.shape))
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
 def test_a_group_that_is_not_finite_is_left_alone(bad):
     w = weights(5, 130, seed=1)
