@@ -497,6 +497,23 @@ __device__ __forceinline__ bool x_item(int N, int I, int lane, int &kp, int &q) 
 // LDS.  Element by element, each load waited for before the next, a tile of 63 columns took four
 // times one of 64 (27648x5120: 239 us against 58; as pieces 82, and 23 columns 40 for 61).  P pieces a thread of THREADS; the last elements,
 // short of a piece, are loaded where they are stored (they end x: nothing may be read behind them).
+//
+// Lane l of a wavefront holding piece l, the stores of one instruction fall into few of the LDS banks (a column is
+// 4 mod 64 banks from the next, a piece eight columns from the next).  For 33..63 columns, where these stores
+// bound the tile, pairs of pieces are dealt to the lanes sixteen pieces (two to four rows of x) apart: 648 passes
+// of the banks a tile for 2016 at 63 columns, 384 for 1152 at 48, a request still 32 whole bytes.  From a graph,
+// dealt and in order, us: 27648x5120 at 63 columns 68.0 and 87.5, 48 63.3 and 72.8, 33 61.7 and 64.3; 5120x27648
+// at 63 62.6 and 84.8; 5120x5120 23.5 and 28.0.  Fewer columns take as long either way (27648x5120 at 17 45.8 and
+// 44.2) and keep the order.
+template <int P, int THREADS>
+__device__ __forceinline__ int flat_piece(int u, int tid) {
+  if constexpr (P == 8 && THREADS == kGroupThreads) {  // (the tile of 33..64 columns: gemm_mfma<false, 2>)
+    return ((tid >> 6) << 9) + ((tid & 62) << 3) + (u << 1) + (tid & 1);
+  } else {
+    return tid + u * THREADS;
+  }
+}
+
 template <int P, int THREADS>
 __device__ __forceinline__ void fetch_flat(uint32_t *d, const uint16_t *__restrict__ x, int k0, int span, int K,
                                            int N, int tid) {
@@ -507,7 +524,7 @@ __device__ __forceinline__ void fetch_flat(uint32_t *d, const uint16_t *__restri
   const uint4 *src = reinterpret_cast<const uint4 *>(x + static_cast<size_t>(k0) * N);
 #pragma unroll
   for (int u = 0; u < P; ++u) {
-    const uint4 t = src[min(tid + u * THREADS, full - 1)];
+    const uint4 t = src[min(flat_piece<P, THREADS>(u, tid), full - 1)];
     d[4 * u + 0] = t.x;
     d[4 * u + 1] = t.y;
     d[4 * u + 2] = t.z;
@@ -526,7 +543,7 @@ __device__ __forceinline__ void scatter_flat(const uint32_t *d, const uint16_t *
   const uint32_t magic = static_cast<uint32_t>(((1ull << 32) + static_cast<uint32_t>(N) - 1) / static_cast<uint32_t>(N));
 #pragma unroll
   for (int u = 0; u < P; ++u) {
-    const int piece = tid + u * THREADS;
+    const int piece = flat_piece<P, THREADS>(u, tid);
     if (piece < full) {
       const int f = 8 * piece;
       int kk = static_cast<int>(__umulhi(static_cast<uint32_t>(f), magic));

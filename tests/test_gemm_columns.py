@@ -30,3 +30,11 @@ def test_odd_columns(n, m, k):
     # one bf16 rounding of each result (2^-9) over fp32 sums of the bf16 weights these tiles multiply
     assert float((y - want).abs().max()) <= 2.0 ** -8 * float(want.abs().max())
     assert float((y - want).norm()) <= 2.5e-3 * float(want.norm())
+
+
+# 33..63 columns are staged in an order of their own (512 pieces a wavefront): spans that end in each of its
+# wavefronts, within a pair and within a piece
+@pytest.mark.parametrize("n", [34, 39, 40, 48, 56, 61, 62])
+@pytest.mark.parametrize("m,k", [(33, 63), (130, 150), (64, 256), (33, 257), (64, 2047)])
+def test_columns_dealt_in_pairs(n, m, k):
+    test_odd_columns(n, m, k)
