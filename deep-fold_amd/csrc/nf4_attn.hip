@@ -761,6 +761,9 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
+      if (base + 16 * r + wave >= vl_max) {
+        break;  // no row of this step is any query's (9 tokens of 40 heads with nothing before them 7.2 -> 6.4 us)
+      }
       const float dot = sum[r] * a.scale;
       const uint64_t moved = __ballot(dot > m);
       const float m2 = fmaxf(m, dot);

@@ -157,6 +157,7 @@ def test_attn_chunk(n_q, n_kv, hd, max_seq, first, n, waves):
     (8, 8, 96, 40, 33, False),    # one query head a KV head: 16 tokens a tile, two tiles and one query
     (6, 2, 130, 1, 64, False),    # three: a tile begins inside a token; rows end on and around whole tiles of 64
     (40, 8, 200, 0, 2, False),    # the first token sees nothing
+    (40, 8, 200, 14, 4, False), (16, 2, 200, 46, 3, False),  # the last tile ends around a step of 16 rows
     (40, 8, 200, 63, 5, False), (16, 2, 200, 126, 4, False), (34, 2, 80, 30, 9, False), (4, 4, 64, 60, 9, False),
     (40, 8, 320, 250, 70, True), (6, 2, 150, 20, 40, True), (1, 1, 70, 30, 17, True)])
 def test_attn_chunk_on_the_matrix_cores(n_q, n_kv, max_seq, first, n, odd):
