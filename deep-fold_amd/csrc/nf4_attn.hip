@@ -17,6 +17,11 @@
 
 #include "nf4_common.h"
 
+// A prompt's attention gives the bits of the decode step's, from kernels of different shape.  So every product of
+// this file that goes unrounded into a sum is written as a fused multiply-add and the compiler fuses none by
+// itself (it chose by the code around: a branch more, and scale * dot - m was rounded once or twice).
+#pragma clang fp contract(off)
+
 namespace chr {
 namespace {
 
@@ -58,9 +63,12 @@ __device__ __forceinline__ void rope8(const uint16_t *t, const uint16_t *cos, co
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const float rot = low ? -b[i] : b[i];
-    out[i] = a[i] * c[i] + rot * s[i];
+    out[i] = fmaf(a[i], c[i], rot * s[i]);
   }
 }
+
+// The weight of a row in a softmax whose maximum is m: exp(scale * sum - m), the difference rounded once.
+__device__ __forceinline__ float row_weight(float scale, float sum, float m) { return __expf(fmaf(scale, sum, -m)); }
 
 struct AttnArgs {
   const uint16_t *q;
@@ -153,9 +161,10 @@ __device__ __forceinline__ void merge_head(const float *m_s, const float *l_s, c
     m = fmaxf(m, __shfl_xor(m, off, kWave));
   }
   const float my_w = __expf(my_m - m);  // weight of split `lane`
-  float l = my_w * my_l;
+  const float wl = my_w * my_l;
+  float l = fmaf(my_w, my_l, __shfl_xor(wl, 32, kWave));
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
+  for (int off = 16; off > 0; off >>= 1) {
     l += __shfl_xor(l, off, kWave);
   }
   const float inv = l > 0.f ? 1.f / l : 0.f;
@@ -180,12 +189,12 @@ __device__ __forceinline__ void merge_head(const float *m_s, const float *l_s, c
       }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        acc += __shfl(my_w, s + j, kWave) * v[j];
+        acc = fmaf(__shfl(my_w, s + j, kWave), v[j], acc);
       }
     }
     for (; s < n_split; ++s) {
       const float v = on ? *(oh + static_cast<size_t>(s) * hd + d) : 0.f;
-      acc += __shfl(my_w, s, kWave) * v;
+      acc = fmaf(__shfl(my_w, s, kWave), v, acc);
     }
     if (on) {
       if (state != nullptr) {
@@ -200,7 +209,8 @@ __device__ __forceinline__ void merge_head(const float *m_s, const float *l_s, c
 // Fold the kWave / LPT lane groups of a wavefront: lanes with equal lane % LPT hold online-softmax
 // states (m, l, acc[8]) of different time-step subsets; afterwards every lane holds the state of
 // their union.  (The row-swap instructions in place of the shuffles for offsets 16 and 32 were
-// measured: no faster.)
+// measured: no faster.)  The first addition is fused, a lane's own product unrounded; of two groups alone (LPT 32)
+// both products are rounded.
 template <int LPT>
 __device__ __forceinline__ void fold_lane_groups(float &m, float &l, float (&acc)[8]) {
   if constexpr (LPT < kWave) {
@@ -210,13 +220,17 @@ __device__ __forceinline__ void fold_lane_groups(float &m, float &l, float (&acc
       mg = fmaxf(mg, __shfl_xor(mg, off, kWave));
     }
     const float w = __expf(m - mg);
-    l *= w;
+    auto add_first = [&](float v) {
+      const float own = v * w, other = __shfl_xor(own, LPT, kWave);
+      return LPT < 32 ? fmaf(v, w, other) : own + other;
+    };
+    l = add_first(l);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      acc[i] *= w;
+      acc[i] = add_first(acc[i]);
     }
 #pragma unroll
-    for (int off = LPT; off < kWave; off <<= 1) {
+    for (int off = 2 * LPT; off < kWave; off <<= 1) {
       l += __shfl_xor(l, off, kWave);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -414,13 +428,11 @@ __global__ __launch_bounds__(INWG ? kWave * WMAX : kWave) void attn_flash(const 
       for (int i = 0; i < 8; ++i) {
         dot = fmaf(qf[i], kf[i], dot);
       }
-      dot = group_sum<LPT>(dot) * a.scale;
+      dot = group_sum<LPT>(dot);
       if (live[u]) {
-        const float m2 = fmaxf(m, dot);
+        const float m2 = fmaxf(m, dot * a.scale);
         const float alpha = __expf(m - m2);
-        const float e = __expf(dot - m2);
-        // (explicit fused multiply-adds: written a * b + c * d the compiler chooses per kernel
-        // which product to fuse, and the chunk kernel must round exactly like this one)
+        const float e = row_weight(a.scale, dot, m2);
         l = fmaf(l, alpha, e);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -578,11 +590,11 @@ __global__ __launch_bounds__(kWave * kMaxGqaWaves) void attn_chunk_gqa(const Att
         for (int i = 0; i < 8; ++i) {
           dot = fmaf(qf[r][i], kf[i], dot);
         }
-        dot = group_sum<LPT>(dot) * a.scale;
+        dot = group_sum<LPT>(dot);
         if (live) {
-          const float m2 = fmaxf(m[r], dot);
+          const float m2 = fmaxf(m[r], dot * a.scale);
           const float alpha = __expf(m[r] - m2);
-          const float e = __expf(dot - m2);
+          const float e = row_weight(a.scale, dot, m2);
           l[r] = fmaf(l[r], alpha, e);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
@@ -767,7 +779,7 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
       const float dot = sum[r] * a.scale;
       const uint64_t moved = __ballot(dot > m);
       const float m2 = fmaxf(m, dot);
-      const float e = __expf(fmaf(a.scale, sum[r], -m2));  // as attn_flash's scaling and difference are contracted
+      const float e = row_weight(a.scale, sum[r], m2);
       float alpha = 1.f;
       if (moved != 0) {
         alpha = __expf(m - m2);
@@ -824,7 +836,7 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
     load_v();
   }
 
-  // fold_lane_groups: the four chains of the wavefront, (0 1) (2 3) as the compiler contracts it there
+  // fold_lane_groups, as its first lane group adds: the four chains of the wavefront, (0 1) (2 3)
   float mg = fmaxf(m, __shfl_xor(m, 16, kWave));
   mg = fmaxf(mg, __shfl_xor(mg, 32, kWave));
   const float w = __expf(m - mg);
@@ -836,7 +848,7 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
   }
   if (lg == 0) {
     sm[li][wave] = mg;
-    sl[li][wave] = fmaf(lb[0], wb[0], __fmul_rn(lb[1], wb[1])) + fmaf(lb[2], wb[2], __fmul_rn(lb[3], wb[3]));
+    sl[li][wave] = fmaf(lb[0], wb[0], lb[1] * wb[1]) + fmaf(lb[2], wb[2], lb[3] * wb[3]);
   }
   float *dst = so + li * kStateStride + wave * HD + lg * 32;
 #pragma unroll
@@ -844,8 +856,7 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
     float o[8];
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
-      o[dt] = fmaf(acc[dt][v], wb[0], __fmul_rn(acc[dt][4 + v], wb[1])) +
-              fmaf(acc[dt][8 + v], wb[2], __fmul_rn(acc[dt][12 + v], wb[3]));
+      o[dt] = fmaf(acc[dt][v], wb[0], acc[dt][4 + v] * wb[1]) + fmaf(acc[dt][8 + v], wb[2], acc[dt][12 + v] * wb[3]);
     }
     *reinterpret_cast<float4 *>(dst + v * 8) = make_float4(o[0], o[1], o[2], o[3]);
     *reinterpret_cast<float4 *>(dst + v * 8 + 4) = make_float4(o[4], o[5], o[6], o[7]);
@@ -921,10 +932,10 @@ __global__ __launch_bounds__(INWG ? kWave * kMaxWgSplits : kWave) void attn_flas
           const int pd = low ? d + half : d - half;
           const float cd = bf16_to_f32(c[d]), sd = bf16_to_f32(s[d]);
           const float tq = bf16_to_f32(qh[d]), pq = bf16_to_f32(qh[pd]);
-          qf[i] = tq * cd + (low ? -pq : pq) * sd;
+          qf[i] = fmaf(tq, cd, (low ? -pq : pq) * sd);
           if (fuse) {
             const float tk = bf16_to_f32(ka[d]), pk = bf16_to_f32(ka[pd]);
-            kcur[i] = tk * cd + (low ? -pk : pk) * sd;
+            kcur[i] = fmaf(tk, cd, (low ? -pk : pk) * sd);
             vcur[i] = bf16_to_f32(va[d]);
             if (writer) {
               const size_t off = (static_cast<size_t>(pos) * a.n_kv + kv_head) * hd + d;
@@ -966,10 +977,10 @@ __global__ __launch_bounds__(INWG ? kWave * kMaxWgSplits : kWave) void attn_flas
     for (int i = 0; i < 4; ++i) {
       dot = fmaf(qf[i], kf[i], dot);
     }
-    dot = wave_sum(dot) * a.scale;
-    const float m2 = fmaxf(m, dot);
+    dot = wave_sum(dot);
+    const float m2 = fmaxf(m, dot * a.scale);
     const float alpha = __expf(m - m2);
-    const float e = __expf(dot - m2);
+    const float e = row_weight(a.scale, dot, m2);
     l = fmaf(l, alpha, e);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -1053,8 +1064,8 @@ __global__ __launch_bounds__(kWave) void rope_kv(uint16_t *__restrict__ q, uint1
     if (d < half) {
       const float t0 = bf16_to_f32(vec[d]);
       const float t1 = bf16_to_f32(vec[d + half]);
-      lo[i] = t0 * bf16_to_f32(c[d]) + (-t1) * bf16_to_f32(s[d]);
-      hi[i] = t1 * bf16_to_f32(c[d + half]) + t0 * bf16_to_f32(s[d + half]);
+      lo[i] = fmaf(t0, bf16_to_f32(c[d]), -t1 * bf16_to_f32(s[d]));
+      hi[i] = fmaf(t1, bf16_to_f32(c[d + half]), t0 * bf16_to_f32(s[d + half]));
     }
   }
   const size_t off = (static_cast<size_t>(pos) * n_kv + head) * hd;
