@@ -220,14 +220,20 @@ __device__ __forceinline__ void fold_lane_groups(float &m, float &l, float (&acc
       mg = fmaxf(mg, __shfl_xor(mg, off, kWave));
     }
     const float w = __expf(m - mg);
-    auto add_first = [&](float v) {
-      const float own = v * w, other = __shfl_xor(own, LPT, kWave);
-      return LPT < 32 ? fmaf(v, w, other) : own + other;
-    };
-    l = add_first(l);
+    const float l_own = l * w;
+    float own[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      acc[i] = add_first(acc[i]);
+      own[i] = acc[i] * w;
+    }
+    auto add_first = [&](float v, float product) {
+      const float other = __shfl_xor(product, LPT, kWave);
+      return LPT < 32 ? fmaf(v, w, other) : product + other;
+    };
+    l = add_first(l, l_own);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      acc[i] = add_first(acc[i], own[i]);
     }
 #pragma unroll
     for (int off = 2 * LPT; off < kWave; off <<= 1) {
@@ -428,11 +434,12 @@ __global__ __launch_bounds__(INWG ? kWave * WMAX : kWave) void attn_flash(const 
       for (int i = 0; i < 8; ++i) {
         dot = fmaf(qf[i], kf[i], dot);
       }
-      dot = group_sum<LPT>(dot);
+      const float sum = group_sum<LPT>(dot);
+      dot = sum * a.scale;
       if (live[u]) {
-        const float m2 = fmaxf(m, dot * a.scale);
+        const float m2 = fmaxf(m, dot);
         const float alpha = __expf(m - m2);
-        const float e = row_weight(a.scale, dot, m2);
+        const float e = row_weight(a.scale, sum, m2);
         l = fmaf(l, alpha, e);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -590,11 +597,12 @@ __global__ __launch_bounds__(kWave * kMaxGqaWaves) void attn_chunk_gqa(const Att
         for (int i = 0; i < 8; ++i) {
           dot = fmaf(qf[r][i], kf[i], dot);
         }
-        dot = group_sum<LPT>(dot);
+        const float sum = group_sum<LPT>(dot);
+        dot = sum * a.scale;
         if (live) {
-          const float m2 = fmaxf(m[r], dot * a.scale);
+          const float m2 = fmaxf(m[r], dot);
           const float alpha = __expf(m[r] - m2);
-          const float e = row_weight(a.scale, dot, m2);
+          const float e = row_weight(a.scale, sum, m2);
           l[r] = fmaf(l[r], alpha, e);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
