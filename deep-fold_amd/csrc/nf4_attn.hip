@@ -895,6 +895,37 @@ bool launch_chunk_gqa(const AttnArgs &a, int n_rep, int n_waves, int n_tok, hipS
   }
 }
 
+// Whether a chunk takes attn_chunk_mfma.  It walks a prefix in the same time for one query a tile and for sixteen,
+// on few workgroups; the vector forms (attn_chunk_gqa a token and KV head, attn_flash a token and query head where
+// no group form is built) fill the chip with shorter ones.  So the line is the workgroups a compute unit of the
+// vector form from which it is the slower one behind the shortest prefixes too (the host does not know the prefix;
+// just above a line the matrix form is up to 8 % slower behind none): vector and matrix form, us, behind 0, 300 and
+// 1791 rows, at a chunk just below each line and one just above:
+//   query heads      below                                        above
+//   1, 3, 7, 16, ..  28 on 4,  80 tokens 8.3/9.4 25/21 110/67     96 heads 32 on 32 10.7/10.0 33/22 144/68
+//   2                32 on 16, 96 tokens 8.7/10.0 27/22 113/67    100 tokens 10.0/10.0 29/22 129/67
+//   4                32 on 8,  64 tokens 7.4/8.3 21/21 82/66      72 tokens 8.8/9.2 26/21 110/67
+//   5                40 on 8,  32 tokens 6.8/7.1 18/20 68/66      33 tokens 7.5/7.2 23/20 95/66
+//   6, 8             --                                           48 on 8, 2 tokens 6.4/5.8 18/17 77/62
+// One query head a KV head of 8, 16 tokens behind 1000 rows: 18 us on the vector unit, 41 in a tile.
+// Byte offsets of 32 bits, rows left out by a score of -inf (scale > 0).
+bool chunk_on_matrix_cores(int n_tok, int n_q, int n_kv, int hd, int n_waves, float scale, int max_seq) {
+  if (n_tok < 2 || hd != 128 || n_waves != kMfmaWaves || !(scale > 0.f) ||
+      static_cast<int64_t>(max_seq) * n_kv * hd >= (int64_t{1} << 30)) {
+    return false;
+  }
+  const int n_rep = n_q / n_kv;
+  int per_cu = 10;
+  int64_t vector_wgs = static_cast<int64_t>(n_tok) * n_q;
+  if (n_rep == 2 || n_rep == 4 || n_rep == 5 || n_rep == 6 || n_rep == 8) {  // as launch_chunk_gqa
+    per_cu = n_rep == 2 ? 6 : (n_rep == 4 ? 2 : (n_rep == 5 ? 1 : 0));
+    vector_wgs = static_cast<int64_t>(n_tok) * n_kv;
+  }
+  const int64_t tiles = (static_cast<int64_t>(n_tok) * n_rep + kMfmaQueries - 1) / kMfmaQueries;
+  return vector_wgs > static_cast<int64_t>(per_cu) * device_cu_count() &&
+         tiles * n_kv <= INT32_MAX / (kWave * kMfmaWaves);
+}
+
 // Any hd <= 256: lane l owns dims l, l+64, l+128, l+192; one time step per
 // iteration.  Slow path for head sizes that are not 8 * 2^n.
 template <bool INWG>
@@ -1233,11 +1264,7 @@ int attn_common(const void *q, const void *k, const void *v, void *out, const vo
   bool shared = false;
   if (mode == 1 && n_tok > 1 && !rope && vec_ok && n_split <= kMaxGqaWaves) {
     const int n_rep = n_q / n_kv;
-    // the matrix cores' form from two tokens on: at 40 query heads on 8 with one tile a KV head (2 tokens behind
-    // 1000 rows) 39.7 us without, 38 to 40 with it, more of either in the comment at the kernel; it takes byte
-    // offsets of 32 bits and leaves rows out by a score of -inf, so scale > 0
-    if (hd == 128 && n_split == kMfmaWaves && scale > 0.f &&
-        static_cast<int64_t>(max_seq) * n_kv * hd < (int64_t{1} << 30)) {
+    if (chunk_on_matrix_cores(n_tok, n_q, n_kv, hd, n_split, scale, max_seq)) {
       const int64_t tiles = (static_cast<int64_t>(n_tok) * n_rep + kMfmaQueries - 1) / kMfmaQueries;
       attn_chunk_mfma<<<dim3(static_cast<unsigned>(tiles * n_kv)), dim3(kWave * kMfmaWaves), 0, st>>>(a);
       shared = true;
@@ -1295,6 +1322,14 @@ extern "C" int chr_dv2_attn_parts(const void *q, const void *k, const void *v,
                                   int32_t max_seq) {
   return attn_common(q, k, v, nullptr, valid_len, state, n_q, n_kv, hd, n_waves, scale, stream,
                      k_act, v_act, cos, sin, position, max_seq, 2, n_parts);
+}
+
+extern "C" int32_t chr_dv2_attn_chunk_form(int32_t n_tok, int32_t n_q, int32_t n_kv, int32_t hd, int32_t n_waves,
+                                           float scale, int32_t max_seq) {
+  if (n_tok < 1 || n_q < 1 || n_kv < 1 || n_q % n_kv != 0) {
+    return -3;
+  }
+  return chunk_on_matrix_cores(n_tok, n_q, n_kv, hd, n_waves, scale, max_seq) ? 1 : 0;
 }
 
 extern "C" int chr_dv2_attn_chunk(const void *q, const void *k, const void *v, void *out,
