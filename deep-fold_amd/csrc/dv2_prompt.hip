@@ -131,13 +131,13 @@ __global__ __launch_bounds__(kPromptThreads) void prompt_gemm(const PromptArgs a
     sp = base + static_cast<size_t>(row) * groups + (tid & 1) * 2;
   }
   const bool odd = (lane & 1) != 0;
-  const char *xp = reinterpret_cast<const char *>(a.x + static_cast<size_t>(tok0) * a.K);
-  const uint32_t x_lane = (static_cast<uint32_t>(wave * 8 + (lane >> 3)) * a.K + ((lane & 7) ^ (lane >> 3)) * 8) * 2;
+  const uint16_t *xp =
+      a.x + static_cast<size_t>(tok0 + wave * 8 + (lane >> 3)) * a.K + ((lane & 7) ^ (lane >> 3)) * 8;
 
   auto load_x = [&](int c, int buf) {
 #pragma unroll
     for (int p = 0; p < 4; ++p) {  // group p of the chunk, tokens 8 wave .. + 8
-      load_to_lds16(reinterpret_cast<const uint16_t *>(xp + static_cast<size_t>(c) * (kChunk * 2) + x_lane + p * (kGroup * 2)),
+      load_to_lds16(xp + c * kChunk + p * kGroup,
                     static_cast<uint32_t>(kXAddr + buf * kXStage + p * (kWindow * 128) + wave * 1024));
     }
   };
@@ -651,8 +651,7 @@ int prompt_args(const chr_nf4_dev_t *w, int32_t n_mats, bool pair, int32_t N, Pr
     rows += w[i].M;
   }
   a.split_chunks = window64_chunks(w, n_mats);
-  constexpr int kMostK = 1 << 24;  // a workgroup's rows of x lie within 32-bit byte offsets
-  if (a.split_chunks < 1 || w[0].K > kMostK || w[0].K % kChunk != 0 || rows > INT32_MAX / 2 || rows % 4 != 0 || w[0].M % 4 != 0) {
+  if (a.split_chunks < 1 || w[0].K % kChunk != 0 || rows > INT32_MAX / 2 || rows % 4 != 0 || w[0].M % 4 != 0) {
     return -3;
   }
   for (int i = n_mats; i <= kPromptMats; ++i) {
