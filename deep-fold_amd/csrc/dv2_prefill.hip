@@ -22,7 +22,7 @@ constexpr int kMaxCols = 64;
 //                  (chr_dv2_gemm_add_sq), and only those are added.  N divides 1024 then;
 //   chains != nullptr (not VEC, N > 16): cols_chains left the sums a thread's rows have here, one launch
 //                  for all workgroups (their additions, repeated by 64 workgroups, were the launch's time:
-//                  5120 rows of 17 to 31 columns 13.9 us, of 33 to 63 columns 25; 8.6 and 13 so, in two).
+//                  5120 rows of 17 to 31 columns 13.7 us, of 33 to 63 columns 24.6; 8.7 and 13.1 so, in two).
 //
 // Thread t owns column t % CP of rows t / CP, t / CP + 1024 / CP, ..; CP is N rounded up to a
 // power of two, threads whose column is >= N idle.  VEC: N is 8, 16, 32 or 64 and rows are 16-byte
@@ -345,6 +345,20 @@ namespace {
 
 constexpr int kChainFloats = 32 * kMaxCols;
 
+int padded_cols(int N) {
+  int cp = 1;
+  while (cp < N) {
+    cp <<= 1;
+  }
+  return cp;
+}
+
+// Whether rms_cols<false> leaves its sums to cols_chains.  Called one by one without a graph two launches and their
+// workspace take the host 10.7 us, one 6.8, so the line is where one launch takes the device that long: 24 columns
+// of 3072 rows 9.2 us, of 4000 11.2, 63 of 1536 rows 9.6, of 2048 11.6.  From a graph, one and two launches: 24
+// columns of 4096 rows 11.4 and 7.7, 63 of 2048 11.8 and 8.1 (and even at 1536 and 1024 rows, 6.2 and 7 us).
+bool chains_apart(int rows, int N) { return N > 16 && rows >= (N <= 32 ? 4096 : 2048); }
+
 int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps,
                     const float *sq, int32_t sq_blocks, void *stream, float *chains = nullptr) {
   if (x == nullptr || w == nullptr || y == nullptr) {
@@ -360,10 +374,7 @@ int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t
     return -2;
   }
   const bool vec = (N == 8 || N == 16 || N == 32 || N == 64) && aligned16(x) && aligned16(y);
-  int cp = 1;
-  while (cp < N) {
-    cp <<= 1;
-  }
+  const int cp = padded_cols(N);
   // enough workgroups to spread the write-out, few enough that the redundant read stays cheap
   const int wgs = max(1, min(64, rows / 64));
   const int rows_per_wg = (rows + wgs - 1) / wgs;
@@ -374,10 +385,8 @@ int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t
         static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w),
         static_cast<uint16_t *>(y), rows, N, cp, eps, rows_per_wg, sq, sq_blocks, nullptr);
   } else {
-    // from a thousand rows on the second launch costs less than what it saves (1000 rows of 17 columns 5.3 us
-    // in one launch, of 33 columns 7.7)
     const int steps = kColsBlock / cp;
-    if (sq != nullptr || cp < 32 || rows < 1024) {
+    if (sq != nullptr || !chains_apart(rows, N)) {
       chains = nullptr;
     }
     if (chains != nullptr) {
@@ -400,6 +409,11 @@ extern "C" int chr_dv2_rms_cols(const void *x, const void *w, void *y, int32_t r
 }
 
 extern "C" int32_t chr_dv2_rms_cols_ws_floats(void) { return kChainFloats; }
+
+extern "C" int32_t chr_dv2_rms_cols_ws_for(int32_t rows, int32_t N) {
+  // (8, 16, 32 and 64 columns are whole vectors)
+  return N >= 1 && N <= kMaxCols && padded_cols(N) != N && chains_apart(rows, N) ? kChainFloats : 0;
+}
 
 extern "C" int chr_dv2_rms_cols_ws(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps, float *ws,
                                    void *stream) {

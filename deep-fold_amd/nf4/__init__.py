@@ -15,6 +15,7 @@ There is no CPU fallback: a missing library or a non-GPU tensor raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 
 import torch
@@ -169,6 +170,7 @@ EXPORTS = (
     ("chr_dv2_gemv_attn", ctypes.c_int, [_DP, _P, _I, _I, _I, _P, _P, _P]),
     ("chr_dv2_rms_cols", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P]),
     ("chr_dv2_rms_cols_ws_floats", ctypes.c_int32, []),
+    ("chr_dv2_rms_cols_ws_for", ctypes.c_int32, [_I, _I]),
     ("chr_dv2_rms_cols_ws", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P, _P]),
     ("chr_dv2_rope_kv_cols", ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     ("chr_dv2_attn_chunk", ctypes.c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I]),
@@ -991,6 +993,11 @@ def _bf16_cuda(t: torch.Tensor, what: str) -> None:
           f"{what} must be a contiguous CUDA bfloat16 tensor")
 
 
+@functools.lru_cache(maxsize=4096)
+def _rms_cols_ws_for(rows: int, n: int) -> int:
+    return int(_load_ext().chr_dv2_rms_cols_ws_for(rows, n))
+
+
 def dv2_rms_cols(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor | None = None,
                  colsq: torch.Tensor | None = None) -> torch.Tensor:
     """RMSNorm of every column of feature-major ``x [rows, N]`` (N <= 64).  ``colsq``: the
@@ -1011,13 +1018,13 @@ def dv2_rms_cols(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor
                                              int(x.size(1)), float(eps), colsq.data_ptr(), blocks, _stream())
         _check_rc("chr_dv2_rms_cols_sq", rc)
         return out
-    lib, n = _load_ext(), int(x.size(1))
-    if n > 16 and n not in (32, 64):
-        ws = torch.empty(int(lib.chr_dv2_rms_cols_ws_floats()), dtype=torch.float32, device=x.device)
-        rc = lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), out.data_ptr(), int(x.size(0)), n, float(eps),
-                                     ws.data_ptr(), _stream())
+    lib, rows, n = _load_ext(), int(x.size(0)), int(x.size(1))
+    if floats := _rms_cols_ws_for(rows, n):
+        ws = torch.empty(floats, dtype=torch.float32, device=x.device)
+        rc = lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, n, float(eps), ws.data_ptr(),
+                                     _stream())
     else:
-        rc = lib.chr_dv2_rms_cols(x.data_ptr(), w.data_ptr(), out.data_ptr(), int(x.size(0)), n, float(eps), _stream())
+        rc = lib.chr_dv2_rms_cols(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, n, float(eps), _stream())
     _check_rc("chr_dv2_rms_cols", rc)
     return out
 
