@@ -2050,8 +2050,9 @@ int launch_pairs(StreamArgs &a, int m_pairs, hipStream_t st) {
 }  // namespace
 
 // Shared with the GEMM entry points, which route N == 1 here.  `rounded`: add is a bias that meets the
-// product's bf16.  The plain kernel adds it (2048 x 2048 through the linear seat 22.3 -> 17.0 us); the staged
-// ones, whose launches are that much longer, leave it to a launch behind them.
+// product's bf16.  The plain kernel adds it (2048 x 2048 through the linear seat, against torch's addition behind
+// the call: 17.4 -> 13.9 us a call, 5.0 -> 3.5 from a graph).  The staged ones, which also serve every ragged K,
+// leave it to a launch behind them (300 x 1000 17.8 -> 17.0 and 6.1 -> 5.6, 5120 x 5120 17.7 -> 16.9 and 8.3 -> 7.6).
 int gemv_entry(const chr_nf4_dev_t *w, const void *x, void *y, void *stream, const void *add,
                const void *rms_w, float rms_eps, const float *sq_in, float *sq_out, bool rounded) {
   if (w == nullptr || x == nullptr || y == nullptr) {

@@ -143,7 +143,8 @@ int chr_nf4_gemv(const chr_nf4_dev_t *w, const void *x, void *y, void *stream,
                  const void *add, const void *rms_w, float rms_eps);
 
 /* y = bf16(W x) + bias[M], the sum rounded to bf16 once more: what an addition behind chr_nf4_gemv gives
- * (gpu/host/linear.py:62-63), in its launch where that is below 16M codes, in a second one otherwise.
+ * (gpu/host/linear.py:62-63).  In its launch where K is a multiple of 64 and M * K below 16M; in a second
+ * launch of the same call for larger matrices and, whatever their size, for a ragged K.
  * -1 without a bias; otherwise chr_nf4_gemv's return codes. */
 int chr_nf4_gemv_bias(const chr_nf4_dev_t *w, const void *x, void *y, const void *bias, void *stream);
 
