@@ -353,11 +353,14 @@ int padded_cols(int N) {
   return cp;
 }
 
-// Whether rms_cols<false> leaves its sums to cols_chains.  Called one by one without a graph two launches and their
-// workspace take the host 10.7 us, one 6.8, so the line is where one launch takes the device that long: 24 columns
-// of 3072 rows 9.2 us, of 4000 11.2, 63 of 1536 rows 9.6, of 2048 11.6.  From a graph, one and two launches: 24
-// columns of 4096 rows 11.4 and 7.7, 63 of 2048 11.8 and 8.1 (and even at 1536 and 1024 rows, 6.2 and 7 us).
-bool chains_apart(int rows, int N) { return N > 16 && rows >= (N <= 32 ? 4096 : 2048); }
+// Whether rms_cols<false> leaves its sums to cols_chains.  Recorded into a graph, one and two launches, us: 24
+// columns of 1280 rows 5.7 / 6.1, 1536 6.2 / 6.1, 2048 7.2 / 6.1; 63 of 1000 rows 7.7 / 7.9, 1024 7.7 / 6.5, 2048
+// 11.8 / 8.1 (inside a model the gap is 1 us wider: a 3B turn of 24 tokens, 72 such norms, 2900 / 2738).  Launched one by one, two launches and their workspace take the host 10.7, one 6.8, so there the line is
+// where the device takes that long: 24 columns of 3072 rows 9.2, of 4000 11.2, 63 of 1536 9.6, of 2048 11.6 (asking
+// whether a launch is recorded takes the host 0.4, and is left out where the answer makes no difference).
+bool chains_apart(int rows, int N, bool recorded) {
+  return N > 16 && rows >= (N <= 32 ? (recorded ? 1536 : 4096) : (recorded ? 1024 : 2048));
+}
 
 int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps,
                     const float *sq, int32_t sq_blocks, void *stream, float *chains = nullptr) {
@@ -386,7 +389,7 @@ int rms_cols_launch(const void *x, const void *w, void *y, int32_t rows, int32_t
         static_cast<uint16_t *>(y), rows, N, cp, eps, rows_per_wg, sq, sq_blocks, nullptr);
   } else {
     const int steps = kColsBlock / cp;
-    if (sq != nullptr || !chains_apart(rows, N)) {
+    if (sq != nullptr || !chains_apart(rows, N, true)) {
       chains = nullptr;
     }
     if (chains != nullptr) {
@@ -410,9 +413,9 @@ extern "C" int chr_dv2_rms_cols(const void *x, const void *w, void *y, int32_t r
 
 extern "C" int32_t chr_dv2_rms_cols_ws_floats(void) { return kChainFloats; }
 
-extern "C" int32_t chr_dv2_rms_cols_ws_for(int32_t rows, int32_t N) {
+extern "C" int32_t chr_dv2_rms_cols_ws_for(int32_t rows, int32_t N, int32_t recorded) {
   // (8, 16, 32 and 64 columns are whole vectors)
-  return N >= 1 && N <= kMaxCols && padded_cols(N) != N && chains_apart(rows, N) ? kChainFloats : 0;
+  return N >= 1 && N <= kMaxCols && padded_cols(N) != N && chains_apart(rows, N, recorded != 0) ? kChainFloats : 0;
 }
 
 extern "C" int chr_dv2_rms_cols_ws(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps, float *ws,

@@ -170,7 +170,7 @@ EXPORTS = (
     ("chr_dv2_gemv_attn", ctypes.c_int, [_DP, _P, _I, _I, _I, _P, _P, _P]),
     ("chr_dv2_rms_cols", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P]),
     ("chr_dv2_rms_cols_ws_floats", ctypes.c_int32, []),
-    ("chr_dv2_rms_cols_ws_for", ctypes.c_int32, [_I, _I]),
+    ("chr_dv2_rms_cols_ws_for", ctypes.c_int32, [_I, _I, _I]),
     ("chr_dv2_rms_cols_ws", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P, _P]),
     ("chr_dv2_rope_kv_cols", ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     ("chr_dv2_attn_chunk", ctypes.c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I]),
@@ -994,8 +994,9 @@ def _bf16_cuda(t: torch.Tensor, what: str) -> None:
 
 
 @functools.lru_cache(maxsize=4096)
-def _rms_cols_ws_for(rows: int, n: int) -> int:
-    return int(_load_ext().chr_dv2_rms_cols_ws_for(rows, n))
+def _rms_cols_ws_for(rows: int, n: int) -> tuple[int, int]:
+    """Workspace worth its second launch: launched, and recorded into a graph."""
+    return tuple(int(_load_ext().chr_dv2_rms_cols_ws_for(rows, n, recorded)) for recorded in (0, 1))
 
 
 def dv2_rms_cols(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor | None = None,
@@ -1019,7 +1020,10 @@ def dv2_rms_cols(x: torch.Tensor, w: torch.Tensor, eps: float, out: torch.Tensor
         _check_rc("chr_dv2_rms_cols_sq", rc)
         return out
     lib, rows, n = _load_ext(), int(x.size(0)), int(x.size(1))
-    if floats := _rms_cols_ws_for(rows, n):
+    floats, recorded = _rms_cols_ws_for(rows, n)
+    if recorded > floats and torch.cuda.is_current_stream_capturing():
+        floats = recorded
+    if floats:
         ws = torch.empty(floats, dtype=torch.float32, device=x.device)
         rc = lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, n, float(eps), ws.data_ptr(),
                                      _stream())

@@ -316,9 +316,10 @@ int chr_dv2_rms_cols(const void *x, const void *w, void *y, int32_t rows, int32_
 
 /* chr_dv2_rms_cols, the same bits, with chr_dv2_rms_cols_ws_floats() fp32 elements of workspace: a tall tile
  * whose columns are no whole vectors has its squares added once, in a launch of its own.  -1 without ws.
- * chr_dv2_rms_cols_ws_for: that number where such a tile is tall enough to be worth it, else 0. */
+ * chr_dv2_rms_cols_ws_for: that number where the tile is tall enough to be worth it, else 0; recorded: of a launch
+ * recorded into a graph, where the second launch costs the host nothing. */
 int32_t chr_dv2_rms_cols_ws_floats(void);
-int32_t chr_dv2_rms_cols_ws_for(int32_t rows, int32_t N);
+int32_t chr_dv2_rms_cols_ws_for(int32_t rows, int32_t N, int32_t recorded);
 int chr_dv2_rms_cols_ws(const void *x, const void *w, void *y, int32_t rows, int32_t N, float eps, float *ws,
                         void *stream);
 
