@@ -354,10 +354,11 @@ int padded_cols(int N) {
 }
 
 // Whether rms_cols<false> leaves its sums to cols_chains.  Recorded into a graph, one and two launches, us: 24
-// columns of 1280 rows 5.7 / 6.1, 1536 6.2 / 6.1, 2048 7.2 / 6.1; 63 of 1000 rows 7.7 / 7.9, 1024 7.7 / 6.5, 2048
-// 11.8 / 8.1 (inside a model the gap is 1 us wider: a 3B turn of 24 tokens, 72 such norms, 2900 / 2738).  Launched one by one, two launches and their workspace take the host 10.7, one 6.8, so there the line is
-// where the device takes that long: 24 columns of 3072 rows 9.2, of 4000 11.2, 63 of 1536 9.6, of 2048 11.6 (asking
-// whether a launch is recorded takes the host 0.4, and is left out where the answer makes no difference).
+// columns of 1280 rows 5.7 / 6.1, 1536 6.2 / 6.1, 2048 7.2 / 6.1; 63 of 1024 rows 7.7 / 6.5, 2048 11.8 / 8.1
+// (inside a model the gap is 1 us wider: a 3B turn of 24 tokens, 72 such norms, 2900 / 2738).  Launched one by one,
+// two launches and their workspace take the host 10.7, one 6.8, so there the line is where the device takes that
+// long: 24 columns of 3072 rows 9.2, of 4000 11.2, 63 of 1536 9.6, of 2048 11.6 (asking whether a launch is recorded
+// takes the host 0.4, and is left out where the answer makes no difference).
 bool chains_apart(int rows, int N, bool recorded) {
   return N > 16 && rows >= (N <= 32 ? (recorded ? 1536 : 4096) : (recorded ? 1024 : 2048));
 }

@@ -516,10 +516,27 @@ __global__ __launch_bounds__(INWG ? kWave * WMAX : kWave) void attn_flash(const 
 // dotted with all REP queries, so L2 traffic (what bounds a chunk: n_q * N workgroups re-read
 // the prefix) drops by REP.  Rows, update order, lane-group fold and LDS merge are those of
 // attn_flash<LPT, true> for each head, so a head's output is bit for bit the same.
+//
+// EITHER (128 dims, four wavefronts): a chunk whose better form hangs on its prefix, which only the device knows.
+// Where token 0 sees matrix_from rows or more the first workgroups are chunk_mfma's tiles and the others end.
 constexpr int kMaxGqaWaves = 8;
+constexpr int kMfmaWaves = 4;
+constexpr int kMfmaQueries = 16;
+__device__ void chunk_mfma(const AttnArgs &a, int block, int blocks);
 
-template <int LPT, int REP>
-__global__ __launch_bounds__(kWave * kMaxGqaWaves) void attn_chunk_gqa(const AttnArgs a) {
+template <int LPT, int REP, bool EITHER = false>
+__global__ __launch_bounds__(kWave *(EITHER ? kMfmaWaves : kMaxGqaWaves), 2) void attn_chunk_gqa(const AttnArgs a,
+                                                                                                 int matrix_from) {
+  if constexpr (EITHER) {
+    if (*a.valid_len >= matrix_from) {
+      const int block = static_cast<int>(blockIdx.x) + a.n_kv * static_cast<int>(blockIdx.y);
+      const int blocks = (a.n_tok * REP + kMfmaQueries - 1) / kMfmaQueries * a.n_kv;
+      if (block < blocks) {
+        chunk_mfma(a, block, blocks);
+      }
+      return;
+    }
+  }
   constexpr int TPW = kWave / LPT;
   constexpr int UNR = 2;  // (4: the same within 0.5% on a prefill, 8: 1 to 5% slower)
   constexpr int HD = 8 * LPT;
@@ -663,10 +680,9 @@ __global__ __launch_bounds__(kWave * kMaxGqaWaves) void attn_chunk_gqa(const Att
 // acc * alpha is left out where no query of a chain moves its maximum (alpha is 1: exact).  Votes by 4 queries
 // instead of 16 (the sums transposed) save two thirds of these products and lose it to the branches (520 us).
 typedef __attribute__((ext_vector_type(16))) float F32x16;
-constexpr int kMfmaWaves = 4;
-constexpr int kMfmaQueries = 16;
 
-__global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const AttnArgs a) {
+// Workgroup `block` of `blocks`.
+__device__ __forceinline__ void chunk_mfma(const AttnArgs &a, int block, int blocks) {
   constexpr int HD = 128;
   constexpr int kTile = 64;                              // rows of a step of the workgroup
   constexpr int kStateStride = kMfmaWaves * HD + 4;      // floats of a query's states: the pad spreads the banks
@@ -679,8 +695,8 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
   const int li = lane & 15, lg = lane >> 4;
   const int rep = a.n_rep;
   // the longest tiles first; neighbouring workgroups take different KV heads, so a KV head stays on a die
-  const int kv_head = static_cast<int>(blockIdx.x) % a.n_kv;
-  const int q0 = (static_cast<int>(gridDim.x) / a.n_kv - 1 - static_cast<int>(blockIdx.x) / a.n_kv) * kMfmaQueries;
+  const int kv_head = block % a.n_kv;
+  const int q0 = (blocks / a.n_kv - 1 - block / a.n_kv) * kMfmaQueries;
   const int n_queries = a.n_tok * rep;
   const int first_len = *a.valid_len;
   const int tok = min(q0 + li, n_queries - 1) / rep;
@@ -881,49 +897,60 @@ __global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const At
   }
 }
 
+__global__ __launch_bounds__(kWave *kMfmaWaves, 2) void attn_chunk_mfma(const AttnArgs a) {
+  chunk_mfma(a, static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x));
+}
+
 template <int LPT>
 bool launch_chunk_gqa(const AttnArgs &a, int n_rep, int n_waves, int n_tok, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(a.n_kv), static_cast<unsigned>(n_tok));
   const dim3 block(static_cast<unsigned>(kWave * n_waves));
   switch (n_rep) {
-    case 2: attn_chunk_gqa<LPT, 2><<<grid, block, 0, st>>>(a); return true;
-    case 4: attn_chunk_gqa<LPT, 4><<<grid, block, 0, st>>>(a); return true;
-    case 5: attn_chunk_gqa<LPT, 5><<<grid, block, 0, st>>>(a); return true;
-    case 6: attn_chunk_gqa<LPT, 6><<<grid, block, 0, st>>>(a); return true;
-    case 8: attn_chunk_gqa<LPT, 8><<<grid, block, 0, st>>>(a); return true;
+    case 2: attn_chunk_gqa<LPT, 2><<<grid, block, 0, st>>>(a, 0); return true;
+    case 4: attn_chunk_gqa<LPT, 4><<<grid, block, 0, st>>>(a, 0); return true;
+    case 5: attn_chunk_gqa<LPT, 5><<<grid, block, 0, st>>>(a, 0); return true;
+    case 6: attn_chunk_gqa<LPT, 6><<<grid, block, 0, st>>>(a, 0); return true;
+    case 8: attn_chunk_gqa<LPT, 8><<<grid, block, 0, st>>>(a, 0); return true;
     default: return false;
   }
 }
 
-// Whether a chunk takes attn_chunk_mfma.  It walks a prefix in the same time for one query a tile and for sixteen,
-// on few workgroups; the vector forms (attn_chunk_gqa a token and KV head, attn_flash a token and query head where
-// no group form is built) fill the chip with shorter ones.  So the line is the workgroups a compute unit of the
-// vector form from which it is the slower one behind the shortest prefixes too (the host does not know the prefix;
-// just above a line the matrix form is up to 8 % slower behind none): vector and matrix form, us, behind 0, 300 and
-// 1791 rows, at a chunk just below each line and one just above:
+// Rows token 0 of a chunk sees from which its attention is faster on the matrix cores (0: however few, INT32_MAX:
+// never).  A tile walks a prefix in the same time for one query and for sixteen, and the tiles are few; the vector
+// forms (attn_chunk_gqa a token and KV head, attn_flash a token and query head where no group form is built) fill the
+// chip with shorter workgroups.  So the lines are workgroups a compute unit of the vector form.  The host does not
+// know the prefix: above a line the matrix form wins behind short ones too (it is up to 8 % slower behind none), below
+// it the vector form is taken or, where two workgroups a compute unit are all there are, the device chooses
+// (attn_chunk_gqa<.., true>: more of them would miss the vector kernel's occupancy).  Vector and matrix form, us, behind
+// 0, 300 and 1791 rows:
 //   query heads      below                                        above
 //   1, 3, 7, 16, ..  28 on 4,  80 tokens 8.3/9.4 25/21 110/67     96 heads 32 on 32 10.7/10.0 33/22 144/68
 //   2                32 on 16, 96 tokens 8.7/10.0 27/22 113/67    100 tokens 10.0/10.0 29/22 129/67
-//   4                32 on 8,  64 tokens 7.4/8.3 21/21 82/66      72 tokens 8.8/9.2 26/21 110/67
-//   5                40 on 8,  32 tokens 6.8/7.1 18/20 68/66      33 tokens 7.5/7.2 23/20 95/66
-//   6, 8             --                                           48 on 8, 2 tokens 6.4/5.8 18/17 77/62
+//   4                32 on 8,  32 tokens 5.7/7.2 15/20 57/65      72 tokens 8.8/9.2 26/21 110/67
+//      between       64 tokens 7.4/8.3 21/21 82/66: from 350 rows
+//   5                                                             40 on 8, 33 tokens 7.5/7.2 23/20 95/66
+//      below         32 tokens 6.8/7.1 18/20 68/66: from 1200 rows
+//   6, 8                                                          48 on 8, 2 tokens 6.4/5.8 18/17 77/62
 // One query head a KV head of 8, 16 tokens behind 1000 rows: 18 us on the vector unit, 41 in a tile.
 // Byte offsets of 32 bits, rows left out by a score of -inf (scale > 0).
-bool chunk_on_matrix_cores(int n_tok, int n_q, int n_kv, int hd, int n_waves, float scale, int max_seq) {
-  if (n_tok < 2 || hd != 128 || n_waves != kMfmaWaves || !(scale > 0.f) ||
-      static_cast<int64_t>(max_seq) * n_kv * hd >= (int64_t{1} << 30)) {
-    return false;
-  }
+int chunk_matrix_from(int n_tok, int n_q, int n_kv, int hd, int n_waves, float scale, int max_seq) {
+  constexpr int kNever = INT32_MAX;
   const int n_rep = n_q / n_kv;
-  int per_cu = 10;
-  int64_t vector_wgs = static_cast<int64_t>(n_tok) * n_q;
-  if (n_rep == 2 || n_rep == 4 || n_rep == 5 || n_rep == 6 || n_rep == 8) {  // as launch_chunk_gqa
-    per_cu = n_rep == 2 ? 6 : (n_rep == 4 ? 2 : (n_rep == 5 ? 1 : 0));
-    vector_wgs = static_cast<int64_t>(n_tok) * n_kv;
-  }
   const int64_t tiles = (static_cast<int64_t>(n_tok) * n_rep + kMfmaQueries - 1) / kMfmaQueries;
-  return vector_wgs > static_cast<int64_t>(per_cu) * device_cu_count() &&
-         tiles * n_kv <= INT32_MAX / (kWave * kMfmaWaves);
+  if (n_tok < 2 || hd != 128 || n_waves != kMfmaWaves || !(scale > 0.f) ||
+      static_cast<int64_t>(max_seq) * n_kv * hd >= (int64_t{1} << 30) ||
+      tiles * n_kv > INT32_MAX / (kWave * kMfmaWaves)) {
+    return kNever;
+  }
+  const int64_t cus = device_cu_count(), shared = static_cast<int64_t>(n_tok) * n_kv;
+  switch (n_rep) {  // the group forms of launch_chunk_gqa
+    case 2: return shared > 6 * cus ? 0 : kNever;
+    case 4: return shared > 2 * cus ? 0 : (shared > cus ? 350 : kNever);
+    case 5: return shared > cus ? 0 : 1200;
+    case 6:
+    case 8: return 0;
+    default: return static_cast<int64_t>(n_tok) * n_q > 10 * cus ? 0 : kNever;
+  }
 }
 
 // Any hd <= 256: lane l owns dims l, l+64, l+128, l+192; one time step per
@@ -1264,9 +1291,18 @@ int attn_common(const void *q, const void *k, const void *v, void *out, const vo
   bool shared = false;
   if (mode == 1 && n_tok > 1 && !rope && vec_ok && n_split <= kMaxGqaWaves) {
     const int n_rep = n_q / n_kv;
-    if (chunk_on_matrix_cores(n_tok, n_q, n_kv, hd, n_split, scale, max_seq)) {
+    const int matrix_from = chunk_matrix_from(n_tok, n_q, n_kv, hd, n_split, scale, max_seq);
+    if (matrix_from == 0) {
       const int64_t tiles = (static_cast<int64_t>(n_tok) * n_rep + kMfmaQueries - 1) / kMfmaQueries;
       attn_chunk_mfma<<<dim3(static_cast<unsigned>(tiles * n_kv)), dim3(kWave * kMfmaWaves), 0, st>>>(a);
+      shared = true;
+    } else if (matrix_from != INT32_MAX) {
+      const dim3 grid(static_cast<unsigned>(n_kv), static_cast<unsigned>(n_tok)), block(kWave * kMfmaWaves);
+      if (n_rep == 4) {
+        attn_chunk_gqa<16, 4, true><<<grid, block, 0, st>>>(a, matrix_from);
+      } else {
+        attn_chunk_gqa<16, 5, true><<<grid, block, 0, st>>>(a, matrix_from);
+      }
       shared = true;
     } else if (hd == 128) {
       shared = launch_chunk_gqa<16>(a, n_rep, n_split, n_tok, st);
@@ -1324,12 +1360,12 @@ extern "C" int chr_dv2_attn_parts(const void *q, const void *k, const void *v,
                      k_act, v_act, cos, sin, position, max_seq, 2, n_parts);
 }
 
-extern "C" int32_t chr_dv2_attn_chunk_form(int32_t n_tok, int32_t n_q, int32_t n_kv, int32_t hd, int32_t n_waves,
-                                           float scale, int32_t max_seq) {
+extern "C" int32_t chr_dv2_attn_chunk_matrix_from(int32_t n_tok, int32_t n_q, int32_t n_kv, int32_t hd, int32_t n_waves,
+                                                  float scale, int32_t max_seq) {
   if (n_tok < 1 || n_q < 1 || n_kv < 1 || n_q % n_kv != 0) {
     return -3;
   }
-  return chunk_on_matrix_cores(n_tok, n_q, n_kv, hd, n_waves, scale, max_seq) ? 1 : 0;
+  return chunk_matrix_from(n_tok, n_q, n_kv, hd, n_waves, scale, max_seq);
 }
 
 extern "C" int chr_dv2_attn_chunk(const void *q, const void *k, const void *v, void *out,

@@ -174,7 +174,7 @@ EXPORTS = (
     ("chr_dv2_rms_cols_ws", ctypes.c_int, [_P, _P, _P, _I, _I, _F, _P, _P]),
     ("chr_dv2_rope_kv_cols", ctypes.c_int, [_P, _P, _P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P]),
     ("chr_dv2_attn_chunk", ctypes.c_int, [_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _F, _P, _I, _I, _I]),
-    ("chr_dv2_attn_chunk_form", ctypes.c_int32, [_I, _I, _I, _I, _I, _F, _I]),
+    ("chr_dv2_attn_chunk_matrix_from", ctypes.c_int32, [_I, _I, _I, _I, _I, _F, _I]),
     ("chr_dv2_swiglu_elems", ctypes.c_int, [_P, _P, _P, ctypes.c_int64, _P]),
     ("chr_dv2_add_cols", ctypes.c_int, [_P, _P, _P, _I, _I, _P]),
     ("chr_dv2_gemm_add", ctypes.c_int, [_DP, _P, _P, _I, _P, ctypes.c_int64, _P, _P, _P]),

@@ -347,10 +347,10 @@ int chr_dv2_attn_chunk(const void *q, const void *k, const void *v, void *out,
                        const void *first_len, int32_t n_tok, int32_t n_q, int32_t n_kv,
                        int32_t hd, int32_t n_waves, float scale, void *stream, int32_t max_seq,
                        int32_t out_tok_stride, int32_t out_dim_stride);
-/* 1 where that launch takes the fp32 matrix instructions (16-byte aligned operands), 0 where the vector unit;
- * the results are the same.  -3: bad arguments.  No launch. */
-int32_t chr_dv2_attn_chunk_form(int32_t n_tok, int32_t n_q, int32_t n_kv, int32_t hd, int32_t n_waves, float scale,
-                                int32_t max_seq);
+/* *first_len from which that launch takes the fp32 matrix instructions (16-byte aligned operands) instead of the
+ * vector unit: 0 always, INT32_MAX never.  The results are the same.  -3: bad arguments.  No launch. */
+int32_t chr_dv2_attn_chunk_matrix_from(int32_t n_tok, int32_t n_q, int32_t n_kv, int32_t hd, int32_t n_waves,
+                                       float scale, int32_t max_seq);
 
 /* y = silu(gate) * up over `count` bf16 elements, the activation rounded to bf16 before the
  * product as torch's two ops round (gpu/decodev2/ops.py:23-24). */
