@@ -919,19 +919,22 @@ bool launch_chunk_gqa(const AttnArgs &a, int n_rep, int n_waves, int n_tok, hipS
 // never).  A tile walks a prefix in the same time for one query and for sixteen, and the tiles are few; the vector
 // forms (attn_chunk_gqa a token and KV head, attn_flash a token and query head where no group form is built) fill the
 // chip with shorter workgroups.  So the lines are workgroups a compute unit of the vector form.  The host does not
-// know the prefix: above a line the matrix form wins behind short ones too (it is up to 8 % slower behind none), below
-// it the vector form is taken or, where two workgroups a compute unit are all there are, the device chooses
-// (attn_chunk_gqa<.., true>: more of them would miss the vector kernel's occupancy).  Vector and matrix form, us, behind
-// 0, 300 and 1791 rows:
-//   query heads      below                                        above
-//   1, 3, 7, 16, ..  28 on 4,  80 tokens 8.3/9.4 25/21 110/67     96 heads 32 on 32 10.7/10.0 33/22 144/68
-//   2                32 on 16, 96 tokens 8.7/10.0 27/22 113/67    100 tokens 10.0/10.0 29/22 129/67
-//   4                32 on 8,  32 tokens 5.7/7.2 15/20 57/65      72 tokens 8.8/9.2 26/21 110/67
-//      between       64 tokens 7.4/8.3 21/21 82/66: from 350 rows
-//   5                                                             40 on 8, 33 tokens 7.5/7.2 23/20 95/66
-//      below         32 tokens 6.8/7.1 18/20 68/66: from 1200 rows
-//   6, 8                                                          48 on 8, 2 tokens 6.4/5.8 18/17 77/62
-// One query head a KV head of 8, 16 tokens behind 1000 rows: 18 us on the vector unit, 41 in a tile.
+// know the prefix: the vector form is taken where it wins behind all of them.  Above, it would win by up to 2 us behind
+// short ones and lose by up to 50 behind long ones, and the tiles are taken; where two workgroups a compute unit are all
+// there are, the device chooses (attn_chunk_gqa<.., true>: more of them would miss the vector kernel's occupancy).
+// Vector and matrix form, us, behind 0, 300, 1000 and 1791 rows:
+//   query heads      at the line                                     above
+//   1, 3, 7, 16, ..  32 on 32, 40 tokens 5.4/7.5 16/20 40/43 67/66   48 tokens 6.4/8.1 18/20 46/44 78/67
+//                    28 on 4,  44 tokens 5.4/8.1 15/20 38/44 64/67   60 tokens 6.9/8.6 20/21 50/44 85/67
+//   2                32 on 16, 48 tokens 5.6/8.1 15/20 38/43 63/67   56 tokens 6.2/8.7 19/21 47/44 79/67
+//                    16 on 8,  96 tokens 6.5/10.3 16/22 39/45 64/68  128 tokens 8.2/11.5 21/23 50/45 81/67
+//   4                32 on 8,  32 tokens 6.1/7.6 14/20 35/42 58/66   72 tokens 8.8/9.2 26/21 .. 110/67
+//      between       64 tokens 7.4/8.3 21/21 .. 82/66: from 350 rows
+//   5                                                                40 on 8, 33 tokens 7.5/7.2 23/20 .. 95/66
+//      below         32 tokens 6.8/7.1 18/20 41/41 68/66: from 1200 rows; 2 tokens, ten queries in the tile's
+//                    sixteen, 17/18 behind 300, 28/28 behind 650, 39/37 behind 950: from 650
+//   6, 8                                                             48 on 8, 2 tokens 6.4/5.8 18/17 .. 77/62
+// One query head a KV head of 8, 16 tokens behind 1000 rows: 17 us on the vector unit, 41 in a tile.
 // Byte offsets of 32 bits, rows left out by a score of -inf (scale > 0).
 int chunk_matrix_from(int n_tok, int n_q, int n_kv, int hd, int n_waves, float scale, int max_seq) {
   constexpr int kNever = INT32_MAX;
@@ -944,12 +947,12 @@ int chunk_matrix_from(int n_tok, int n_q, int n_kv, int hd, int n_waves, float s
   }
   const int64_t cus = device_cu_count(), shared = static_cast<int64_t>(n_tok) * n_kv;
   switch (n_rep) {  // the group forms of launch_chunk_gqa
-    case 2: return shared > 6 * cus ? 0 : kNever;
+    case 2: return shared > 3 * cus ? 0 : kNever;
     case 4: return shared > 2 * cus ? 0 : (shared > cus ? 350 : kNever);
-    case 5: return shared > cus ? 0 : 1200;
+    case 5: return shared > cus ? 0 : (n_tok == 2 ? 650 : 1200);
     case 6:
     case 8: return 0;
-    default: return static_cast<int64_t>(n_tok) * n_q > 10 * cus ? 0 : kNever;
+    default: return static_cast<int64_t>(n_tok) * n_q > 5 * cus ? 0 : kNever;
   }
 }
 
