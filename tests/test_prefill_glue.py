@@ -51,8 +51,10 @@ def test_rms_cols(rows, n):
     assert np.abs(got - t.cpu().numpy().T).max() <= 2 ** -7 * max(1.0, np.abs(ref).max())
 
 
-# 32 and 16 chains a column, rows that end inside a step and inside a batch of 32, just above and below the line
-@pytest.mark.parametrize("rows,n", [(5120, 17), (1024, 31), (1025, 24), (5120, 63), (1039, 33), (4099, 50), (1023, 40)])
+# 32 and 16 chains a column, rows that end inside a step and inside a batch of 32, above and below the lines from which
+# the library takes two launches (1536 rows up to 31 columns, 1024 from 33 on) and the wrapper asks for them
+@pytest.mark.parametrize("rows,n", [(5120, 17), (1024, 31), (1025, 24), (1536, 31), (1569, 24), (5120, 63), (1039, 33),
+                                    (4099, 50), (1023, 40)])
 def test_rms_cols_in_two_launches(rows, n):
     say("rms_cols two launches", rows, n)
     x, w = bf16_tensor(rnd((rows, n), rows + n, 1.5)), bf16_tensor(rnd((rows,), 3, 1.0))
@@ -60,6 +62,10 @@ def test_rms_cols_in_two_launches(rows, n):
     lib = nf4._load_ext()
     assert lib.chr_dv2_rms_cols(x.data_ptr(), w.data_ptr(), one.data_ptr(), rows, n, 1e-6, nf4._stream()) == 0
     assert torch.equal(nf4.dv2_rms_cols(x, w, 1e-6), one)
+    two, ws = torch.zeros_like(x), torch.full((lib.chr_dv2_rms_cols_ws_floats(),), float("nan"), device=DEV)
+    assert lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), two.data_ptr(), rows, n, 1e-6, ws.data_ptr(), nf4._stream()) == 0
+    assert torch.equal(two, one)
+    assert torch.isnan(ws).all().item() == (lib.chr_dv2_rms_cols_ws_for(rows, n, 1) == 0)
     assert lib.chr_dv2_rms_cols_ws(x.data_ptr(), w.data_ptr(), one.data_ptr(), rows, n, 1e-6, None, None) == -1
 
 
@@ -162,8 +168,9 @@ def test_attn_chunk(n_q, n_kv, hd, max_seq, first, n, waves):
     (40, 8, 320, 250, 70, True), (6, 2, 150, 20, 40, True), (1, 1, 70, 30, 17, True)])
 def test_attn_chunk_on_the_matrix_cores(n_q, n_kv, max_seq, first, n, odd):
     """Four wavefronts, 128 dims: every token has the bits of the decode step's kernel, also where rows behind a
-    token's own (``odd``: and rows it sees) hold infinities and NaN."""
-    say("attn_chunk_mfma", n_q, n_kv, max_seq, first, n, odd)
+    token's own (``odd``: and rows it sees) hold infinities and NaN.  Which of the forms a chunk of this kind takes
+    hangs on its heads and tokens; test_attn_chunk_form.py runs this test where each is sure to be taken."""
+    say("attn_chunk, 128 dims", n_q, n_kv, max_seq, first, n, odd)
     q, kc, vc = rnd((n, n_q * 128), 31, 2.0), rnd((max_seq, n_kv, 128), 32), rnd((max_seq, n_kv, 128), 33)
     last = min(first + n - 1, max_seq)
     kc[last:], vc[last:] = np.nan, np.inf
