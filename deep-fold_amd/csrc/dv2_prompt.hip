@@ -53,7 +53,9 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
 // and the start of a chunk; 18 000 clocks a workgroup lie outside the loop.  Gate and up of 27648 x 5120 at
 // 1792 tokens 1.38 ms (0.74 PFLOP/s; 1.70 with every block's lookups, products and scaling one after the
 // other), down 5120 x 27648 0.70 (0.89), at 512 tokens 13824 x 5120 207 us (263), 5120 x 13824 104 (132),
-// 5120 x 5120 55 (69), 7168 x 5120 68 (86); the clock is at 1.9 to 2.3 GHz in these launches.
+// 5120 x 5120 55 (69), 7168 x 5120 68 (86); on a faster card 1.24 and 0.67 ms, 192, 90, 45 and 57 us.  There the
+// matrix cores are busy 0.33 to 0.42 of the clocks, vector instructions issue in 0.52 to 0.59, and the clock falls with
+// a launch's length: 2.35 GHz at 45 us, 2.0 to 2.2 at 150 to 650, 1.86 at 1.2 ms.
 //
 // 256 rows x 64 tokens.  As in the 64-column tile a wavefront sums group w % 4 of every chunk of
 // 256, four 16-wide products a group in the same order of k, scaled into its accumulators group by
@@ -69,8 +71,8 @@ __device__ __forceinline__ uint16_t swiglu_bf16(float gate, float up) {
 // for the last time.  The order is pinned (sched_barrier): the compiler pulls the units apart again.
 //
 // Codes: a lane pair fetches the 32 bytes of a row's group; two neighbouring rows' fetches are handed to the
-// lanes that multiply them by two lane exchanges (hand_over; ds_bpermute, 6 clocks of LDS each, took a third
-// of its time).  x straight to LDS in 128-byte rows (a token's group), 16-byte pieces XORed with the row's low
+// lanes that multiply them by two lane exchanges (hand_over; on their own no faster than ds_bpermute, which is 6
+// clocks of LDS each).  x straight to LDS in 128-byte rows (a token's group), 16-byte pieces XORed with the row's low
 // bits, and so the scales.  Flat loads to LDS in flight turn every wait for a register into a wait for all of
 // them: codes, x and scales have half a chunk or more to arrive, which no launch here was seen to wait for
 // (without any of the loads the loop takes as long).

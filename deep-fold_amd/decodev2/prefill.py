@@ -169,7 +169,7 @@ class ChunkPrefill:
     def whole_windows(self, n: int) -> int:
         """Tokens in front of an ``n``-token prompt that go through together: its whole windows,
         where there are two or more of the default width.  Two, as two graph replays and as one pass
-        (ms): 3B 8.45 / 6.96, 14B 12.7 / 10.7, 32B 24.9 / 17.9, two layers of the 3B 0.58 / 0.50."""
+        (ms): 3B 8.35 / 6.42, 14B 12.75 / 8.66, 32B 24.7 / 15.0, two layers of the 3B 0.66 / 0.58."""
         whole = int(n) - int(n) % self.MAX_WIDTH
         if self.width != self.MAX_WIDTH or whole < 2 * self.MAX_WIDTH or not self._serves_windows():
             return 0
